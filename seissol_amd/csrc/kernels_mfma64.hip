@@ -1,4 +1,4 @@
-// Host side of the FP64 engines' matrix-core local pass: the FP64 fragments of
+// Host side of the FP64 engines' matrix-core neighbour pass: the FP64 fragments of
 // the global matrices and the dispatch over the orders 3-7 (the kernels of one
 // order are built by kernels_mfma64_o<O>.hip).
 #include <hip/hip_runtime.h>
@@ -15,50 +15,13 @@
 namespace sdg {
 namespace {
 
-// A (rows x cols, 0 outside) in the lane order of v_mfma_f64_16x16x4_f64's A
-// operand: lane l of fragment (mt, ks) holds A[16 mt + l % 16][4 ks + l / 16]
-void appendFragments64(const std::function<double(int, int)>& A, int rows, int cols, int mtiles, int ksteps,
-                       double* out) {
-  for (int mt = 0; mt < mtiles; ++mt)
-    for (int ks = 0; ks < ksteps; ++ks) {
-      double* base = out + (static_cast<int64_t>(mt) * ksteps + ks) * 64;
-      for (int l = 0; l < 64; ++l) {
-        const int r = 16 * mt + l % 16, c = 4 * ks + l / 16;
-        base[l] = (r < rows && c < cols) ? A(r, c) : 0.0;
-      }
-    }
-}
-
 template <int O>
 int uploadData64(EngineState& s, const double* gm) {
   using S = mfma64::Shape64<O>;
   const auto g = globalMatrixLayout(O);
-  const int B = S::B, B2 = S::B2, B2P = S::B2P;
+  const int B = S::B, B2 = S::B2;
   std::vector<double> frags(S::total, 0.0);
-  for (int j = 0; j < 3; ++j) {
-    appendFragments64([&](int r, int c) { return -gm[g.kDivMT + (j * B + r) * B + c]; }, B, B, S::MT, S::KSB,
-                      frags.data() + S::ck + static_cast<int64_t>(j) * S::MT * S::KSB * 64);
-    appendFragments64([&](int r, int c) { return gm[g.kDivM + (j * B + r) * B + c]; }, B, B, S::MT, S::KSB,
-                      frags.data() + S::vol + static_cast<int64_t>(j) * S::MT * S::KSB * 64);
-  }
-  // the four face operands stacked with B2P rows each: traces (fMrT_f / M2) I
-  appendFragments64(
-      [&](int r, int c) {
-        const int m = r % B2P;
-        return m < B2 ? gm[g.fMrT + ((r / B2P) * B2 + m) * B + c] / gm[g.mass2 + m] : 0.0;
-      },
-      S::FR, B, S::MTF, S::KSB, frags.data() + S::fmrt);
-  // rDivM_f diag(M2), one face at a time: [m-tile][face][k-step]
-  for (int mt = 0; mt < S::MT; ++mt)
-    for (int f = 0; f < 4; ++f)
-      for (int ks = 0; ks < S::KSF; ++ks) {
-        double* base = frags.data() + S::rdm + ((static_cast<int64_t>(mt) * 4 + f) * S::KSF + ks) * 64;
-        for (int l = 0; l < 64; ++l) {
-          const int r = 16 * mt + l % 16, m = 4 * ks + l / 16;
-          base[l] = (r < B && m < B2) ? gm[g.rDivM + (f * B + r) * B2 + m] * gm[g.mass2 + m] : 0.0;
-        }
-      }
-  // the neighbour pass: rDivM_f per face, and fP_h as rows of at most O non-zeros
+  // rDivM_f per face, and fP_h as rows of at most O non-zeros
   for (int mt = 0; mt < S::MT; ++mt)
     for (int f = 0; f < 4; ++f)
       for (int ks = 0; ks < S::KSF; ++ks) {
@@ -91,18 +54,6 @@ int uploadData64(EngineState& s, const double* gm) {
   return SDG_OK;
 }
 
-int localOrders64(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream,
-                  const mfma64::LtsOut64* lts) {
-  switch (e.order) {
-    case 3: return mfma64::MfmaOrder64<3>::local(e, coeffs, layer, stream, lts);
-    case 4: return mfma64::MfmaOrder64<4>::local(e, coeffs, layer, stream, lts);
-    case 5: return mfma64::MfmaOrder64<5>::local(e, coeffs, layer, stream, lts);
-    case 6: return mfma64::MfmaOrder64<6>::local(e, coeffs, layer, stream, lts);
-    case 7: return mfma64::MfmaOrder64<7>::local(e, coeffs, layer, stream, lts);
-    default: setError("the FP64 matrix-core pass supports orders 3..7"); return SDG_ERR_UNSUPPORTED;
-  }
-}
-
 }  // namespace
 
 int64_t mfma64::fragmentCount(int order) {
@@ -131,14 +82,6 @@ bool hasMfma64(const EngineState& e) {
   return e.arithmetic == SDG_FP64 && e.mfma64Frags != nullptr && e.kernels == SDG_KERNELS_AUTO;
 }
 
-int launchAderLocalMfma64(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
-  if (layer->derivatives != nullptr) {
-    const mfma64::LtsOut64 lts{nullptr, static_cast<double*>(layer->derivatives), 1, 0};
-    return localOrders64(e, coeffs, layer, stream, &lts);
-  }
-  return localOrders64(e, coeffs, layer, stream, nullptr);
-}
-
 int launchNeighborMfma64(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
   switch (e.order) {
     case 3: return mfma64::MfmaOrder64<3>::neighbor(e, layer, stream);
@@ -148,12 +91,6 @@ int launchNeighborMfma64(const EngineState& e, const sdg_layer* layer, hipStream
     case 7: return mfma64::MfmaOrder64<7>::neighbor(e, layer, stream);
     default: setError("the FP64 matrix-core pass supports orders 3..7"); return SDG_ERR_UNSUPPORTED;
   }
-}
-
-int launchLocalIntegrationMfma64(const EngineState& e, const double* coeffs, const sdg_layer* layer,
-                                 int resetBuffers, hipStream_t stream) {
-  const mfma64::LtsOut64 lts{layer->lts_setup, static_cast<double*>(layer->derivatives), resetBuffers, 0};
-  return localOrders64(e, coeffs, layer, stream, &lts);
 }
 
 }  // namespace sdg

@@ -1,0 +1,163 @@
+// Host side of the matrix-core passes in the engine's real type: the fragments
+// of the global matrices, the k-step ranges that hold each row tile's
+// non-zeros, and the dispatch over the orders 3-7 (the kernels of one order
+// are built by kernels_mx_o<O>.hip).
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <functional>
+#include <vector>
+
+#include "engine.h"
+#include "global_matrices.h"
+#include "mx_common.h"
+
+namespace sdg {
+namespace {
+
+using Matrix = std::function<double(int, int)>;
+
+// One row tile (16 rows) of A: fragments over k-steps [0, ksteps) in the lane
+// order of the A operand, and the range of k-steps that holds its non-zeros
+// (entries above 1e-13 of the largest of the whole matrix: the generator's
+// quadrature leaves rounding noise where the exact value is zero)
+template <typename real>
+void tileFragments(const Matrix& A, int ksteps, real* out) {
+  for (int ks = 0; ks < ksteps; ++ks)
+    for (int l = 0; l < 64; ++l) out[ks * 64 + l] = static_cast<real>(A(mx::fragRow<real>(l % 16), 4 * ks + l / 16));
+}
+// rows < rowEnd, columns < colEnd; lo < hi always (a zero tile keeps k-step 0)
+void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, double threshold, int* out) {
+  int lo = 1 << 20, hi = 0;
+  for (const Matrix& A : As)
+    for (int r = 0; r < rowEnd && r < 16; ++r)
+      for (int c = 0; c < colEnd; ++c)
+        if (std::fabs(A(r, c)) > threshold) {
+          lo = lo < c / 4 ? lo : c / 4;
+          hi = hi > c / 4 + 1 ? hi : c / 4 + 1;
+        }
+  out[0] = hi == 0 ? 0 : lo;
+  out[1] = hi == 0 ? 1 : hi;
+}
+double largest(const double* p, int64_t n) {
+  double m = 0.0;
+  for (int64_t i = 0; i < n; ++i) m = std::max(m, std::fabs(p[i]));
+  return 1e-13 * m;
+}
+
+template <typename real, int O>
+int uploadOrder(EngineState& s, const double* gm) {
+  using G = mx::Geo<O>;
+  const auto g = globalMatrixLayout(O);
+  constexpr int B = G::B, B2 = G::B2, B2P = G::B2P, KS = G::KS;
+  std::vector<real> frags(G::total, real(0));
+  std::vector<int> ranges(G::rTotal, 0);
+  const double tolT = largest(gm + g.kDivMT, 3LL * B * B), tolV = largest(gm + g.kDivM, 3LL * B * B);
+  const double tolF = largest(gm + g.fMrT, 4LL * B * B2), tolR = largest(gm + g.rDivM, 4LL * B * B2);
+  for (int t = 0; t < G::MT; ++t) {
+    std::vector<Matrix> ck, vol;
+    for (int j = 0; j < 3; ++j) {
+      ck.push_back([=](int r, int c) {
+        r += 16 * t;
+        return r < B && c < B ? -gm[g.kDivMT + (j * B + r) * B + c] : 0.0;
+      });
+      vol.push_back([=](int r, int c) {
+        r += 16 * t;
+        return r < B && c < B ? gm[g.kDivM + (j * B + r) * B + c] : 0.0;
+      });
+      tileFragments<real>(ck[j], KS, frags.data() + G::ck + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
+      tileFragments<real>(vol[j], KS, frags.data() + G::vol + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
+    }
+    // derivative d has basis3(O - d) rows of basis3(O - d + 1) columns
+    for (int d = 1; d < O; ++d)
+      tileRange(ck, mx::basis3(O - d) - 16 * t, mx::basis3(O - d + 1), tolT,
+                ranges.data() + G::rCk + 2 * ((d - 1) * G::MT + t));
+    tileRange(vol, 16, B, tolV, ranges.data() + G::rVol + 2 * t);
+    for (int f = 0; f < 4; ++f) {
+      const Matrix R = [=](int r, int c) {
+        r += 16 * t;
+        return r < B && c < B2 ? gm[g.rDivM + (f * B + r) * B2 + c] : 0.0;
+      };
+      tileFragments<real>([&](int r, int c) { return c < B2 ? R(r, c) * gm[g.mass2 + c] : 0.0; }, G::KSF,
+                          frags.data() + G::flux + (static_cast<int64_t>(t) * 4 + f) * G::KSF * 64);
+      tileRange({R}, 16, B2, tolR, ranges.data() + G::rFlux + 2 * (t * 4 + f));
+    }
+  }
+  for (int t = 0; t < G::MTF; ++t) {
+    const Matrix F = [=](int r, int c) {
+      const int f = G::traceFace(t, r / 4), m = G::traceRow(t, r / 4) + r % 4;
+      return m < B2 && c < B ? gm[g.fMrT + (f * B2 + m) * B + c] : 0.0;
+    };
+    tileFragments<real>(
+        [&](int r, int c) {
+          const int m = G::traceRow(t, r / 4) + r % 4;
+          return m < B2 ? F(r, c) / gm[g.mass2 + m] : 0.0;
+        },
+        KS, frags.data() + G::trace + static_cast<int64_t>(t) * KS * 64);
+    tileRange({F}, 16, B, tolF, ranges.data() + G::rTrace + 2 * t);
+  }
+  if (s.mxFrags == nullptr) SDG_HIP_CHECK(hipMalloc(&s.mxFrags, frags.size() * sizeof(real)));
+  if (s.mxRanges == nullptr)
+    SDG_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&s.mxRanges), ranges.size() * sizeof(int)));
+  SDG_HIP_CHECK(hipMemcpy(s.mxFrags, frags.data(), frags.size() * sizeof(real), hipMemcpyHostToDevice));
+  SDG_HIP_CHECK(hipMemcpy(s.mxRanges, ranges.data(), ranges.size() * sizeof(int), hipMemcpyHostToDevice));
+  return SDG_OK;
+}
+
+template <typename F>
+int orders(const EngineState& e, F&& f) {
+  switch (e.order) {
+    case 3: return f(mx::Order<3>{});
+    case 4: return f(mx::Order<4>{});
+    case 5: return f(mx::Order<5>{});
+    case 6: return f(mx::Order<6>{});
+    case 7: return f(mx::Order<7>{});
+    default: setError("the matrix-core passes support orders 3..7"); return SDG_ERR_UNSUPPORTED;
+  }
+}
+
+}  // namespace
+
+int uploadMx(EngineState& s, const double* gm) {
+  const bool dbl = s.arithmetic == SDG_FP64;
+  switch (s.order) {
+    case 3: return dbl ? uploadOrder<double, 3>(s, gm) : uploadOrder<float, 3>(s, gm);
+    case 4: return dbl ? uploadOrder<double, 4>(s, gm) : uploadOrder<float, 4>(s, gm);
+    case 5: return dbl ? uploadOrder<double, 5>(s, gm) : uploadOrder<float, 5>(s, gm);
+    case 6: return dbl ? uploadOrder<double, 6>(s, gm) : uploadOrder<float, 6>(s, gm);
+    case 7: return dbl ? uploadOrder<double, 7>(s, gm) : uploadOrder<float, 7>(s, gm);
+    default: return SDG_OK;  // orders 2 and 8: the VALU kernels
+  }
+}
+
+bool hasMx(const EngineState& e) { return e.mxFrags != nullptr && e.kernels == SDG_KERNELS_AUTO; }
+
+int launchAderMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
+  const mx::LtsOut lts{layer->lts_setup, layer->derivatives, 1, 0};
+  return orders(e, [&](auto o) { return o.local(e, mx::kPredict, coeffs, layer, false, &lts, stream); });
+}
+
+int launchLocalMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
+  return orders(e, [&](auto o) { return o.local(e, mx::kFlux, nullptr, layer, false, nullptr, stream); });
+}
+
+int launchAderLocalMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
+  // only the FP64 neighbour pass reads traces of this kernel
+  const bool fp64 = e.arithmetic == SDG_FP64;
+  // FP64: the buffer and derivatives of every cell; FP32: per the layer's LTS setup where it has one
+  const mx::LtsOut lts{fp64 ? nullptr : layer->lts_setup, layer->derivatives, 1, 0};
+  const bool some = lts.deriv != nullptr || lts.setup != nullptr;
+  return orders(e, [&](auto o) {
+    return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, fp64, some ? &lts : nullptr, stream);
+  });
+}
+
+int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
+                             hipStream_t stream) {
+  const mx::LtsOut lts{layer->lts_setup, layer->derivatives, resetBuffers, 0};
+  return orders(e, [&](auto o) {
+    return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, e.arithmetic == SDG_FP64, &lts, stream);
+  });
+}
+
+}  // namespace sdg

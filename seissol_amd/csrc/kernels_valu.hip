@@ -1281,10 +1281,11 @@ DeviceMatrixLayout deviceMatrixLayout(int order) {
 }
 
 int launchAder(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
+  if (hasMx(e)) return launchAderMx(e, coeffs, layer, stream);
   return dispatch<AderOp>(e, coeffs, layer, stream, false, 1);
 }
 int launchAderLocal(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
-  if (hasMfma64(e)) return launchAderLocalMfma64(e, coeffs, layer, stream);
+  if (hasMx(e)) return launchAderLocalMx(e, coeffs, layer, stream);
   return dispatch<AderOp>(e, coeffs, layer, stream, true, 1);
 }
 int launchLocalIntegration(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
@@ -1296,6 +1297,7 @@ int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs,
   return dispatch<LtsNeighborOp>(e, layer, stream, timeCoeffs, subtimeCoeffs, variant);
 }
 int launchLocal(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
+  if (hasMx(e)) return launchLocalMx(e, layer, stream);
   return dispatch<LocalOp>(e, layer, stream);
 }
 int launchNeighbor(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {

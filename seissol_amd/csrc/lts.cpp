@@ -72,10 +72,12 @@ int defaultNeighborVariant(const EngineState& e) {
 int localVariants(const EngineState& e) { return matrixCoreLocal(e) ? 1 + kTileVariants : kTileVariants; }
 
 int runLocal(const EngineState& e, const double* coeffs, const sdg_layer* own, int reset, hipStream_t s, int v) {
-  if (!matrixCoreLocal(e)) return launchLocalIntegration(e, coeffs, own, reset, s, v);
+  if (!matrixCoreLocal(e))
+    return v == 0 && hasMx(e) ? launchLocalIntegrationMx(e, coeffs, own, reset, s)
+                              : launchLocalIntegration(e, coeffs, own, reset, s, v);
   if (v == 0)
     return matrixCore(e.arithmetic) ? launchLocalIntegrationMfma(e, coeffs, own, reset, s)
-                                    : launchLocalIntegrationMfma64(e, coeffs, own, reset, s);
+                                    : launchLocalIntegrationMx(e, coeffs, own, reset, s);
   return launchLocalIntegration(e, coeffs, own, reset, s, v - 1);
 }
 

@@ -516,11 +516,14 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic) {
   int rc = uploadMatrices(e->s, gm.data());
   if (rc == SDG_OK && matrixCore(arithmetic)) rc = uploadMfma(e->s, gm.data());
   if (rc == SDG_OK && arithmetic == SDG_FP64) rc = uploadMfma64(e->s, gm.data());
+  if (rc == SDG_OK) rc = uploadMx(e->s, gm.data());
   if (rc != SDG_OK) {
     if (e->s.matrices) (void)hipFree(e->s.matrices);
     if (e->s.mfmaFrags) (void)hipFree(e->s.mfmaFrags);
     if (e->s.mfmaTables) (void)hipFree(e->s.mfmaTables);
     if (e->s.mfma64Frags) (void)hipFree(e->s.mfma64Frags);
+    if (e->s.mxFrags) (void)hipFree(e->s.mxFrags);
+    if (e->s.mxRanges) (void)hipFree(e->s.mxRanges);
     delete e;
     return rc;
   }
@@ -530,7 +533,8 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic) {
 
 int sdg_engine_set_global_matrices(sdg_engine* engine, const double* host_matrices) {
   if (engine == nullptr || host_matrices == nullptr) { setError("invalid arguments"); return SDG_ERR_INVALID; }
-  const int rc = uploadMatrices(engine->s, host_matrices);
+  int rc = uploadMatrices(engine->s, host_matrices);
+  if (rc == SDG_OK) rc = uploadMx(engine->s, host_matrices);
   if (rc != SDG_OK) return rc;
   if (engine->s.arithmetic == SDG_FP64) return uploadMfma64(engine->s, host_matrices);
   if (!matrixCore(engine->s.arithmetic)) return rc;
@@ -582,6 +586,8 @@ int sdg_engine_destroy(sdg_engine* engine) {
   if (engine->s.mfmaTables) SDG_HIP_CHECK(hipFree(engine->s.mfmaTables));
   if (engine->s.drMatrices) SDG_HIP_CHECK(hipFree(engine->s.drMatrices));
   if (engine->s.mfma64Frags) SDG_HIP_CHECK(hipFree(engine->s.mfma64Frags));
+  if (engine->s.mxFrags) SDG_HIP_CHECK(hipFree(engine->s.mxFrags));
+  if (engine->s.mxRanges) SDG_HIP_CHECK(hipFree(engine->s.mxRanges));
   delete engine;
   return SDG_OK;
 }

@@ -1,0 +1,84 @@
+"""The matrix-core passes in the engine's real type against the VALU kernels
+of the same engine (GPU tests): predictor, local integral and the fused LTS
+pass, every order they serve, ragged layers and enough workgroups to put the
+memory system under load."""
+import ctypes as C
+
+import pytest
+
+from seissol_amd import _capi
+from seissol_amd._capi import check, lib, ptr
+from seissol_amd.kernels import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def random_layer(eng, order, arith, n, align, star, seed, setup=False):
+    """Arrays of random values (the kernels are linear maps of the DOFs: no mesh is needed)."""
+    import torch
+    rt = torch.float64 if arith == "fp64" else torch.float32
+    ld, reals, dsize = C.c_int32(), C.c_int64(), C.c_int64()
+    check(lib().sdg_layout_sizes(eng.handle, C.byref(ld), C.byref(reals), C.byref(dsize)), "sdg_layout_sizes")
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *shape: torch.rand(shape, generator=gen, device="cuda", dtype=rt) * 2 - 1
+    a = dict(dofs=rnd(n, 9, ld.value), integrated=rnd(n, 9, ld.value), derivatives=rnd(n, dsize.value),
+             star=rnd(n, 3, 24 if star == "compact" else 81), aplus=rnd(n, 4, 81))
+    if setup:
+        bits = torch.randint(0, 8, (n,), generator=gen, device="cuda", dtype=torch.int32) << 8
+        a["setup"] = bits.to(torch.int16)
+    a["view"] = _capi.Layer(n, ptr(a["dofs"]), ptr(a["integrated"]), ptr(a["derivatives"]), ptr(a["star"]),
+                            ptr(a["aplus"]), None, None, None, None, None, ptr(a.get("setup")), 0, 0, 0)
+    return a
+
+
+def run_local(eng, a, part, reset):
+    import torch
+    coeffs = (C.c_double * 8)(1.0, 0.5, 0.2, 0.1, 0.05, 0.02, 0.01, 0.005)
+    s, view = torch.cuda.current_stream().cuda_stream, C.byref(a["view"])
+    if part == "ader":
+        check(lib().sdg_compute_batched_ader(eng.handle, coeffs, 1.0, view, s), part)
+    elif part == "local":
+        check(lib().sdg_compute_batched_integral(eng.handle, view, s), part)
+    else:
+        check(lib().sdg_compute_local_integration(eng.handle, coeffs, 1.0, view, reset, s), part)
+    torch.cuda.synchronize()
+
+
+def same(a, b, keys, tol, what):
+    import torch
+    for k in keys:
+        assert torch.isfinite(a[k]).all(), (what, k)
+        err = float((a[k] - b[k]).abs().max() / b[k].abs().max())
+        print(f"{what} {k}: largest difference / largest value {err:.1e}", flush=True)
+        assert err < tol, (what, k)
+
+
+# sums of at most 3 * 84 products in O - 1 <= 6 nested steps: 1e4 roundings at the very most
+@pytest.mark.parametrize("arith,tol", [("fp64", 1e-12), ("fp32", 5e-5)])
+@pytest.mark.parametrize("order", [3, 4, 5, 6, 7])
+def test_local_passes_equal_the_valu_kernels(gpu, order, arith, tol):
+    for n, align, star, part, reset in ((1, 0, "dense", "ader", 1), (17, 128, "compact", "local", 1),
+                                        (333, 0, "compact", "lts", 1), (333, 128, "dense", "lts", 0)):
+        print(f"mx {arith} order={order} n={n} align={align} {star} {part}", flush=True)
+        sides = []
+        for family in ("auto", "valu"):
+            eng = Engine(order, arith)
+            eng.set_layout(align, star)
+            eng.set_kernels(family)
+            a = random_layer(eng, order, arith, n, align, star, 7 * order + n, setup=part == "lts")
+            run_local(eng, a, part, reset)
+            sides.append(a)
+        same(*sides, ("dofs", "integrated", "derivatives"), tol, f"{part} n={n}")
+
+
+@pytest.mark.parametrize("arith,tol", [("fp64", 1e-12), ("fp32", 5e-5)])
+def test_local_pass_under_memory_load(gpu, arith, tol):
+    # thousands of workgroups with all their stores in flight
+    sides = []
+    for family in ("auto", "valu"):
+        eng = Engine(6, arith)
+        eng.set_kernels(family)
+        a = random_layer(eng, 6, arith, 50_000, 0, "dense", 3, setup=True)
+        run_local(eng, a, "lts", 0)
+        sides.append(a)
+    same(*sides, ("dofs", "integrated", "derivatives"), tol, f"{arith} n=50000")
