@@ -77,6 +77,7 @@ struct EngineState {
   // matrix-core passes of mx_local.h
   void* mxFrags = nullptr;
   int* mxRanges = nullptr;
+  bool mxNeighbor = false;  // the fP_h are sparse enough for the neighbour pass of mx_neighbor.h
 };
 
 // the layout of `layer` (its strides, 0 = the dense defaults) under the engine's settings
@@ -110,6 +111,9 @@ constexpr int kNeighborRowsVariant = kTileVariants;
 constexpr int kNeighborVariants = kTileVariants + 1;
 int launchLocalIntegration(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
                            hipStream_t stream, int variant = 0);
+// the neighbour pass's variant before any tuning, which is the matrix-core
+// pass where the engine has it
+int defaultNeighborVariant(const EngineState& e);
 int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs, const double* subtimeCoeffs,
                                  const sdg_layer* layer, hipStream_t stream, int variant = 0);
 // kernels_mfma.hip
@@ -128,6 +132,11 @@ int launchLocalMx(const EngineState& e, const sdg_layer* layer, hipStream_t stre
 int launchAderLocalMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream);
 int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
                              hipStream_t stream);
+// the neighbour pass from the neighbours' buffers (LTS: with the time
+// coefficients, else nullptr: global time stepping)
+bool hasNeighborMx(const EngineState& e);
+int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
+                     const double* subtimeCoeffs, hipStream_t stream);
 // kernels_mfma64.hip: the FP64 neighbour pass on the matrix cores from the FP64
 // face traces the local pass wrote (layer->face_traces, [n][4][9][B2P])
 bool hasMfma64(const EngineState& e);

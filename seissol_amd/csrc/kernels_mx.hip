@@ -4,6 +4,7 @@
 // are built by kernels_mx_o<O>.hip).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <functional>
 #include <vector>
@@ -26,15 +27,16 @@ void tileFragments(const Matrix& A, int ksteps, real* out) {
   for (int ks = 0; ks < ksteps; ++ks)
     for (int l = 0; l < 64; ++l) out[ks * 64 + l] = static_cast<real>(A(mx::fragRow<real>(l % 16), 4 * ks + l / 16));
 }
-// rows < rowEnd, columns < colEnd; lo < hi always (a zero tile keeps k-step 0)
-void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, double threshold, int* out) {
+// rows < rowEnd, columns < colEnd, in steps of `step` columns; lo < hi always (a zero tile keeps k-step 0)
+void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, double threshold, int step,
+               int* out) {
   int lo = 1 << 20, hi = 0;
   for (const Matrix& A : As)
     for (int r = 0; r < rowEnd && r < 16; ++r)
       for (int c = 0; c < colEnd; ++c)
         if (std::fabs(A(r, c)) > threshold) {
-          lo = lo < c / 4 ? lo : c / 4;
-          hi = hi > c / 4 + 1 ? hi : c / 4 + 1;
+          lo = std::min(lo, c / step);
+          hi = std::max(hi, c / step + 1);
         }
   out[0] = hi == 0 ? 0 : lo;
   out[1] = hi == 0 ? 1 : hi;
@@ -54,6 +56,7 @@ int uploadOrder(EngineState& s, const double* gm) {
   std::vector<int> ranges(G::rTotal, 0);
   const double tolT = largest(gm + g.kDivMT, 3LL * B * B), tolV = largest(gm + g.kDivM, 3LL * B * B);
   const double tolF = largest(gm + g.fMrT, 4LL * B * B2), tolR = largest(gm + g.rDivM, 4LL * B * B2);
+  bool sparseFP = true;  // a caller's own matrices may have fuller rows: no neighbour pass here then
   for (int t = 0; t < G::MT; ++t) {
     std::vector<Matrix> ck, vol;
     for (int j = 0; j < 3; ++j) {
@@ -70,9 +73,9 @@ int uploadOrder(EngineState& s, const double* gm) {
     }
     // derivative d has basis3(O - d) rows of basis3(O - d + 1) columns
     for (int d = 1; d < O; ++d)
-      tileRange(ck, mx::basis3(O - d) - 16 * t, mx::basis3(O - d + 1), tolT,
+      tileRange(ck, mx::basis3(O - d) - 16 * t, mx::basis3(O - d + 1), tolT, 4,
                 ranges.data() + G::rCk + 2 * ((d - 1) * G::MT + t));
-    tileRange(vol, 16, B, tolV, ranges.data() + G::rVol + 2 * t);
+    tileRange(vol, 16, B, tolV, 4, ranges.data() + G::rVol + 2 * t);
     for (int f = 0; f < 4; ++f) {
       const Matrix R = [=](int r, int c) {
         r += 16 * t;
@@ -80,7 +83,8 @@ int uploadOrder(EngineState& s, const double* gm) {
       };
       tileFragments<real>([&](int r, int c) { return c < B2 ? R(r, c) * gm[g.mass2 + c] : 0.0; }, G::KSF,
                           frags.data() + G::flux + (static_cast<int64_t>(t) * 4 + f) * G::KSF * 64);
-      tileRange({R}, 16, B2, tolR, ranges.data() + G::rFlux + 2 * (t * 4 + f));
+      tileFragments<real>(R, G::KSF, frags.data() + G::rdm + (static_cast<int64_t>(t) * 4 + f) * G::KSF * 64);
+      tileRange({R}, 16, B2, tolR, 4, ranges.data() + G::rFlux + 2 * (t * 4 + f));
     }
   }
   for (int t = 0; t < G::MTF; ++t) {
@@ -94,8 +98,42 @@ int uploadOrder(EngineState& s, const double* gm) {
           return m < B2 ? F(r, c) / gm[g.mass2 + m] : 0.0;
         },
         KS, frags.data() + G::trace + static_cast<int64_t>(t) * KS * 64);
-    tileRange({F}, 16, B, tolF, ranges.data() + G::rTrace + 2 * t);
+    tileRange({F}, 16, B, tolF, 4, ranges.data() + G::rTrace + 2 * t);
   }
+  // rT_j of the neighbour pass: lane l of block k holds columns 8 k + 2 (l / 16) + {0, 1}
+  const double tolU = largest(gm + g.rT, 4LL * B2 * B);
+  for (int j = 0; j < 4; ++j)
+    for (int r = 0; r < G::RT; ++r) {
+      const Matrix U = [=](int i, int c) {
+        i += 16 * r;
+        return i < B2 && c < B ? gm[g.rT + (j * B2 + i) * B + c] : 0.0;
+      };
+      real* const out = frags.data() + G::rt + (static_cast<int64_t>(j) * G::RT + r) * G::KB8 * 128;
+      for (int k = 0; k < G::KB8; ++k)
+        for (int l = 0; l < 64; ++l)
+          for (int i = 0; i < 2; ++i)
+            out[(k * 64 + l) * 2 + i] = static_cast<real>(U(mx::fragRow<real>(l % 16), 8 * k + 2 * (l / 16) + i));
+      tileRange({U}, 16, B, tolU, 8, ranges.data() + G::rRt + 2 * (j * G::RT + r));
+    }
+  // fP_h as rows of at most O non-zeros, padded with zeros
+  for (int h = 0; h < 3; ++h) {
+    const double tolP = largest(gm + g.fP + h * B2 * B2, int64_t(B2) * B2);
+    for (int r = 0; r < B2; ++r) {
+      int cnt = 0;
+      for (int c = 0; c < B2; ++c) {
+        const double v = gm[g.fP + (h * B2 + r) * B2 + c];
+        if (std::fabs(v) <= tolP) continue;
+        if (cnt == O) {
+          sparseFP = false;
+          break;
+        }
+        frags[G::fP + (h * B2 + r) * O + cnt] = static_cast<real>(v);
+        frags[G::fPCol + (h * B2 + r) * O + cnt] = static_cast<real>(c);
+        ++cnt;
+      }
+    }
+  }
+  s.mxNeighbor = sparseFP;
   if (s.mxFrags == nullptr) SDG_HIP_CHECK(hipMalloc(&s.mxFrags, frags.size() * sizeof(real)));
   if (s.mxRanges == nullptr)
     SDG_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&s.mxRanges), ranges.size() * sizeof(int)));
@@ -131,6 +169,13 @@ int uploadMx(EngineState& s, const double* gm) {
 }
 
 bool hasMx(const EngineState& e) { return e.mxFrags != nullptr && e.kernels == SDG_KERNELS_AUTO; }
+
+bool hasNeighborMx(const EngineState& e) { return hasMx(e) && e.mxNeighbor; }
+
+int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
+                     const double* subtimeCoeffs, hipStream_t stream) {
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, timeCoeffs, subtimeCoeffs, stream); });
+}
 
 int launchAderMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
   const mx::LtsOut lts{layer->lts_setup, layer->derivatives, 1, 0};

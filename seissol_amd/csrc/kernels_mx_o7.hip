@@ -1,4 +1,5 @@
 // Matrix-core passes in the real type, ORDER 7.
 #include "mx_local.h"
+#include "mx_neighbor.h"
 
 template struct sdg::mx::Order<7>;

@@ -1294,6 +1294,8 @@ int launchLocalIntegration(const EngineState& e, const double* coeffs, const sdg
 }
 int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs, const double* subtimeCoeffs,
                                  const sdg_layer* layer, hipStream_t stream, int variant) {
+  if (variant == defaultNeighborVariant(e) && hasNeighborMx(e))
+    return launchNeighborMx(e, layer, timeCoeffs, subtimeCoeffs, stream);
   return dispatch<LtsNeighborOp>(e, layer, stream, timeCoeffs, subtimeCoeffs, variant);
 }
 int launchLocal(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
@@ -1301,6 +1303,7 @@ int launchLocal(const EngineState& e, const sdg_layer* layer, hipStream_t stream
   return dispatch<LocalOp>(e, layer, stream);
 }
 int launchNeighbor(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
+  if (hasNeighborMx(e)) return launchNeighborMx(e, layer, nullptr, nullptr, stream);
   return dispatch<NeighborOp>(e, layer, stream, static_cast<const double*>(nullptr),
                               static_cast<const double*>(nullptr));
 }

@@ -27,6 +27,16 @@
 
 using namespace sdg;
 
+// Neighbour-pass variant before any tuning: numbered as the VALU kernel that
+// was measured faster on the vector ALUs (one element per 16-lane row for the
+// FP32 kernel at orders 3-6 and the FP64 kernel at orders 4-5, else tile 0);
+// at orders 3-7 that number runs the matrix-core pass, faster than any of them.
+int sdg::defaultNeighborVariant(const EngineState& e) {
+  const bool fp64 = e.arithmetic == SDG_FP64;
+  const bool rows = fp64 ? (e.order >= 4 && e.order <= 5) : (e.order >= 3 && e.order <= 6);
+  return rows ? kNeighborRowsVariant : 0;
+}
+
 namespace {
 
 constexpr uint16_t kNHD0 = 1u << 0;  // neighbour on face 0 provides derivatives
@@ -57,18 +67,11 @@ bool ltsLayerOk(const sdg_layer* L, bool neighbors, const char* who) {
 // shapes; a matrix-core engine has its matrix-core pass (variant 0) and the
 // FP32 VALU shapes after it.  The neighbour pass is the VALU kernel of the
 // engine's real type (FP32 for the matrix-core engines) with kTileVariants
-// shapes, then the one-element-per-row kernel (kNeighborRowsVariant).
+// shapes, then the one-element-per-row kernel (kNeighborRowsVariant); its default
+// variant is the matrix-core pass where the engine has it.
 // The FP64 engine (orders 3-7, kernel family AUTO) likewise has its FP64
 // matrix-core pass as variant 0.
 bool matrixCoreLocal(const EngineState& e) { return matrixCore(e.arithmetic) || hasMfma64(e); }
-// Neighbour-pass variant before any tuning: one element per 16-lane row for
-// the FP32 kernel at orders 3-6 and the FP64 kernel at orders 4-5 (where
-// the autotuner picked it on every cluster), else tile 0.
-int defaultNeighborVariant(const EngineState& e) {
-  const bool fp64 = e.arithmetic == SDG_FP64;
-  const bool rows = fp64 ? (e.order >= 4 && e.order <= 5) : (e.order >= 3 && e.order <= 6);
-  return rows ? kNeighborRowsVariant : 0;
-}
 int localVariants(const EngineState& e) { return matrixCoreLocal(e) ? 1 + kTileVariants : kTileVariants; }
 
 int runLocal(const EngineState& e, const double* coeffs, const sdg_layer* own, int reset, hipStream_t s, int v) {

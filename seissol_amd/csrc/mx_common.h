@@ -71,13 +71,21 @@ struct Geo {
   static constexpr int64_t vol = ck + 3LL * MT * KS * 64;        // [MT][3][KS]
   static constexpr int64_t trace = vol + 3LL * MT * KS * 64;     // [MTF][KS]     rT_f = fMrT_f / M2
   static constexpr int64_t flux = trace + 1LL * MTF * KS * 64;   // [MT][4][KSF]  rDivM_f diag(M2)
-  static constexpr int64_t total = flux + 4LL * MT * KSF * 64;
+  // neighbour pass: rT_j in blocks of 8 columns (a lane's two consecutive
+  // ones in one load), rDivM_f, and fP_h as rows of O (value, column) entries
+  static constexpr int RT = cdiv(B2, 16), KB8 = cdiv(B, 8);
+  static constexpr int64_t rt = flux + 4LL * MT * KSF * 64;      // [4][RT][KB8][64][2]
+  static constexpr int64_t rdm = rt + 4LL * RT * KB8 * 128;      // [MT][4][KSF]
+  static constexpr int64_t fP = rdm + 4LL * MT * KSF * 64;       // [3][B2][O] values
+  static constexpr int64_t fPCol = fP + 3LL * B2 * O;            // [3][B2][O] columns (exact integers)
+  static constexpr int64_t total = fPCol + 3LL * B2 * O;
   // k-step ranges [lo, hi) that hold a row tile's non-zeros, as (lo, hi) pairs
   static constexpr int rCk = 0;                       // [O - 1][MT]
   static constexpr int rVol = rCk + 2 * (O - 1) * MT; // [MT]
   static constexpr int rTrace = rVol + 2 * MT;        // [MTF]
   static constexpr int rFlux = rTrace + 2 * MTF;      // [MT][4]
-  static constexpr int rTotal = rFlux + 2 * 4 * MT;
+  static constexpr int rRt = rFlux + 2 * 4 * MT;      // [4][RT], in blocks of 8 columns
+  static constexpr int rTotal = rRt + 2 * 4 * RT;
 };
 
 // column stride of X: quads aligned to 16 bytes, and the 16 elements' columns
@@ -250,6 +258,9 @@ template <int O>
 struct Order {
   static int local(const EngineState& e, int parts, const double* coeffs, const sdg_layer* layer, bool traces,
                    const LtsOut* lts, hipStream_t stream);
+  // neighbour flux; gts / sub: time coefficients of the LTS pass (nullptr: global time stepping)
+  static int neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub,
+                      hipStream_t stream);
 };
 
 }  // namespace mx

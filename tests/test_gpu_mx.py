@@ -82,3 +82,45 @@ def test_local_pass_under_memory_load(gpu, arith, tol):
         run_local(eng, a, "lts", 0)
         sides.append(a)
     same(*sides, ("dofs", "integrated", "derivatives"), tol, f"{arith} n=50000")
+
+
+def run_neighbor(eng, a, lts):
+    import torch
+    time = (C.c_double * 8)(1.0, 0.5, 0.2, 0.1, 0.05, 0.02, 0.01, 0.005)
+    sub = (C.c_double * 8)(0.5, 0.4, 0.3, 0.2, 0.1, 0.05, 0.02, 0.01)
+    s, view = torch.cuda.current_stream().cuda_stream, C.byref(a["view"])
+    if lts:
+        check(lib().sdg_compute_neighboring_integration(eng.handle, time, sub, view, s), "neighbour lts")
+    else:
+        check(lib().sdg_compute_batched_neighbors_integral(eng.handle, view, s), "neighbour")
+    torch.cuda.synchronize()
+
+
+# n, alignment, sides drawn from [0, sides), LTS: one element; ragged; one side only (full
+# groups); every side; enough elements for every CU
+@pytest.mark.parametrize("arith,tol", [("fp64", 1e-12), ("fp32", 5e-5)])
+@pytest.mark.parametrize("order", [3, 4, 5, 6, 7])
+def test_neighbour_pass_equals_the_valu_kernels(gpu, order, arith, tol):
+    import torch
+    for n, align, sides, lts in ((1, 0, 4, False), (17, 128, 4, True), (333, 0, 1, False), (333, 0, 2, True),
+                                 (9001, 128, 4, True), (9001, 0, 4, False)):
+        print(f"mx neighbour {arith} order={order} n={n} align={align} sides={sides} lts={lts}", flush=True)
+        results = []
+        for family in ("auto", "valu"):
+            eng = Engine(order, arith)
+            eng.set_layout(align, "compact")
+            eng.set_kernels(family)
+            a = random_layer(eng, order, arith, n, align, "compact", 5 * order + n, setup=True)
+            gen = torch.Generator(device="cuda").manual_seed(n)
+            draw = lambda hi, shape, t: torch.randint(0, hi, shape, generator=gen, device="cuda").to(t)
+            a["neighbors"] = draw(n, (n, 4), torch.int32)
+            a["relations"] = torch.stack([draw(sides, (n, 4), torch.uint8), draw(3, (n, 4), torch.uint8)], -1)
+            a["types"] = (draw(8, (n, 4), torch.int32) == 0).to(torch.uint8)  # some dynamic-rupture faces
+            a["aminus"] = torch.rand((n, 4, 81), generator=gen, device="cuda", dtype=a["dofs"].dtype) * 2 - 1
+            a["setup"] = draw(1 << 11, (n,), torch.int16)
+            v = a["view"]
+            v.aminus, v.face_neighbors, v.face_relations = ptr(a["aminus"]), ptr(a["neighbors"]), ptr(a["relations"])
+            v.face_types, v.lts_setup = ptr(a["types"]), ptr(a["setup"])
+            run_neighbor(eng, a, lts)
+            results.append(a)
+        same(*results, ("dofs",), tol, f"neighbour n={n} lts={lts}")
