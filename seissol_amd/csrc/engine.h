@@ -68,8 +68,6 @@ struct EngineState {
   void* mfmaTables = nullptr;
   // dynamic rupture face matrices (V3mTo2n, V3mTo2nTWDivM), on first use
   void* drMatrices = nullptr;
-  // FP64 engines of orders 3-7: FP64 fragments of the matrix-core neighbour pass
-  void* mfma64Frags = nullptr;
   // SDG_KERNELS_AUTO: the matrix-core passes where the engine has them;
   // SDG_KERNELS_VALU: the VALU kernels only (sdg_engine_set_kernels)
   int kernels = SDG_KERNELS_AUTO;
@@ -137,11 +135,9 @@ int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const s
 bool hasNeighborMx(const EngineState& e);
 int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
                      const double* subtimeCoeffs, hipStream_t stream);
-// kernels_mfma64.hip: the FP64 neighbour pass on the matrix cores from the FP64
-// face traces the local pass wrote (layer->face_traces, [n][4][9][B2P])
-bool hasMfma64(const EngineState& e);
-int launchNeighborMfma64(const EngineState& e, const sdg_layer* layer, hipStream_t stream);
-int uploadMfma64(EngineState& s, const double* globalMatrices);
+// the same from the face traces the local pass wrote (layer->face_traces,
+// [n][4][9][B2P] in the real type)
+int launchNeighborTracesMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream);
 // the LTS local pass on the matrix cores: buffers and derivatives per the
 // layer's lts_setup (TimeCluster::computeLocalIntegration), no face traces
 int launchLocalIntegrationMfma(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,

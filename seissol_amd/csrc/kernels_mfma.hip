@@ -49,14 +49,18 @@ int launchLocalIntegrationMfma(const EngineState& e, const double* coeffs, const
 }
 
 int launchNeighborMfma(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  switch (e.order) {
-    case 3: return mfma::MfmaOrder<3>::neighbor(e, layer, stream);
-    case 4: return mfma::MfmaOrder<4>::neighbor(e, layer, stream);
-    case 5: return mfma::MfmaOrder<5>::neighbor(e, layer, stream);
-    case 6: return mfma::MfmaOrder<6>::neighbor(e, layer, stream);
-    case 7: return mfma::MfmaOrder<7>::neighbor(e, layer, stream);
-    default: setError("matrix-core path supports orders 3..7"); return SDG_ERR_UNSUPPORTED;
-  }
+  // The FP32 pass from the traces is the faster one (60k cells, random links,
+  // whole f16x3 step, split products -> FP32: ORDER 3 369 -> 171 us, ORDER 4
+  // 358 -> 280, ORDER 5 543 -> 448, ORDER 7 1120 -> 1001; bf16x6 ORDER 6 784 ->
+  // 761), except at ORDER 6 with two planes (f16x3 530 -> 519, but 7.98 ->
+  // 8.00 ms on 1M cells; bf16x3 459 -> 478).
+  if (e.order == mfma::kSplitNeighborOrder && e.arithmetic != SDG_BF16X6)
+    return mfma::MfmaOrder<mfma::kSplitNeighborOrder>::neighbor(e, layer, stream);
+  bool v4 = false;
+  if (!mfma::vectorAccess(cellLayout(e, layer), layer->dofs, nullptr, "matrix-core neighbour pass", v4) &&
+      layer->num_elements > 0)
+    return SDG_ERR_INVALID;
+  return launchNeighborTracesMx(e, layer, stream);
 }
 
 }  // namespace sdg

@@ -56,7 +56,9 @@ int uploadOrder(EngineState& s, const double* gm) {
   std::vector<int> ranges(G::rTotal, 0);
   const double tolT = largest(gm + g.kDivMT, 3LL * B * B), tolV = largest(gm + g.kDivM, 3LL * B * B);
   const double tolF = largest(gm + g.fMrT, 4LL * B * B2), tolR = largest(gm + g.rDivM, 4LL * B * B2);
-  bool sparseFP = true;  // a caller's own matrices may have fuller rows: no neighbour pass here then
+  // a caller's own matrices may have fuller rows: an FP32 engine has no
+  // neighbour pass here then, an FP64 engine refuses them
+  bool sparseFP = true;
   for (int t = 0; t < G::MT; ++t) {
     std::vector<Matrix> ck, vol;
     for (int j = 0; j < 3; ++j) {
@@ -124,6 +126,10 @@ int uploadOrder(EngineState& s, const double* gm) {
         const double v = gm[g.fP + (h * B2 + r) * B2 + c];
         if (std::fabs(v) <= tolP) continue;
         if (cnt == O) {
+          if (sizeof(real) == 8) {
+            setError("face permutation matrix with more than `order` non-zeros in a row");
+            return SDG_ERR_INVALID;
+          }
           sparseFP = false;
           break;
         }
@@ -174,7 +180,11 @@ bool hasNeighborMx(const EngineState& e) { return hasMx(e) && e.mxNeighbor; }
 
 int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
                      const double* subtimeCoeffs, hipStream_t stream) {
-  return orders(e, [&](auto o) { return o.neighbor(e, layer, timeCoeffs, subtimeCoeffs, stream); });
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, timeCoeffs, subtimeCoeffs, false, stream); });
+}
+
+int launchNeighborTracesMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, nullptr, nullptr, true, stream); });
 }
 
 int launchAderMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {

@@ -71,7 +71,7 @@ bool ltsLayerOk(const sdg_layer* L, bool neighbors, const char* who) {
 // variant is the matrix-core pass where the engine has it.
 // The FP64 engine (orders 3-7, kernel family AUTO) likewise has its FP64
 // matrix-core pass as variant 0.
-bool matrixCoreLocal(const EngineState& e) { return matrixCore(e.arithmetic) || hasMfma64(e); }
+bool matrixCoreLocal(const EngineState& e) { return matrixCore(e.arithmetic) || (e.arithmetic == SDG_FP64 && hasMx(e)); }
 int localVariants(const EngineState& e) { return matrixCoreLocal(e) ? 1 + kTileVariants : kTileVariants; }
 
 int runLocal(const EngineState& e, const double* coeffs, const sdg_layer* own, int reset, hipStream_t s, int v) {

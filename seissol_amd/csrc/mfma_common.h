@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <string>
 
 #include "engine.h"
 
@@ -67,6 +68,23 @@ struct LtsOut {
   int pad_ = 0;
 };
 
+// 16-byte DOF accesses: every block starts on a multiple of 4 reals and the
+// arrays are 16-byte aligned (always so for B a multiple of 4 on aligned arrays)
+inline bool vectorAccess(const CellLayout& lay, const void* dofs, const void* integ, const char* who, bool& v4) {
+  const bool aligned = (reinterpret_cast<uintptr_t>(dofs) % 16 == 0) &&
+                       (integ == nullptr || reinterpret_cast<uintptr_t>(integ) % 16 == 0);
+  v4 = lay.ldq % 4 == 0 && aligned;
+  if (lay.ldq % 4 == 0 && !aligned) {
+    setError(std::string(who) + ": dofs and time_integrated must be 16-byte aligned");
+    return false;
+  }
+  return true;
+}
+
+// the order at which the neighbour pass runs on split products (f16x3 and
+// bf16x3; every other one runs the FP32 pass of mx_neighbor.h)
+constexpr int kSplitNeighborOrder = 6;
+
 // host entry points of one order's kernels
 template <int O>
 struct MfmaOrder {
@@ -77,42 +95,4 @@ struct MfmaOrder {
 };
 
 }  // namespace mfma
-
-namespace mfma64 {
-using mfma::basis2;
-using mfma::basis3;
-using mfma::cdiv;
-using mfma::kCols;
-using mfma::kTileElems;
-
-constexpr int cceil4(int a) { return (a + 3) / 4 * 4; }
-
-// geometry of the FP64 neighbour kernel per order: one wave per basis row
-// tile; the face operand, the gathered traces, AminusT and the fP tables in LDS
-template <int O>
-struct Shape64 {
-  static constexpr int B = basis3(O);
-  static constexpr int B2 = basis2(O);
-  static constexpr int MT = cdiv(B, 16);        // row tiles of the basis index
-  static constexpr int B2P = cceil4(B2);        // face rows padded to a multiple of 4
-  static constexpr int KSF = B2P / 4;           // k-steps of one face's flux product
-  static constexpr int LDW = B2P + 2;           // doubles per W column of one face
-  static constexpr int NWAVES = MT;
-  static constexpr int NTHREADS = 64 * NWAVES;
-  // fragment offsets (doubles): one fragment = 64 lanes x 1 double; fP_h rows
-  // as O (value, column) entries
-  static constexpr int64_t rdmN = 0;                                // [MT][4][KSF], rDivM_f
-  static constexpr int64_t tFP = rdmN + 4LL * MT * KSF * 64;        // [3][B2][O] values
-  static constexpr int64_t tFPCol = tFP + 3LL * B2 * O;             // [3][B2][O] columns (exact integers)
-  static constexpr int64_t total = tFPCol + 3LL * B2 * O;
-};
-
-// host entry of one order's FP64 matrix-core neighbour pass
-template <int O>
-struct MfmaOrder64 {
-  static int neighbor(const EngineState& e, const sdg_layer* layer, hipStream_t stream);
-};
-// fragment count (doubles) of the FP64 matrix-core kernels of `order` (0: none)
-int64_t fragmentCount(int order);
-}  // namespace mfma64
 }  // namespace sdg

@@ -1045,19 +1045,6 @@ void launchVariants(bool v4, bool def, F&& launch) {
   else launch(std::true_type{}, std::false_type{});
 }
 
-// 16-byte DOF accesses: every block starts on a multiple of 4 reals and the
-// arrays are 16-byte aligned (always so for B a multiple of 4 on aligned arrays)
-inline bool vectorAccess(const CellLayout& lay, const void* dofs, const void* integ, const char* who, bool& v4) {
-  const bool aligned = (reinterpret_cast<uintptr_t>(dofs) % 16 == 0) &&
-                       (integ == nullptr || reinterpret_cast<uintptr_t>(integ) % 16 == 0);
-  v4 = lay.ldq % 4 == 0 && aligned;
-  if (lay.ldq % 4 == 0 && !aligned) {
-    setError(std::string(who) + ": dofs and time_integrated must be 16-byte aligned");
-    return false;
-  }
-  return true;
-}
-
 // lts == nullptr: the proxy/GTS local pass (traces written, derivatives never);
 // otherwise the LTS local pass: buffers and derivatives per the cells' setup,
 // traces written only when the layer has them
@@ -1124,11 +1111,10 @@ int localDispatch(const EngineState& e, const double* coeffs, const sdg_layer* l
 
 template <int O>
 int neighborDispatch(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  switch (e.arithmetic) {
-    case SDG_BF16X6: return neighborImpl<O, 3>(e, layer, stream);
-    case SDG_F16X3: return neighborImpl<O, 16>(e, layer, stream);
-    default: return neighborImpl<O, 2>(e, layer, stream);
-  }
+  if constexpr (O == kSplitNeighborOrder)
+    return e.arithmetic == SDG_F16X3 ? neighborImpl<O, 16>(e, layer, stream) : neighborImpl<O, 2>(e, layer, stream);
+  setError("the split-product neighbour pass is built for one order");
+  return SDG_ERR_UNSUPPORTED;
 }
 
 }  // namespace

@@ -258,8 +258,9 @@ template <int O>
 struct Order {
   static int local(const EngineState& e, int parts, const double* coeffs, const sdg_layer* layer, bool traces,
                    const LtsOut* lts, hipStream_t stream);
-  // neighbour flux; gts / sub: time coefficients of the LTS pass (nullptr: global time stepping)
-  static int neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub,
+  // neighbour flux; gts / sub: time coefficients of the LTS pass (nullptr: global time stepping);
+  // traces: from the layer's face traces instead of the neighbours' DOFs
+  static int neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub, bool traces,
                       hipStream_t stream);
 };
 

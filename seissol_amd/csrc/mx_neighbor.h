@@ -1,16 +1,19 @@
-// Neighbour flux from the neighbours' time-integrated DOFs on the matrix cores
-// in the engine's real type (Neighbor.cpp:66-109, TimeCommon.cpp:40-87; spec
+// Neighbour flux on the matrix cores in the engine's real type
+// (Neighbor.cpp:66-109, TimeCommon.cpp:40-87; spec
 // codegen/kernels/aderdg.py:414-431), global and local time stepping:
-// Q += sum_f rDivM_f ((fP_h (rT_j I_nb)) AminusT_f).
+// Q += sum_f rDivM_f ((fP_h U_f) AminusT_f) with U_f = rT_j I_nb, formed here
+// from the neighbours' time-integrated DOFs or read as the face traces that
+// the local pass wrote.
 //
 // A workgroup handles a tile of 16 elements, that is 64 tasks (element, face),
 // in three phases:
-//  1. U = rT_j I_nb.  The tasks are sorted by the side j of their neighbour
+//  1. U.  From DOFs: the tasks are sorted by the side j of their neighbour
 //     into groups of 16 with one j each, so that rT_j is the stationary
 //     operand of a matrix instruction whose 16 columns are one quantity of
 //     16 tasks.  The neighbours' DOFs go from global memory straight into the
 //     operand registers (each value feeds one or two row tiles only, LDS would
 //     not be reused); a group is split over three waves by quantities.
+//     From traces: copied to LDS, every load of the tile in flight at once.
 //  2. W = (fP_h U) AminusT_f per task on 16 lanes, in place of U: fP_h as rows
 //     of at most ORDER non-zeros, AminusT read once per task and broadcast
 //     across its lanes (DPP row_newbcast).
@@ -19,6 +22,10 @@
 // workgroup of eight waves per CU; 56 KB in FP32), which leaves two barriers
 // per tile.  Bound by the matrix instructions (FP64) or, on random links, by
 // the gather of four neighbours' DOFs per element.
+// From traces this replaced a kernel that went face by face, nine barriers a
+// tile, one wave per row tile: FP64 steps of 60k cells 608 -> 286 us at ORDER
+// 3, 487 -> 428 at 4, 793 -> 721 at 5, 2148 -> 1952 at 7; 400k cells at ORDER
+// 6 7.34 -> 7.11 ms; 500 cells at ORDER 4 52 -> 35 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -65,7 +72,11 @@ __device__ inline void loadPair(const real* __restrict__ q, int row, real (&v)[2
   }
 }
 
-template <typename real, int O, bool LTS>
+// what the neighbour pass reads: the neighbours' buffers, buffers or
+// derivatives (local time stepping), or the face traces rT_j I of the local pass
+constexpr int kFromDofs = 0, kFromLts = 1, kFromTraces = 2;
+
+template <typename real, int O, int SRC>
 __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, real>::SIMD_WAVES)) void kNeighborMx(
     int64_t n, const real* __restrict__ frag, const int* __restrict__ ranges, real* __restrict__ dofs,
     const real* __restrict__ integ, const real* __restrict__ deriv, const int32_t* __restrict__ neighbors,
@@ -75,6 +86,7 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
   using N = NeighborGeo<O, real>;
   using V4 = typename Vec<real>::V4;
   constexpr int B = G::B, B2 = G::B2, B2P = G::B2P, FS = N::FS, ES = N::ES, RS = sizeof(real);
+  constexpr bool LTS = SRC == kFromLts;
   __shared__ __attribute__((aligned(16))) real sU[kElems * ES];  // U, then W: [element][face][quantity][B2P]
   __shared__ real sFP[3 * B2 * O];
   __shared__ int sFPCol[3 * B2 * O];
@@ -107,115 +119,137 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
     }
     sNb[lane] = regular ? nb : 0;
     sMeta[lane] = meta;
-    sSlot[lane] = -1;
-    if (lane < N::MAXGROUPS * 16 - 64) sSlot[64 + lane] = -1;
-    waveSync();
-    int group = 0;
+    if constexpr (SRC == kFromTraces) {
+      sSlot[lane] = regular ? side : -1;
+    } else {
+      sSlot[lane] = -1;
+      if (lane < N::MAXGROUPS * 16 - 64) sSlot[64 + lane] = -1;
+      waveSync();
+      int group = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint64_t mask = __ballot(regular && side == j);
-      const int before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
-                                                   __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
-      if (regular && side == j) sSlot[16 * group + before] = lane;
-      const int groups = (__popcll(mask) + 15) / 16;
-      if (lane < groups) sSide[group + lane] = j;
-      group += groups;
+      for (int j = 0; j < 4; ++j) {
+        const uint64_t mask = __ballot(regular && side == j);
+        const int before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
+        if (regular && side == j) sSlot[16 * group + before] = lane;
+        const int groups = (__popcll(mask) + 15) / 16;
+        if (lane < groups) sSide[group + lane] = j;
+        group += groups;
+      }
+      if (lane == 0) sSide[N::MAXGROUPS] = group;
     }
-    if (lane == 0) sSide[N::MAXGROUPS] = group;
   }
   __syncthreads();
 
-  // phase 1: units of (group, three quantities)
-  const int units = 3 * __builtin_amdgcn_readfirstlane(sSide[N::MAXGROUPS]);
+  if constexpr (SRC == kFromTraces) {
+    // phase 1: the traces [neighbour][side][quantity][B2P], every load of a
+    // thread in flight before its first store
+    constexpr int TR4 = FS / 4, N4 = cdiv(64 * TR4, N::THREADS);
+    V4 v[N4];
+#pragma unroll
+    for (int u = 0; u < N4; ++u) {
+      const int i = min(static_cast<int>(threadIdx.x) + u * N::THREADS, 64 * TR4 - 1), t = i / TR4;
+      const int side = max(sSlot[t], 0);  // a task without a neighbour reads cell 0's first trace; its W is zero
+      v[u] = *reinterpret_cast<const V4*>(integ + (static_cast<int64_t>(sNb[t]) * 4 + side) * FS + 4 * (i % TR4));
+    }
+#pragma unroll
+    for (int u = 0; u < N4; ++u) {
+      const int i = threadIdx.x + u * N::THREADS, t = i / TR4;
+      if (i < 64 * TR4) *reinterpret_cast<V4*>(sU + (t >> 2) * ES + (t & 3) * FS + 4 * (i % TR4)) = v[u];
+    }
+  } else {
+    // phase 1: units of (group, three quantities)
+    const int units = 3 * __builtin_amdgcn_readfirstlane(sSide[N::MAXGROUPS]);
 #pragma unroll 1
-  for (int u = w; u < units; u += N::WAVES) {
-    const int group = u / 3, q0 = 3 * (u % 3);
-    const int j = __builtin_amdgcn_readfirstlane(sSide[group]);
-    const int task = sSlot[16 * group + c];
-    const int t = task < 0 ? 0 : task;
-    const int64_t nb = task < 0 ? 0 : sNb[t];
-    // the neighbour's time integral: its buffer, or its derivatives integrated
-    // over this step (GTS relation: time coefficients, else the sub-interval's)
-    [[maybe_unused]] bool fromDeriv = false;
-    [[maybe_unused]] bool gts = false;
-    if constexpr (LTS) {
-      const int meta = sMeta[t];
-      fromDeriv = task >= 0 && (meta >> 3 & 1);
-      gts = meta >> 4 & 1;
-    }
-    real x[G::KB8][3][2];
-    {
-      const real* const src = integ + nb * lay.qStride + q0 * lay.ldq;
-#pragma unroll
-      for (int k = 0; k < G::KB8; ++k)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) loadPair<B>(src + q * lay.ldq, 8 * k + 2 * g, x[k][q]);
-    }
-    if constexpr (LTS) {
-      if (__ballot(fromDeriv) != 0) {
-        const real* src = deriv + nb * lay.dsize;
-        real y[G::KB8][3][2];
-#pragma unroll
-        for (int k = 0; k < G::KB8; ++k)
-#pragma unroll
-          for (int q = 0; q < 3; ++q) y[k][q][0] = y[k][q][1] = real(0);
-        staticFor<O>([&](auto dI) {
-          constexpr int d = decltype(dI)::value, m = basis3(O - d);
-          const int ldm = lay.rows(m);
-          const real cd = gts ? cf.gts[d] : cf.sub[d];
-#pragma unroll
-          for (int k = 0; k < cdiv(m, 8); ++k)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-              real v[2];
-              if constexpr (m >= 2) {
-                loadPair<m>(src + (q0 + q) * ldm, 8 * k + 2 * g, v);
-              } else {
-                const real v0 = src[(q0 + q) * ldm];
-                v[0] = g == 0 ? v0 : real(0);
-                v[1] = real(0);
-              }
-              y[k][q][0] += cd * v[0];
-              y[k][q][1] += cd * v[1];
-            }
-          src += 9LL * ldm;
-        });
-#pragma unroll
-        for (int k = 0; k < G::KB8; ++k)
-#pragma unroll
-          for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) x[k][q][i] = fromDeriv ? y[k][q][i] : x[k][q][i];
+    for (int u = w; u < units; u += N::WAVES) {
+      const int group = u / 3, q0 = 3 * (u % 3);
+      const int j = __builtin_amdgcn_readfirstlane(sSide[group]);
+      const int task = sSlot[16 * group + c];
+      const int t = task < 0 ? 0 : task;
+      const int64_t nb = task < 0 ? 0 : sNb[t];
+      // the neighbour's time integral: its buffer, or its derivatives integrated
+      // over this step (GTS relation: time coefficients, else the sub-interval's)
+      [[maybe_unused]] bool fromDeriv = false;
+      [[maybe_unused]] bool gts = false;
+      if constexpr (LTS) {
+        const int meta = sMeta[t];
+        fromDeriv = task >= 0 && (meta >> 3 & 1);
+        gts = meta >> 4 & 1;
       }
-    }
-    V4 acc[G::RT][3];
+      real x[G::KB8][3][2];
+      {
+        const real* const src = integ + nb * lay.qStride + q0 * lay.ldq;
 #pragma unroll
-    for (int r = 0; r < G::RT; ++r)
+        for (int k = 0; k < G::KB8; ++k)
 #pragma unroll
-      for (int q = 0; q < 3; ++q) acc[r][q] = V4{0, 0, 0, 0};
-    typedef real V2 __attribute__((ext_vector_type(2)));
+          for (int q = 0; q < 3; ++q) loadPair<B>(src + q * lay.ldq, 8 * k + 2 * g, x[k][q]);
+      }
+      if constexpr (LTS) {
+        if (__ballot(fromDeriv) != 0) {
+          const real* src = deriv + nb * lay.dsize;
+          real y[G::KB8][3][2];
 #pragma unroll
-    for (int r = 0; r < G::RT; ++r) {
-      const V2* const fr =
-          reinterpret_cast<const V2*>(frag + G::rt + (static_cast<int64_t>(j) * G::RT + r) * G::KB8 * 128) + lane;
-      const int lo = ranges[G::rRt + 2 * (j * G::RT + r)], hi = ranges[G::rRt + 2 * (j * G::RT + r) + 1];
+          for (int k = 0; k < G::KB8; ++k)
 #pragma unroll
-      for (int k = 0; k < G::KB8; ++k)
-        if (k >= lo && k < hi) {  // uniform
-          const V2 a = fr[k * 64];
+            for (int q = 0; q < 3; ++q) y[k][q][0] = y[k][q][1] = real(0);
+          staticFor<O>([&](auto dI) {
+            constexpr int d = decltype(dI)::value, m = basis3(O - d);
+            const int ldm = lay.rows(m);
+            const real cd = gts ? cf.gts[d] : cf.sub[d];
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+            for (int k = 0; k < cdiv(m, 8); ++k)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) acc[r][q] = mma(a[i], x[k][q][i], acc[r][q]);
+              for (int q = 0; q < 3; ++q) {
+                real v[2];
+                if constexpr (m >= 2) {
+                  loadPair<m>(src + (q0 + q) * ldm, 8 * k + 2 * g, v);
+                } else {
+                  const real v0 = src[(q0 + q) * ldm];
+                  v[0] = g == 0 ? v0 : real(0);
+                  v[1] = real(0);
+                }
+                y[k][q][0] += cd * v[0];
+                y[k][q][1] += cd * v[1];
+              }
+            src += 9LL * ldm;
+          });
+#pragma unroll
+          for (int k = 0; k < G::KB8; ++k)
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+              for (int i = 0; i < 2; ++i) x[k][q][i] = fromDeriv ? y[k][q][i] : x[k][q][i];
         }
-    }
-    if (task >= 0) {
-      real* const out = sU + (task >> 2) * ES + (task & 3) * FS + q0 * B2P + 4 * g;
+      }
+      V4 acc[G::RT][3];
 #pragma unroll
       for (int r = 0; r < G::RT; ++r)
-        if (16 * r + 4 * g < B2P)
 #pragma unroll
-          for (int q = 0; q < 3; ++q) *reinterpret_cast<V4*>(out + q * B2P + 16 * r) = acc[r][q];
+        for (int q = 0; q < 3; ++q) acc[r][q] = V4{0, 0, 0, 0};
+      typedef real V2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+      for (int r = 0; r < G::RT; ++r) {
+        const V2* const fr =
+            reinterpret_cast<const V2*>(frag + G::rt + (static_cast<int64_t>(j) * G::RT + r) * G::KB8 * 128) + lane;
+        const int lo = ranges[G::rRt + 2 * (j * G::RT + r)], hi = ranges[G::rRt + 2 * (j * G::RT + r) + 1];
+#pragma unroll
+        for (int k = 0; k < G::KB8; ++k)
+          if (k >= lo && k < hi) {  // uniform
+            const V2 a = fr[k * 64];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int q = 0; q < 3; ++q) acc[r][q] = mma(a[i], x[k][q][i], acc[r][q]);
+          }
+      }
+      if (task >= 0) {
+        real* const out = sU + (task >> 2) * ES + (task & 3) * FS + q0 * B2P + 4 * g;
+#pragma unroll
+        for (int r = 0; r < G::RT; ++r)
+          if (16 * r + 4 * g < B2P)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *reinterpret_cast<V4*>(out + q * B2P + 16 * r) = acc[r][q];
+      }
     }
   }
   __syncthreads();
@@ -299,7 +333,8 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
 }
 
 template <typename real, int O>
-int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, const double* sub, hipStream_t stream) {
+int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, const double* sub, bool traces,
+                 hipStream_t stream) {
   using N = NeighborGeo<O, real>;
   const int64_t n = L->num_elements;
   if (n == 0) return SDG_OK;
@@ -311,14 +346,16 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, c
     }
   const CellLayout lay = cellLayout(st, L);
   const dim3 grid(static_cast<unsigned>((n + kElems - 1) / kElems));
-  auto launch = [&](auto ltsI) {
-    kNeighborMx<real, O, decltype(ltsI)::value><<<grid, N::THREADS, 0, stream>>>(
+  auto launch = [&](auto srcI) {
+    kNeighborMx<real, O, decltype(srcI)::value><<<grid, N::THREADS, 0, stream>>>(
         n, static_cast<const real*>(st.mxFrags), st.mxRanges, static_cast<real*>(L->dofs),
-        static_cast<const real*>(L->time_integrated), static_cast<const real*>(L->derivatives), L->face_neighbors,
-        L->face_relations, static_cast<const real*>(L->aminus), L->face_types, L->lts_setup, cf, lay);
+        static_cast<const real*>(traces ? L->face_traces : L->time_integrated),
+        static_cast<const real*>(L->derivatives), L->face_neighbors, L->face_relations,
+        static_cast<const real*>(L->aminus), L->face_types, L->lts_setup, cf, lay);
   };
-  if (gts != nullptr && L->lts_setup != nullptr) launch(std::true_type{});
-  else launch(std::false_type{});
+  if (traces) launch(std::integral_constant<int, kFromTraces>{});
+  else if (gts != nullptr && L->lts_setup != nullptr) launch(std::integral_constant<int, kFromLts>{});
+  else launch(std::integral_constant<int, kFromDofs>{});
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;
 }
@@ -326,10 +363,10 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, c
 }  // namespace
 
 template <int O>
-int Order<O>::neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub,
+int Order<O>::neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub, bool traces,
                        hipStream_t stream) {
-  return e.arithmetic == SDG_FP64 ? neighborImpl<double, O>(e, layer, gts, sub, stream)
-                                  : neighborImpl<float, O>(e, layer, gts, sub, stream);
+  return e.arithmetic == SDG_FP64 ? neighborImpl<double, O>(e, layer, gts, sub, traces, stream)
+                                  : neighborImpl<float, O>(e, layer, gts, sub, traces, stream);
 }
 
 }  // namespace mx

@@ -342,12 +342,12 @@ int proxyRun(const EngineState& st, int kernel_id, int steps, double dt, const s
   // the FP64 matrix-core passes hand FP64 face traces from the local pass to
   // the neighbour pass (the local pass still writes I); as for the
   // matrix-core forms, `neigh` alone reads the traces of the last local pass
-  const bool mc64 = hasMfma64(st) && layer->face_traces != nullptr;
+  const bool mc64 = st.arithmetic == SDG_FP64 && hasNeighborMx(st) && layer->face_traces != nullptr;
   for (int step = 0; step < steps; ++step) {
     int rc = SDG_OK;
     if (mc64 && kernel_id <= 2) {
       if (kernel_id == 0 || kernel_id == 1) rc = launchAderLocal(st, coeffs, layer, s);
-      if (rc == SDG_OK && (kernel_id == 0 || kernel_id == 2)) rc = launchNeighborMfma64(st, layer, s);
+      if (rc == SDG_OK && (kernel_id == 0 || kernel_id == 2)) rc = launchNeighborTracesMx(st, layer, s);
       if (rc != SDG_OK) return rc;
       continue;
     }
@@ -515,13 +515,11 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic) {
   generateGlobalMatrices(order, gm.data());
   int rc = uploadMatrices(e->s, gm.data());
   if (rc == SDG_OK && matrixCore(arithmetic)) rc = uploadMfma(e->s, gm.data());
-  if (rc == SDG_OK && arithmetic == SDG_FP64) rc = uploadMfma64(e->s, gm.data());
   if (rc == SDG_OK) rc = uploadMx(e->s, gm.data());
   if (rc != SDG_OK) {
     if (e->s.matrices) (void)hipFree(e->s.matrices);
     if (e->s.mfmaFrags) (void)hipFree(e->s.mfmaFrags);
     if (e->s.mfmaTables) (void)hipFree(e->s.mfmaTables);
-    if (e->s.mfma64Frags) (void)hipFree(e->s.mfma64Frags);
     if (e->s.mxFrags) (void)hipFree(e->s.mxFrags);
     if (e->s.mxRanges) (void)hipFree(e->s.mxRanges);
     delete e;
@@ -534,11 +532,9 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic) {
 int sdg_engine_set_global_matrices(sdg_engine* engine, const double* host_matrices) {
   if (engine == nullptr || host_matrices == nullptr) { setError("invalid arguments"); return SDG_ERR_INVALID; }
   int rc = uploadMatrices(engine->s, host_matrices);
+  if (rc == SDG_OK && matrixCore(engine->s.arithmetic)) rc = uploadMfma(engine->s, host_matrices);
   if (rc == SDG_OK) rc = uploadMx(engine->s, host_matrices);
-  if (rc != SDG_OK) return rc;
-  if (engine->s.arithmetic == SDG_FP64) return uploadMfma64(engine->s, host_matrices);
-  if (!matrixCore(engine->s.arithmetic)) return rc;
-  return uploadMfma(engine->s, host_matrices);
+  return rc;
 }
 
 int sdg_engine_set_kernels(sdg_engine* engine, int family) {
@@ -585,7 +581,6 @@ int sdg_engine_destroy(sdg_engine* engine) {
   if (engine->s.mfmaFrags) SDG_HIP_CHECK(hipFree(engine->s.mfmaFrags));
   if (engine->s.mfmaTables) SDG_HIP_CHECK(hipFree(engine->s.mfmaTables));
   if (engine->s.drMatrices) SDG_HIP_CHECK(hipFree(engine->s.drMatrices));
-  if (engine->s.mfma64Frags) SDG_HIP_CHECK(hipFree(engine->s.mfma64Frags));
   if (engine->s.mxFrags) SDG_HIP_CHECK(hipFree(engine->s.mxFrags));
   if (engine->s.mxRanges) SDG_HIP_CHECK(hipFree(engine->s.mxRanges));
   delete engine;

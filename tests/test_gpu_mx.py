@@ -8,7 +8,7 @@ import pytest
 
 from seissol_amd import _capi
 from seissol_amd._capi import check, lib, ptr
-from seissol_amd.kernels import Engine
+from seissol_amd.kernels import Engine, global_matrices, num_basis, num_face_basis, padded_face_basis
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +124,44 @@ def test_neighbour_pass_equals_the_valu_kernels(gpu, order, arith, tol):
             run_neighbor(eng, a, lts)
             results.append(a)
         same(*results, ("dofs",), tol, f"neighbour n={n} lts={lts}")
+
+
+# the neighbour pass from face traces (global time stepping); the sums have at
+# most O + 9 + 4 * 28 = 128 terms: 128 roundings of 2^-53 / 2^-24
+@pytest.mark.parametrize("arith,order,tol", [(a, o, t) for a, t, orders in (
+    ("fp64", 1.5e-14, (3, 4, 5, 6, 7)), ("f16x3", 8e-6, (3, 4, 5, 7)), ("bf16x6", 8e-6, (3, 6))) for o in orders])
+def test_neighbour_pass_from_traces(gpu, arith, order, tol):
+    import torch
+    gm = {k: torch.from_numpy(v).cuda() for k, v in global_matrices(order).items() if k in ("rDivM", "fP")}
+    B2, B2P = num_face_basis(order), padded_face_basis(order)
+    for n, align, dr in ((1, 0, False), (17, 128, True), (333, 0, True), (9001, 0, False)):
+        print(f"traces {arith} order={order} n={n} align={align}", flush=True)
+        eng = Engine(order, arith)
+        eng.set_layout(align, "compact")
+        a = random_layer(eng, order, arith, n, align, "compact", 3 * order + n)
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        draw = lambda hi, shape, t: torch.randint(0, hi, shape, generator=gen, device="cuda").to(t)
+        rt = a["dofs"].dtype
+        nb, side, h = draw(n, (n, 4), torch.int32), draw(4, (n, 4), torch.uint8), draw(3, (n, 4), torch.uint8)
+        types = (draw(8, (n, 4), torch.int32) == 0).to(torch.uint8) if dr else None
+        relations = torch.stack([side, h], -1)
+        aminus = torch.rand((n, 4, 81), generator=gen, device="cuda", dtype=rt) * 2 - 1
+        traces = torch.rand((n, 4, 9, B2P), generator=gen, device="cuda", dtype=rt) * 2 - 1
+        v = a["view"]
+        v.aminus, v.face_neighbors, v.face_relations = ptr(aminus), ptr(nb), ptr(relations)
+        v.face_types, v.face_traces = ptr(types), ptr(traces)
+        B = num_basis(order)
+        want = a["dofs"][:, :, :B].double()
+        for f in range(4):
+            u = traces[nb[:, f].long(), side[:, f].long()][:, :, :B2].double()  # [n][q][m]
+            u = (gm["fP"][h[:, f].long()] @ u.transpose(1, 2).contiguous()).transpose(1, 2).contiguous()
+            w = aminus[:, f].reshape(n, 9, 9).double() @ u                       # [n][p][m]
+            if dr:
+                w[types[:, f] != 0] = 0
+            want = want + w @ gm["rDivM"][f].T.contiguous()
+        check(lib().sdg_proxy_run(eng.handle, 2, 1, 1e-3, C.byref(v), torch.cuda.current_stream().cuda_stream), "neigh")
+        torch.cuda.synchronize()
+        got = a["dofs"][:, :, :B].double()
+        err = float((got - want).abs().max() / want.abs().max())
+        print(f"  largest difference / largest value {err:.1e}", flush=True)
+        assert err < tol
