@@ -207,6 +207,11 @@ int launchAderLocalMx(const EngineState& e, const double* coeffs, const sdg_laye
   });
 }
 
+int launchLocalTracesMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, const mx::LtsOut* lts,
+                        hipStream_t stream) {
+  return orders(e, [&](auto o) { return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, true, lts, stream); });
+}
+
 int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
                              hipStream_t stream) {
   const mx::LtsOut lts{layer->lts_setup, layer->derivatives, resetBuffers, 0};

@@ -20,7 +20,9 @@ constexpr int maxOf(int a, int b) { return a > b ? a : b; }
 constexpr int kElems = 16;         // elements per tile: the columns of one matrix instruction
 constexpr int kCols = 9 * kElems;  // GEMM columns (quantity, element) -> 16 q + e
 constexpr int kStarLd = 73;        // an element's 72 star values, padded against bank conflicts
-constexpr int kAplusLd = 325;      // an element's 4 x 81 AplusT values, padded likewise
+// an element's 4 x 81 AplusT values: 16-byte pieces aligned, conflict-free
+template <typename real>
+constexpr int kAplusLd = sizeof(real) == 8 ? 326 : 324;
 
 // where the compact star values (24 per direction) of output quantity p lie,
 // and the input quantities they multiply
@@ -55,14 +57,6 @@ struct Geo {
   static constexpr int traceRow(int t, int g) {
     return B2P <= 8 ? 4 * (g % 2) : (t < 4 ? 4 * g : (B2P <= 24 ? 16 + 4 * (g % 2) : 16 + 4 * g));
   }
-  // Waves of the local pass: a pair shares the row tiles pair and
-  // 2 PAIRS - 1 - pair (low tiles have the long products of the predictor,
-  // high ones those of the volume); its first wave forms the stresses, its
-  // second the velocities, which cost the same (see mx_local.h).
-  static constexpr int PAIRS = O == 3 ? 1 : (O == 7 ? 4 : 2);
-  static constexpr int WAVES = 2 * PAIRS, THREADS = 64 * WAVES;
-  static constexpr int TW = MT > PAIRS ? 2 : 1;       // row tiles per wave
-  static constexpr int TT = MTF > WAVES ? 2 : 1;      // trace tiles per wave
   // rows of the X area: the DOFs; dQ_1 and, behind it, dQ_2; two faces' W
   static constexpr int R1 = ceil4(basis3(O - 1)), R2 = O > 2 ? ceil4(basis3(O - 2)) : 0;
   static constexpr int XROWS = maxOf(maxOf(KB, R1 + R2), 2 * B2P);
@@ -188,6 +182,17 @@ struct Buffer {
       __builtin_amdgcn_raw_buffer_store_b128(x.u, rsrc, off, 0, 0);
     }
   }
+  // 16 bytes at byte offset `off`
+  __device__ inline auto load16(int off) const {
+    typedef unsigned U4 __attribute__((ext_vector_type(4)));
+    typedef real VP __attribute__((ext_vector_type(16 / sizeof(real))));
+    union {
+      U4 u;
+      VP v;
+    } x;
+    x.u = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
+    return x.v;
+  }
   __device__ inline real load1(int off, int s) const {
     if constexpr (sizeof(real) == 8) {
       typedef unsigned U2 __attribute__((ext_vector_type(2)));
@@ -265,4 +270,10 @@ struct Order {
 };
 
 }  // namespace mx
+
+// the fused local pass in FP32 or FP64 writing the layer's face traces, with
+// the outputs of `lts` (nullptr: neither derivatives nor LTS setup; a layer
+// without time_integrated: no buffer)
+int launchLocalTracesMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, const mx::LtsOut* lts,
+                        hipStream_t stream);
 }  // namespace sdg
