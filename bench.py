@@ -480,9 +480,8 @@ def main(argv=None) -> int:
         "vs_baseline": None,
         "plain_fp64": plain,
         "speedup_vs_plain_fp64": (value / plain["value"]) if plain else None,
-        "dtype": {"fp64": "f64", "fp32": "f32", "bf16x3": "f32 (2-plane split-bf16 MFMA, f32 accumulate)",
-                  "bf16x6": "f32 (3-plane split-bf16 MFMA, f32 accumulate)",
-                  "f16x3": "f32 (2-plane split-fp16 MFMA on power-of-two scaled operands, f32 accumulate)"}[args.form],
+        "dtype": "f64" if args.form == "fp64" else (
+            "f32 (2-plane split-bf16 MFMA, f32 accumulate)" if args.form == "bf16x3" and args.order >= 6 else "f32"),
         "data": "synthetic",
         "config": {"workload": f"elastic ADER-DG element update (proxy `all`), ORDER {args.order}, "
                                f"{setup.n} tetrahedra, {args.mesh} mesh, {args.form}, {args.star} star, "
@@ -495,15 +494,15 @@ def main(argv=None) -> int:
                      "traffic": traffic, "bytes_per_element": ab[dom],
                      "launch_ms": per_kernel[dom], "other_launch_ms": {k: v for k, v in per_kernel.items() if k != dom},
                      "matrix_core": {
-                         # dense peaks: fp16/bf16 2.5 PFLOP/s; FP64 78.6 TFLOP/s (the FP64 engine's
-                         # matrix-core pass, orders 3-7); the FP32 form runs on the VALU
-                         "peak_tflops": 2500.0 if args.form in ("bf16x3", "bf16x6", "f16x3")
-                         else (78.6 if args.form == "fp64" and 3 <= args.order <= 7 else None),
+                         # dense peaks: bf16 2.5 PFLOP/s (split products); FP32 157.3 and FP64 78.6
+                         # TFLOP/s (the matrix-core passes in the real type, orders 3-7)
+                         "peak_tflops": 2500.0 if args.form == "bf16x3" and args.order >= 6
+                         else (None if not 3 <= args.order <= 7 else 78.6 if args.form == "fp64" else 157.3),
                          # counter-measured (rocprofv3 MFMA_MOPS x 512 per launch) over this run's launch time
                          "achieved_tflops": (mfma["flop"] / (per_kernel[dom] / 1e3) / 1e12) if mfma else None,
                          "busy_frac": mfma["busy_frac"] if mfma else None,
                          "counter_source": mfma["source"] if mfma else None,
-                         # the dense contractions x split products (sdg_performance_estimate)
+                         # the dense contractions x the form's split products (sdg_performance_estimate)
                          "estimate_tflops": mma_tflops, "estimate_flop_per_element": est.hardware_flop}},
     }
     if not args.no_cpu:

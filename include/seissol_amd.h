@@ -28,11 +28,12 @@ extern "C" {
 
 /* arithmetic of the element-update kernels */
 #define SDG_FP64 0   /* plain FP64: the drop-in for the reference GPU path */
-#define SDG_FP32 1   /* FP32 storage and VALU arithmetic                    */
-#define SDG_BF16X3 2 /* FP32 storage, MFMA with 2-plane bf16 splits (3 products), FP32 accumulate */
-#define SDG_BF16X6 3 /* FP32 storage, MFMA with 3-plane bf16 splits (6 products), FP32 accumulate */
-#define SDG_F16X3 4  /* FP32 storage, MFMA with 2-plane fp16 splits of power-of-two scaled operands
-                        (3 products), FP32 accumulate */
+#define SDG_FP32 1   /* FP32 storage and arithmetic                         */
+/* FP32 storage and face traces between the passes, FP32 accumulation, products
+ * of at least the named accuracy: FP32 ones wherever they are the faster */
+#define SDG_BF16X3 2 /* 2-plane bf16 splits, about 2^-17 (split products at orders 6 and 7) */
+#define SDG_BF16X6 3 /* 3-plane bf16 splits, about 2^-24 (FP32 products at every order)      */
+#define SDG_F16X3 4  /* 2-plane fp16 splits, about 2^-21 (FP32 products at every order)      */
 
 /* storage of the per-cell star matrices (sdg_engine_set_layout) */
 #define SDG_STAR_DENSE 0   /* [3][81]: three 9x9 column-major matrices                          */

@@ -63,7 +63,7 @@ struct EngineState {
   int starFormat = SDG_STAR_DENSE;
   void* matrices = nullptr;  // device, real type of the engine
   DeviceMatrixLayout layout{};
-  // matrix-core arithmetics: pre-split 16-bit fragments and FP32 tables
+  // split-product engines: pre-split bf16 fragments and FP32 tables
   void* mfmaFrags = nullptr;
   void* mfmaTables = nullptr;
   // dynamic rupture face matrices (V3mTo2n, V3mTo2nTWDivM), on first use
@@ -115,7 +115,6 @@ int defaultNeighborVariant(const EngineState& e);
 int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs, const double* subtimeCoeffs,
                                  const sdg_layer* layer, hipStream_t stream, int variant = 0);
 // kernels_mfma.hip
-int64_t mfmaFragmentCount(int order);
 int launchLocalMfma(const EngineState& e, const double* coeffs, const sdg_layer* layer, bool writeIntegrated,
                     hipStream_t stream);
 int launchNeighborMfma(const EngineState& e, const sdg_layer* layer, hipStream_t stream);

@@ -57,7 +57,7 @@ int uploadOrder(EngineState& s, const double* gm) {
   const double tolT = largest(gm + g.kDivMT, 3LL * B * B), tolV = largest(gm + g.kDivM, 3LL * B * B);
   const double tolF = largest(gm + g.fMrT, 4LL * B * B2), tolR = largest(gm + g.rDivM, 4LL * B * B2);
   // a caller's own matrices may have fuller rows: an FP32 engine has no
-  // neighbour pass here then, an FP64 engine refuses them
+  // neighbour pass here then, every other one refuses them
   bool sparseFP = true;
   for (int t = 0; t < G::MT; ++t) {
     std::vector<Matrix> ck, vol;
@@ -126,7 +126,7 @@ int uploadOrder(EngineState& s, const double* gm) {
         const double v = gm[g.fP + (h * B2 + r) * B2 + c];
         if (std::fabs(v) <= tolP) continue;
         if (cnt == O) {
-          if (sizeof(real) == 8) {
+          if (sizeof(real) == 8 || matrixCore(s.arithmetic)) {
             setError("face permutation matrix with more than `order` non-zeros in a row");
             return SDG_ERR_INVALID;
           }

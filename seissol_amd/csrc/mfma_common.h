@@ -15,10 +15,10 @@ constexpr int basis3(int o) { return o * (o + 1) * (o + 2) / 6; }
 constexpr int basis2(int o) { return o * (o + 1) / 2; }
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// 16-bit elements (bf16 or fp16) of one (m-tile, k-step) fragment set: 64
-// lanes x 8 values for each of three split planes, one plane after the other.
+// bf16 elements of one (m-tile, k-step) fragment set: 64 lanes x 8 values for
+// each of the two planes, one plane after the other.
 constexpr int kFragPlane = 512;
-constexpr int kFragPair = 3 * kFragPlane;
+constexpr int kFragPair = 2 * kFragPlane;
 constexpr int kTileElems = 16;        // elements per workgroup tile
 constexpr int kCols = 9 * kTileElems; // GEMM columns (quantity, element)
 
@@ -45,15 +45,10 @@ struct MShape {
   // rDivM_f one face at a time: k-step f holds face f's B2 columns, zero-padded to 32
   static constexpr int64_t rdmF = rdm + 1LL * MT * KSF * kFragPair;  // [MT][4]
   static constexpr int64_t total = rdmF + 4LL * MT * kFragPair;
-  // float tables: invM2[B2], fP[3][B2][B2] as at most O non-zeros per row
-  // (every fP_h row has at most O), unscale factors of the stationary
-  // matrices [ck0, ck1, ck2, vol0, vol1, vol2, fmrt, rdm, rdmF] (1 unless
-  // the fragments were scaled by a power of two)
-  static constexpr int tInvM2 = 0;
-  static constexpr int tFP = B2;                  // fP_h rows as O (value) entries: [3][B2][O]
+  // float tables: fP[3][B2][B2] as at most O non-zeros per row (every fP_h row has at most O)
+  static constexpr int tFP = 0;                   // fP_h rows as O (value) entries: [3][B2][O]
   static constexpr int tFPCol = tFP + 3 * B2 * O; // their columns (exact small integers): [3][B2][O]
-  static constexpr int tAUn = tFPCol + 3 * B2 * O;
-  static constexpr int tTotal = tAUn + 9;
+  static constexpr int tTotal = tFPCol + 3 * B2 * O;
 };
 
 // local-time-stepping outputs of the local pass (TimeCluster.cpp:380-434):
@@ -81,8 +76,20 @@ inline bool vectorAccess(const CellLayout& lay, const void* dofs, const void* in
   return true;
 }
 
-// the order at which the neighbour pass runs on split products (f16x3 and
-// bf16x3; every other one runs the FP32 pass of mx_neighbor.h)
+// Which engines run on split products: the two-plane form, whose three bf16
+// products per contraction beat the FP32 pass of mx_local.h where the row
+// tiles are full.  Every other matrix-core form runs the FP32 passes, which
+// are at least as accurate: their 4-row k-steps skip the matrices' zeros
+// (32-row steps are mostly padding at low orders), they need no column scales
+// (f16x3) and half the products of three planes (bf16x6).  Whole step, random
+// links, split -> FP32 local pass: f16x3 ORDER 6 1M cells 7.93 -> 7.42 ms, 10k
+// 119 -> 106 us, 1k 59.3 -> 58.8; ORDER 7 120k 1965 -> 1917; f16x3 60k ORDER 3
+// 171 -> 121, ORDER 4 280 -> 189, ORDER 5 448 -> 326; bf16x6 ORDER 6 60k 784 ->
+// 529, ORDER 7 120k 2225 -> 1914; bf16x3 60k ORDER 5 403 -> 326, but ORDER 6
+// 200k 1335 -> 1392 and ORDER 7 120k 1677 -> 1914.
+inline bool splitProducts(const EngineState& e) { return e.arithmetic == SDG_BF16X3 && e.order >= 6; }
+// Their neighbour pass: at ORDER 7 the FP32 pass from the traces is faster (60k
+// cells 921 -> 862 us a step), at ORDER 6 it is not (459 -> 478).
 constexpr int kSplitNeighborOrder = 6;
 
 // host entry points of one order's kernels

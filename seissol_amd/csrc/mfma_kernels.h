@@ -1,19 +1,12 @@
-// Kernel templates of the element update on the matrix cores (included by
-// the per-order sources kernels_mfma_o<O>.hip): FP32 data, split 16-bit products,
-// FP32 accumulation (arithmetics SDG_BF16X3, SDG_BF16X6 and SDG_F16X3).
+// Kernel templates of the element update on the matrix cores in split bf16
+// products (SDG_BF16X3 at orders 6 and 7; included by the per-order sources
+// kernels_mfma_o<O>.hip): FP32 data, FP32 accumulation.
 //
 // Every contraction with a global matrix A (kDivMT, kDivM, fMrT, rDivM) is a
 // GEMM  Y(M x 144) += A(M x K) X(K x 144)  over a tile of 16 elements, the 144
 // columns being (quantity p, element e) -> 16 p + e.  Both operands are split
-// into planes of a 16-bit type (x = x0 + x1 [+ x2], each plane the rounding of
-// the remainder) and the plane products run as v_mfma_f32_16x16x32_{bf16,f16}:
-//   V = 2  (bf16, 2 planes): A0X0 + A0X1 + A1X0                      ~2^-17
-//   V = 3  (bf16, 3 planes): + A0X2 + A2X0 + A1X1                     ~2^-24
-//   V = 16 (fp16, 2 planes): A0X0 + A0X1 + A1X0                      ~2^-21
-// The fp16 form scales every X column (and every stationary matrix) by a
-// power of two that brings its largest magnitude into [2^13, 2^14), so the
-// 5-bit exponent of fp16 never limits; the scales are exact and are divided
-// out of the FP32 results.
+// into two bf16 planes (x = x0 + x1, each plane the rounding of the remainder)
+// and A0X0 + A0X1 + A1X0 runs as v_mfma_f32_16x16x32_bf16, about 2^-17.
 //
 // One wave owns one 16-row tile of the basis index for all 9 quantities of the
 // 16 elements, so a lane holds rows 4g..4g+3 (g = lane / 16) of element
@@ -27,7 +20,8 @@
 //  kLocalMfma:    CK derivatives + time integral, volume, local flux of the
 //                 four faces; writes Q and the face traces rT_f I.
 //  kNeighborMfma: neighbour flux rDivM_f ((fP_h Tr) AminusT_f) from the traces
-//                 the neighbours wrote; updates Q.
+//                 the neighbours wrote; updates Q (ORDER 6; at ORDER 7 the FP32
+//                 pass of mx_neighbor.h is the faster one).
 // Operator sequence: codegen/kernels/aderdg.py:321-537 (the neighbour's rT_j I
 // is produced by the neighbour itself, rT_j = diag(1/M2) fMrT_j).
 #pragma once
@@ -47,39 +41,9 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-template <int V>
-struct Prec;
-template <>
-struct Prec<2> {
-  using T = __bf16;
-  using V8 = bf16x8;
-  using V4 = bf16x4;
-  static constexpr int NX = 2;
-  static constexpr bool scaled = false;
-};
-template <>
-struct Prec<3> {
-  using T = __bf16;
-  using V8 = bf16x8;
-  using V4 = bf16x4;
-  static constexpr int NX = 3;
-  static constexpr bool scaled = false;
-};
-template <>
-struct Prec<16> {
-  using T = _Float16;
-  using V8 = halfx8;
-  using V4 = halfx4;
-  static constexpr int NX = 2;
-  static constexpr bool scaled = true;
-};
-
-// largest |x| of a scaled column: [2^13, 2^14)
-constexpr int kScaleExp = 13;
+constexpr int NX = 2;  // planes
 
 __device__ constexpr int kStarQ[9][3] = {{6, 7, 8}, {6, 7, 8}, {6, 7, 8}, {6, 7, -1}, {7, 8, -1},
                                          {6, 8, -1}, {0, 3, 5}, {1, 3, 4}, {2, 4, 5}};
@@ -96,205 +60,103 @@ struct CoeffsF {
 };
 
 
-// geometry of the two kernels per order and variant
-template <int O, int V>
+// geometry of the two kernels per order
+template <int O>
 struct Cfg {
   using S = MShape<O>;
-  static constexpr int NX = Prec<V>::NX;
-  static constexpr bool scaled = Prec<V>::scaled;
   static constexpr int LDX_L = S::KMAX + 8;  // local kernel: padded column stride
-  static constexpr int LDS_L = NX * kCols * LDX_L * 2 + kTileElems * 72 * 4 + 9 * 16 * kTileElems * 4 +
-                               (scaled ? S::MT * kCols * 4 : 0);
-  static constexpr int WAVES_L = (V != 3 && LDS_L <= 81920) ? 2 : 1;
+  static constexpr int LDS_L = NX * kCols * LDX_L * 2 + kTileElems * 72 * 4 + 9 * 16 * kTileElems * 4;
+  static constexpr int WAVES_L = LDS_L <= 81920 ? 2 : 1;
   // neighbour kernel: one face's operand at a time (32 rows, 8 of padding in the stride)
   static constexpr int LDX_N = 40;
   static constexpr int LDS_N = NX * kCols * LDX_N * 2 + kTileElems * 9 * S::B2P * 4 + kTileElems * 81 * 4 +
-                               3 * S::B2 * O * 8 + (scaled ? kCols * 4 : 0) + 2 * kTileElems * 4 * 4;
+                               3 * S::B2 * O * 8 + 2 * kTileElems * 4 * 4;
   static constexpr int WGS_N = 163840 / LDS_N;  // workgroups per CU that the LDS allows
   // minimum waves per SIMD asked of the register allocator: three when the LDS
   // lets three or more waves per SIMD run
-  static constexpr int WAVES_N = V == 3 ? 1 : (WGS_N * S::MT >= 12 ? 3 : 2);
+  static constexpr int WAVES_N = WGS_N * S::MT >= 12 ? 3 : 2;
 };
 
 __device__ inline floatx4 mma(bf16x8 a, bf16x8 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ inline floatx4 mma(halfx8 a, halfx8 b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
 
 // split product, smallest terms first
-template <int V>
-__device__ inline floatx4 mfmaSplit(const typename Prec<V>::V8 (&a)[Prec<V>::NX],
-                                    const typename Prec<V>::V8 (&b)[Prec<V>::NX], floatx4 c) {
-  if constexpr (V == 3) {
-    c = mma(a[1], b[1], c);
-    c = mma(a[2], b[0], c);
-    c = mma(a[0], b[2], c);
-  }
+__device__ inline floatx4 mfmaSplit(const bf16x8 (&a)[NX], const bf16x8 (&b)[NX], floatx4 c) {
   c = mma(a[1], b[0], c);
   c = mma(a[0], b[1], c);
   c = mma(a[0], b[0], c);
   return c;
 }
 
-template <int V>
-__device__ inline void split(float x, typename Prec<V>::T (&parts)[Prec<V>::NX]) {
-  using T = typename Prec<V>::T;
+__device__ inline void split(float x, __bf16 (&parts)[NX]) {
   float rest = x;
 #pragma unroll
-  for (int i = 0; i < Prec<V>::NX; ++i) {
-    parts[i] = static_cast<T>(rest);
+  for (int i = 0; i < NX; ++i) {
+    parts[i] = static_cast<__bf16>(rest);
     rest -= static_cast<float>(parts[i]);
   }
 }
 
 // X planes: NX consecutive arrays of kCols * LDX 16-bit values
-template <int V, int LDX>
-__device__ inline void storeX4(typename Prec<V>::T* xs, int col, int k0, const float (&v)[4], float scale) {
-  using P = Prec<V>;
-  typename P::V4 out[P::NX];
+template <int LDX>
+__device__ inline void storeX4(__bf16* xs, int col, int k0, const float (&v)[4]) {
+  bf16x4 out[NX];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    typename P::T parts[P::NX];
-    split<V>(v[j] * scale, parts);
+    __bf16 parts[NX];
+    split(v[j], parts);
 #pragma unroll
-    for (int i = 0; i < P::NX; ++i) out[i][j] = parts[i];
+    for (int i = 0; i < NX; ++i) out[i][j] = parts[i];
   }
 #pragma unroll
-  for (int i = 0; i < P::NX; ++i)
-    *reinterpret_cast<typename P::V4*>(xs + i * kCols * LDX + col * LDX + k0) = out[i];
-}
-
-template <int V, int LDX>
-__device__ inline void storeX1(typename Prec<V>::T* xs, int col, int k, float v) {
-  typename Prec<V>::T parts[Prec<V>::NX];
-  split<V>(v, parts);
-#pragma unroll
-  for (int i = 0; i < Prec<V>::NX; ++i) xs[i * kCols * LDX + col * LDX + k] = parts[i];
+  for (int i = 0; i < NX; ++i) *reinterpret_cast<bf16x4*>(xs + i * kCols * LDX + col * LDX + k0) = out[i];
 }
 
 // two consecutive rows k0, k0 + 1 (k0 even) of one column: one 32-bit store per plane
-template <int V, int LDX>
-__device__ inline void storeX2(typename Prec<V>::T* xs, int col, int k0, float v0, float v1) {
-  using P = Prec<V>;
-  typedef typename P::T T2 __attribute__((ext_vector_type(2)));
-  typename P::T a[P::NX], b[P::NX];
-  split<V>(v0, a);
-  split<V>(v1, b);
+template <int LDX>
+__device__ inline void storeX2(__bf16* xs, int col, int k0, float v0, float v1) {
+  typedef __bf16 T2 __attribute__((ext_vector_type(2)));
+  __bf16 a[NX], b[NX];
+  split(v0, a);
+  split(v1, b);
 #pragma unroll
-  for (int i = 0; i < P::NX; ++i) *reinterpret_cast<T2*>(xs + i * kCols * LDX + col * LDX + k0) = T2{a[i], b[i]};
+  for (int i = 0; i < NX; ++i) *reinterpret_cast<T2*>(xs + i * kCols * LDX + col * LDX + k0) = T2{a[i], b[i]};
 }
 
-template <int V, int LDX>
-__device__ inline void storeZero4(typename Prec<V>::T* xs, int col, int k0) {
-  using P = Prec<V>;
-  typename P::V4 z;
+template <int LDX>
+__device__ inline void storeZero4(__bf16* xs, int col, int k0) {
+  bf16x4 z;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) z[j] = static_cast<typename P::T>(0.0f);
+  for (int j = 0; j < 4; ++j) z[j] = static_cast<__bf16>(0.0f);
 #pragma unroll
-  for (int i = 0; i < P::NX; ++i) *reinterpret_cast<typename P::V4*>(xs + i * kCols * LDX + col * LDX + k0) = z;
+  for (int i = 0; i < NX; ++i) *reinterpret_cast<bf16x4*>(xs + i * kCols * LDX + col * LDX + k0) = z;
 }
 
-// power-of-two scale of a column with largest magnitude cm, and its inverse,
-// built from the exponent bits (exponent clamped to [-100, 127])
-__device__ inline void columnScale(float cm, float& scale, float& unscale) {
-  const int biased = static_cast<int>((__float_as_uint(cm) >> 23) & 0xffu);
-  if (cm > 0.0f && biased != 0xff) {
-    const int k = max(biased - 127, -100);
-    scale = __uint_as_float(static_cast<unsigned>(127 + kScaleExp - k) << 23);
-    unscale = __uint_as_float(static_cast<unsigned>(127 - kScaleExp + k) << 23);
-  } else {
-    scale = 1.0f;
-    unscale = 1.0f;
-  }
-}
-
-// Lane reductions in registers (no LDS round trip); every lane of the wave
-// must be active.
-// max over the wave's four 16-lane rows (lanes e, e + 16, e + 32, e + 48):
-// gfx950's row swaps exchange rows 0-1 with 2-3, then rows 0 with 1 and 2 with 3
-__device__ inline float rowsMax4(float m) {
-  const unsigned u = __float_as_uint(m);
-  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const unsigned u2 = __float_as_uint(m);
-  const auto b = __builtin_amdgcn_permlane16_swap(u2, u2, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-// max over each 16-lane row through DPP: partners lane ^ 1 and lane ^ 2
-// (quad_perm), then the mirrored lane within 8 and within 16 lanes
-template <int CTRL>
-__device__ inline float dppMove(float m) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(m), __float_as_int(m), CTRL, 0xF, 0xF, false));
-}
-__device__ inline float rowMax16(float m) {
-  m = fmaxf(m, dppMove<0xB1>(m));   // quad_perm [1, 0, 3, 2]
-  m = fmaxf(m, dppMove<0x4E>(m));   // quad_perm [2, 3, 0, 1]
-  m = fmaxf(m, dppMove<0x141>(m));  // row_half_mirror
-  return fmaxf(m, dppMove<0x140>(m));  // row_mirror
-}
-
-// largest magnitude of each quantity column over the rows this wave holds
-// (lanes of one element differ in lane / 16), written to sMax[w][16 q + e]
-template <int R>
-__device__ inline void waveColumnMax(const float (&v)[R][9][4], bool has, float* sMax, int w, int lane) {
-  const int g = lane >> 4, e = lane & 15;
-  float m[9];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    m[q] = 0.0f;
-    if (has)
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) m[q] = fmaxf(m[q], fabsf(v[r][q][j]));
-    m[q] = rowsMax4(m[q]);
-  }
-  if (g == 0)
-#pragma unroll
-    for (int q = 0; q < 9; ++q) sMax[w * kCols + q * 16 + e] = m[q];
-}
-
-// column scales of this lane's element from the maxima of the WAVES waves
-template <int WAVES>
-__device__ inline void columnScales(const float* sMax, int e, float (&scale)[9], float (&unscale)[9]) {
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    float cm = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) cm = fmaxf(cm, sMax[w * kCols + q * 16 + e]);
-    columnScale(cm, scale[q], unscale[q]);
-  }
-}
-
-template <int V>
-__device__ inline typename Prec<V>::V8 loadFrag(const uint16_t* __restrict__ base, int lane) {
-  return *reinterpret_cast<const typename Prec<V>::V8*>(base + lane * 8);
+__device__ inline bf16x8 loadFrag(const uint16_t* __restrict__ base, int lane) {
+  return *reinterpret_cast<const bf16x8*>(base + lane * 8);
 }
 
 // acc[jj][i] += A_jj(tile) X(:, quantity Q0 + i)  for JJ matrices with
 // fragment bases a[jj] and NQ consecutive quantities
-template <int V, int JJ, int Q0, int NQ, int LDX>
+template <int JJ, int Q0, int NQ, int LDX>
 __device__ inline void gemmTile(floatx4 (&acc)[JJ][NQ], const uint16_t* const (&a)[JJ], int ksteps,
-                                const typename Prec<V>::T* xs, int lane) {
-  using P = Prec<V>;
-  constexpr int NX = P::NX;
+                                const __bf16* xs, int lane) {
   const int g = lane >> 4, e = lane & 15;
   for (int kk = 0; kk < ksteps; ++kk) {
-    typename P::V8 af[JJ][NX];
+    bf16x8 af[JJ][NX];
 #pragma unroll
     for (int jj = 0; jj < JJ; ++jj)
 #pragma unroll
-      for (int i = 0; i < NX; ++i) af[jj][i] = loadFrag<V>(a[jj] + kk * kFragPair + i * kFragPlane, lane);
+      for (int i = 0; i < NX; ++i) af[jj][i] = loadFrag(a[jj] + kk * kFragPair + i * kFragPlane, lane);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int off = ((Q0 + q) * 16 + e) * LDX + kk * 32 + 8 * g;
-      typename P::V8 bf[NX];
+      bf16x8 bf[NX];
 #pragma unroll
-      for (int i = 0; i < NX; ++i) bf[i] = *reinterpret_cast<const typename P::V8*>(xs + i * kCols * LDX + off);
+      for (int i = 0; i < NX; ++i) bf[i] = *reinterpret_cast<const bf16x8*>(xs + i * kCols * LDX + off);
 #pragma unroll
-      for (int jj = 0; jj < JJ; ++jj) acc[jj][q] = mfmaSplit<V>(af[jj], bf, acc[jj][q]);
+      for (int jj = 0; jj < JJ; ++jj) acc[jj][q] = mfmaSplit(af[jj], bf, acc[jj][q]);
     }
   }
 }
@@ -336,22 +198,20 @@ __device__ inline void loadRows(const float* q, const float* qSafe, int ld, int 
   }
 }
 
-// q[p * ld + j] += (add ? add[p][j] : 0) + acc[p][j] * s * un[p] for the
-// lane's rows below B (16-byte accesses when V4 and the four rows are all real)
+// q[p * ld + j] += acc[p][j] for the lane's rows below B (16-byte accesses
+// when V4 and the four rows are all real)
 template <int B, bool V4>
-__device__ inline void updateRows(float* q, int ld, int row0, const floatx4 (&acc)[9], float s, const float (&un)[9],
-                                  const float (*add)[4]) {
+__device__ inline void updateRows(float* q, int ld, int row0, const floatx4 (&acc)[9]) {
   if (V4 && (B % 4 == 0 || row0 + 3 < B)) {
     if (row0 < B)
 #pragma unroll
       for (int p = 0; p < 9; ++p) {
         float4* d = reinterpret_cast<float4*>(q + p * ld);
         float4 x = *d;
-        const float sc = s * un[p];
-        x.x += (add ? add[p][0] : 0.0f) + acc[p][0] * sc;
-        x.y += (add ? add[p][1] : 0.0f) + acc[p][1] * sc;
-        x.z += (add ? add[p][2] : 0.0f) + acc[p][2] * sc;
-        x.w += (add ? add[p][3] : 0.0f) + acc[p][3] * sc;
+        x.x += acc[p][0];
+        x.y += acc[p][1];
+        x.z += acc[p][2];
+        x.w += acc[p][3];
         *d = x;
       }
   } else {
@@ -359,23 +219,18 @@ __device__ inline void updateRows(float* q, int ld, int row0, const floatx4 (&ac
     for (int p = 0; p < 9; ++p)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (row0 + j < B) q[p * ld + j] += (add ? add[p][j] : 0.0f) + acc[p][j] * (s * un[p]);
+        if (row0 + j < B) q[p * ld + j] += acc[p][j];
   }
 }
 
-// Y += sum_j (A_j X) star_j for the lane's element, with the matrix and
-// column scales divided out (the star values in LDS carry the CK matrices'
-// scales; kFactor: times aUn[j] as well).  The products run in three passes over input
+// Y += sum_j (A_j X) star_j for the lane's element.  The products run in three passes over input
 // quantity groups {6,7,8}, {0,1,2}, {3,4,5}, each holding 3 x 3 accumulator
 // tiles (the elastic star matrix maps velocities (6..8) to stresses (0..5)
 // and stresses to velocities); the three matrices' fragments of a k-step are
 // loaded inside the pass (L2-resident), which keeps them out of the live set.
-template <int V, int KSMAX, int LDX, bool kFactor>
-__device__ inline void gemmStars(const uint16_t* const (&a)[3], int ks, const typename Prec<V>::T* xs, int lane,
-                                 const float* sS, const float (&aUn)[3], const float (&colUn)[9], float (&y)[9][4],
-                                 int passMask = 7) {
-  using P = Prec<V>;
-  constexpr int NX = P::NX;
+template <int KSMAX, int LDX>
+__device__ inline void gemmStars(const uint16_t* const (&a)[3], int ks, const __bf16* xs, int lane,
+                                 const float* sS, float (&y)[9][4], int passMask = 7) {
   const int g = lane >> 4, e = lane & 15;
 #pragma unroll
   for (int pass = 0; pass < 3; ++pass) {
@@ -389,19 +244,19 @@ __device__ inline void gemmStars(const uint16_t* const (&a)[3], int ks, const ty
 #pragma unroll
     for (int kk = 0; kk < KSMAX; ++kk)
       if (kk < ks) {
-        typename P::V8 af[1][3][NX];
+        bf16x8 af[1][3][NX];
 #pragma unroll
         for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
-          for (int i = 0; i < NX; ++i) af[0][jj][i] = loadFrag<V>(a[jj] + kk * kFragPair + i * kFragPlane, lane);
+          for (int i = 0; i < NX; ++i) af[0][jj][i] = loadFrag(a[jj] + kk * kFragPair + i * kFragPlane, lane);
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
           const int off = ((q0 + i) * 16 + e) * LDX + kk * 32 + 8 * g;
-          typename P::V8 bf[NX];
+          bf16x8 bf[NX];
 #pragma unroll
-          for (int pl = 0; pl < NX; ++pl) bf[pl] = *reinterpret_cast<const typename P::V8*>(xs + pl * kCols * LDX + off);
+          for (int pl = 0; pl < NX; ++pl) bf[pl] = *reinterpret_cast<const bf16x8*>(xs + pl * kCols * LDX + off);
 #pragma unroll
-          for (int jj = 0; jj < 3; ++jj) acc[jj][i] = mfmaSplit<V>(af[0][jj], bf, acc[jj][i]);
+          for (int jj = 0; jj < 3; ++jj) acc[jj][i] = mfmaSplit(af[0][jj], bf, acc[jj][i]);
         }
       }
     // contraction with the star matrices for the outputs this group feeds
@@ -414,8 +269,7 @@ __device__ inline void gemmStars(const uint16_t* const (&a)[3], int ks, const ty
           if (k < kStarCnt[p]) {
             const int qi = kStarQ[p][k];
             if (qi >= q0 && qi < q0 + 3) {
-              const float sv = kFactor ? sS[jj * 24 + kStarOff[p] + k] * aUn[jj] * colUn[qi]
-                                       : sS[jj * 24 + kStarOff[p] + k] * colUn[qi];
+              const float sv = sS[jj * 24 + kStarOff[p] + k];
 #pragma unroll
               for (int j = 0; j < 4; ++j) y[p][j] += acc[jj][qi - q0][j] * sv;
             }
@@ -425,22 +279,19 @@ __device__ inline void gemmStars(const uint16_t* const (&a)[3], int ks, const ty
 
 // DEF: the arrays have the default layout (DOF blocks [9][B], operators 243 /
 // 72, 324 reals apart), so every stride is a compile-time constant
-template <int O, int V, bool V4, bool LTS, bool DEF>
-__global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLocalMfma(
-    int64_t n, const uint16_t* __restrict__ frag, const float* __restrict__ tables, CoeffsF<O> cf,
+template <int O, bool V4, bool LTS, bool DEF>
+__global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O>::WAVES_L)) void kLocalMfma(
+    int64_t n, const uint16_t* __restrict__ frag, CoeffsF<O> cf,
     float* __restrict__ dofs, float* __restrict__ integ, float* __restrict__ traces,
     const float* __restrict__ star, const float* __restrict__ aplus, const uint8_t* __restrict__ faceTypes,
     CellLayout lay, LtsOut lts) {
   using S = MShape<O>;
-  using C = Cfg<O, V>;
-  using T = typename Prec<V>::T;
-  constexpr int B = S::B, B2 = S::B2, MT = S::MT, LDX = C::LDX_L, FR = S::FR, NX = C::NX;
-  constexpr bool scaled = C::scaled;
+  using C = Cfg<O>;
+  constexpr int B = S::B, B2 = S::B2, MT = S::MT, LDX = C::LDX_L, FR = S::FR;
   constexpr int TPW = cdiv(S::MTF, MT);
-  __shared__ __attribute__((aligned(16))) T xs[NX * kCols * LDX];
+  __shared__ __attribute__((aligned(16))) __bf16 xs[NX * kCols * LDX];
   __shared__ float sStar[kTileElems * 72];
   __shared__ float sStage[3 * 3 * 16 * kTileElems];  // CK partial sums handed between waves (3 slots)
-  __shared__ float sMax[scaled ? MT * kCols : 1];
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));  // wave-uniform
@@ -455,12 +306,6 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
   float* const tileDofs = dofs + E0 * qStride;
   const int laneQ = e * static_cast<int>(qStride) + 16 * w + 4 * g;
   float* const tileTraces = traces + E0 * 36 * S::B2P;
-  const float* aUn = tables + S::tAUn;
-  const float aUnCk[3] = {aUn[0], aUn[1], aUn[2]};
-  // the volume products' factor relative to the staged star values (powers
-  // of two; 1 when kDivM's fragments carry the scales of kDivMT's)
-  const float aUnVol[3] = {aUn[3] / aUn[0], aUn[4] / aUn[1], aUn[5] / aUn[2]};
-  const float aUnF = aUn[6], aUnR = aUn[7];
 
   {
     // the tile's compact star matrices, every load of a thread issued before
@@ -485,14 +330,10 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
         sv[u] = star[el * starStride + 81 * (r / 24) + kStarPos[r % 24]];
       }
     }
-    // staged times the CK matrices' unscale factor of their direction (a
-    // power of two: exact), which the CK products then need not apply
 #pragma unroll
     for (int u = 0; u < SI; ++u) {
       const int i = threadIdx.x + u * S::THREADS;
-      const int jd = (i % 72) / 24;
-      const float f = jd == 0 ? aUnCk[0] : (jd == 1 ? aUnCk[1] : aUnCk[2]);
-      if (i < kTileElems * 72) sStar[i] = E0 + i / 72 < n ? sv[u] * f : 0.0f;
+      if (i < kTileElems * 72) sStar[i] = E0 + i / 72 < n ? sv[u] : 0.0f;
     }
   }
 
@@ -526,18 +367,10 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
 #pragma unroll
     for (int j = 0; j < 4; ++j) iacc[0][p][j] = cf.c[0] * q[0][p][j];
   // X <- Q
-  float cs[9], un[9];
 #pragma unroll
-  for (int p = 0; p < 9; ++p) cs[p] = un[p] = 1.0f;
-  if constexpr (scaled) {
-    waveColumnMax<1>(q, true, sMax, w, lane);
-    __syncthreads();
-    columnScales<MT>(sMax, e, cs, un);
-  }
-#pragma unroll
-  for (int p = 0; p < 9; ++p) storeX4<V, LDX>(xs, p * 16 + e, 16 * w + 4 * g, q[0][p], cs[p]);
+  for (int p = 0; p < 9; ++p) storeX4<LDX>(xs, p * 16 + e, 16 * w + 4 * g, q[0][p]);
   for (int t = MT + w; t < S::KPB / 16; t += MT)
-    for (int p = 0; p < 9; ++p) storeZero4<V, LDX>(xs, p * 16 + e, 16 * t + 4 * g);
+    for (int p = 0; p < 9; ++p) storeZero4<LDX>(xs, p * 16 + e, 16 * t + 4 * g);
   __syncthreads();
   const float* sS = sStar + e * 72;
 
@@ -577,7 +410,7 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
       const uint16_t* a[3] = {frag + S::ck + (0LL * MT + tile) * S::KSB * kFragPair,
                               frag + S::ck + (1LL * MT + tile) * S::KSB * kFragPair,
                               frag + S::ck + (2LL * MT + tile) * S::KSB * kFragPair};
-      gemmStars<V, S::KSB, LDX, false>(a, ks, xs, lane, sS, aUnCk, un, dq[0], mask);
+      gemmStars<S::KSB, LDX>(a, ks, xs, lane, sS, dq[0], mask);
     }
     if (mode != 0) {
       if (slot >= 0)
@@ -613,20 +446,18 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
             if (16 * w + 4 * g + j < m) cellDeriv[doff + p * ldm + 16 * w + 4 * g + j] = dq[0][p][j];
       doff += 9LL * ldm;
     }
-    if constexpr (scaled) waveColumnMax<1>(dq, w < mtiles, sMax, w, lane);
     __syncthreads();
-    if constexpr (scaled) columnScales<MT>(sMax, e, cs, un);
     if (w < mtiles) {
 #pragma unroll
       for (int p = 0; p < 9; ++p) {
-        storeX4<V, LDX>(xs, p * 16 + e, 16 * w + 4 * g, dq[0][p], cs[p]);
+        storeX4<LDX>(xs, p * 16 + e, 16 * w + 4 * g, dq[0][p]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) iacc[0][p][j] += cf.c[d] * dq[0][p][j];
       }
     }
     for (int t = w; t < kpNext / 16; t += MT)
       if (t >= mtiles)
-        for (int p = 0; p < 9; ++p) storeZero4<V, LDX>(xs, p * 16 + e, 16 * t + 4 * g);
+        for (int p = 0; p < 9; ++p) storeZero4<LDX>(xs, p * 16 + e, 16 * t + 4 * g);
     __syncthreads();
   }
 
@@ -657,15 +488,10 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
       for (int j = 0; j < 4; ++j)
         if (row0 + j < B) elemInteg[p * ldq + row0 + j] = old[p][j] + iacc[0][p][j];
   }
-  if constexpr (scaled) {
-    waveColumnMax<1>(iacc, true, sMax, w, lane);
-    __syncthreads();
-    columnScales<MT>(sMax, e, cs, un);
-  }
 #pragma unroll
-  for (int p = 0; p < 9; ++p) storeX4<V, LDX>(xs, p * 16 + e, 16 * w + 4 * g, iacc[0][p], cs[p]);
+  for (int p = 0; p < 9; ++p) storeX4<LDX>(xs, p * 16 + e, 16 * w + 4 * g, iacc[0][p]);
   for (int t = MT + w; t < S::KPB / 16; t += MT)
-    for (int p = 0; p < 9; ++p) storeZero4<V, LDX>(xs, p * 16 + e, 16 * t + 4 * g);
+    for (int p = 0; p < 9; ++p) storeZero4<LDX>(xs, p * 16 + e, 16 * t + 4 * g);
   __syncthreads();
 
   // face traces rT_f I = (fMrT_f / M2) I (rows f * B2P + m): the fragments
@@ -683,11 +509,11 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
 #pragma unroll
       for (int p = 0; p < 9; ++p) acc[0][p] = floatx4{0, 0, 0, 0};
       const uint16_t* a[1] = {frag + S::fmrt + static_cast<int64_t>(t) * S::KSB * kFragPair};
-      if (E0 < n) gemmTile<V, 1, 0, 9, LDX>(acc, a, S::KSB, xs, lane);
+      if (E0 < n) gemmTile<1, 0, 9, LDX>(acc, a, S::KSB, xs, lane);
 #pragma unroll
       for (int p = 0; p < 9; ++p)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) tr[ti][p][j] = acc[0][p][j] * (aUnF * un[p]);
+        for (int j = 0; j < 4; ++j) tr[ti][p][j] = acc[0][p][j];
       // the traces: the lane's four rows lie in one
       // face (faces padded to B2P rows, a multiple of 4), one 16-byte store
       // per quantity into the padded layout [element][face][quantity][B2P]
@@ -715,7 +541,7 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
     // `E0 < n` holds for every launched tile; the guard gives this GEMM (and
     // the trace GEMM above) a block of its own, with which the register
     // allocator keeps the kernel free of spills
-    if (E0 < n) gemmStars<V, S::KSB, LDX, true>(a, S::KSB, xs, lane, sS, aUnVol, un, vol);
+    if (E0 < n) gemmStars<S::KSB, LDX>(a, S::KSB, xs, lane, sS, vol);
   }
 
   // Once every wave has finished the volume GEMM, the X area is free until W
@@ -780,57 +606,49 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_L)) void kLoc
         vol[p][j] = 16 * w + 4 * g + j < B ? sVol[(e * 9 + p) * B + 16 * w + 4 * g + j] : 0.0f;
   }
 
-  if constexpr (scaled) waveColumnMax<TPW>(tr, true, sMax, w, lane);
   __syncthreads();
-  if constexpr (scaled) columnScales<MT>(sMax, e, cs, un);
 #pragma unroll
   for (int ti = 0; ti < TPW; ++ti) {
     const int t = w + ti * MT;
     if (t < S::MTF)
 #pragma unroll
-      for (int p = 0; p < 9; ++p) storeX4<V, LDX>(xs, p * 16 + e, 16 * t + 4 * g, tr[ti][p], cs[p]);
+      for (int p = 0; p < 9; ++p) storeX4<LDX>(xs, p * 16 + e, 16 * t + 4 * g, tr[ti][p]);
   }
   for (int t = S::MTF + w; t < S::KPF / 16; t += MT)
-    for (int p = 0; p < 9; ++p) storeZero4<V, LDX>(xs, p * 16 + e, 16 * t + 4 * g);
+    for (int p = 0; p < 9; ++p) storeZero4<LDX>(xs, p * 16 + e, 16 * t + 4 * g);
   __syncthreads();
 
   // local flux: Q += [rDivM_0 .. rDivM_3] W, the accumulators starting from the
-  // volume term divided by the (power-of-two) unscale factors, so that the
-  // update needs no separately live volume registers
+  // volume term
   {
     floatx4 acc[1][9];
 #pragma unroll
-    for (int p = 0; p < 9; ++p) {
-      const float inv = 1.0f / (aUnR * un[p]);
+    for (int p = 0; p < 9; ++p)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[0][p][j] = vol[p][j] * inv;
-    }
+      for (int j = 0; j < 4; ++j) acc[0][p][j] = vol[p][j];
     const uint16_t* a[1] = {frag + S::rdm + static_cast<int64_t>(w) * S::KSF * kFragPair};
-    gemmTile<V, 1, 0, 9, LDX>(acc, a, S::KSF, xs, lane);
-    if (valid) updateRows<B, V4>(tileDofs + laneQ, ldq, 16 * w + 4 * g, acc[0], aUnR, un, nullptr);
+    gemmTile<1, 0, 9, LDX>(acc, a, S::KSF, xs, lane);
+    if (valid) updateRows<B, V4>(tileDofs + laneQ, ldq, 16 * w + 4 * g, acc[0]);
   }
 }
 
-template <int O, int V, bool V4, bool DEF>
-__global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_N)) void kNeighborMfma(
+template <int O, bool V4, bool DEF>
+__global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O>::WAVES_N)) void kNeighborMfma(
     int64_t n, const uint16_t* __restrict__ frag, const float* __restrict__ tables, float* __restrict__ dofs,
     const float* __restrict__ traces, const int32_t* __restrict__ neighbors, const uint8_t* __restrict__ faceRel,
     const float* __restrict__ aminus, const uint8_t* __restrict__ faceTypes, CellLayout lay) {
   using S = MShape<O>;
-  using C = Cfg<O, V>;
-  using T = typename Prec<V>::T;
-  constexpr int B = S::B, B2 = S::B2, B2P = S::B2P, LDX = C::LDX_N, NX = C::NX;
-  constexpr bool scaled = C::scaled;
+  using C = Cfg<O>;
+  constexpr int B = S::B, B2 = S::B2, B2P = S::B2P, LDX = C::LDX_N;
   constexpr int HALF = B2P / 2;                  // row pairs of one (padded) face
   static_assert(HALF <= 16 && B2P <= 32 && LDX >= 32, "a face's row pairs fit a 16-lane group, its rows a k-step");
   constexpr int GROUPS = S::THREADS / 16;        // 16-lane groups per pass, one element each
   constexpr int PASSES = cdiv(kTileElems, GROUPS);
-  __shared__ __attribute__((aligned(16))) T xs[NX * kCols * LDX];  // face operand: rows [0, B2P) of one face, the rest zero
+  __shared__ __attribute__((aligned(16))) __bf16 xs[NX * kCols * LDX];  // face operand: rows [0, B2P) of one face, the rest zero
   __shared__ __attribute__((aligned(16))) float sTr[kTileElems * 9 * B2P];
   __shared__ float sAm[kTileElems * 81];
   __shared__ float sFP[3 * B2 * O];   // fP_h rows: O (value, column) entries each
   __shared__ int sFPCol[3 * B2 * O];
-  __shared__ float sUn[scaled ? kCols : 1];  // unscale factor of each operand column of the current face
   __shared__ int sLink[kTileElems * 4];  // trace index nb * 4 + side of (element, face), -1: none
   __shared__ int sRel[kTileElems * 4];   // orientation h of (element, face)
   constexpr int TR = 9 * B2P;                                  // floats of one (padded) face trace
@@ -886,7 +704,7 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_N)) void kNei
     for (int i = threadIdx.x; i < kCols * (32 - B2P); i += blockDim.x) {
       const int col = i / (32 - B2P), k = B2P + i % (32 - B2P);
 #pragma unroll
-      for (int pl = 0; pl < NX; ++pl) xs[pl * kCols * LDX + col * LDX + k] = static_cast<T>(0.0f);
+      for (int pl = 0; pl < NX; ++pl) xs[pl * kCols * LDX + col * LDX + k] = static_cast<__bf16>(0.0f);
     }
   }
   __syncthreads();
@@ -916,8 +734,7 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_N)) void kNei
   floatx4 tot[1][9];
 #pragma unroll
   for (int p = 0; p < 9; ++p) tot[0][p] = floatx4{0, 0, 0, 0};
-  // face by face: W_f = (fP_h Tr_f) AminusT_f into the operand (the fp16 form
-  // scales each column by a power of two), then Q += rDivM_f W_f as one k-step
+  // face by face: W_f = (fP_h Tr_f) AminusT_f into the operand, then Q += rDivM_f W_f as one k-step
 #pragma unroll 1
   for (int f = 0; f < 4; ++f) {
     // the previous face's items have read sTr / sAm (barrier before its product)
@@ -932,7 +749,7 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_N)) void kNei
       if (idx < kTileElems * 81) sAm[idx] = av[i];
     }
     if (f < 3) gather(f + 1);
-    __syncthreads();  // also: every wave's product of the previous face has read xs and sUn
+    __syncthreads();  // also: every wave's product of the previous face has read xs
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
       // rows 2 rp and 2 rp + 1 of face f of element s (rows >= B2 are padding: zero)
@@ -982,44 +799,15 @@ __global__ __launch_bounds__(MShape<O>::THREADS, (Cfg<O, V>::WAVES_N)) void kNei
         w0[p] = regular ? w0[p] : 0.0f;
         w1[p] = regular ? w1[p] : 0.0f;
       }
-      if constexpr (scaled) {
-        // column maxima over the 16 lanes of the element (idle lanes hold zeros)
 #pragma unroll
-        for (int p = 0; p < 9; ++p) {
-          const float m = rowMax16(fmaxf(fabsf(w0[p]), fabsf(w1[p])));
-          float sc, inv;
-          columnScale(m, sc, inv);
-          if (act) storeX2<V, LDX>(xs, p * 16 + s, r0, w0[p] * sc, w1[p] * sc);
-          if (s < kTileElems && rp == 0) sUn[p * 16 + s] = inv;
-        }
-      } else {
-#pragma unroll
-        for (int p = 0; p < 9; ++p)
-          if (act) storeX2<V, LDX>(xs, p * 16 + s, r0, w0[p], w1[p]);
-      }
+      for (int p = 0; p < 9; ++p)
+        if (act) storeX2<LDX>(xs, p * 16 + s, r0, w0[p], w1[p]);
     }
     __syncthreads();
     const uint16_t* a[1] = {frag + S::rdmF + (static_cast<int64_t>(w) * 4 + f) * kFragPair};
-    if constexpr (scaled) {
-      floatx4 acc[1][9];
-#pragma unroll
-      for (int p = 0; p < 9; ++p) acc[0][p] = floatx4{0, 0, 0, 0};
-      gemmTile<V, 1, 0, 9, LDX>(acc, a, 1, xs, lane);
-#pragma unroll
-      for (int p = 0; p < 9; ++p) {
-        const float un = sUn[p * 16 + e];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) tot[0][p][j] += acc[0][p][j] * un;
-      }
-    } else {
-      gemmTile<V, 1, 0, 9, LDX>(tot, a, 1, xs, lane);
-    }
+    gemmTile<1, 0, 9, LDX>(tot, a, 1, xs, lane);
   }
-  float one[9];
-#pragma unroll
-  for (int p = 0; p < 9; ++p) one[p] = 1.0f;
-  const float aUnR = tables[S::tAUn + 8];
-  if (valid) updateRows<B, V4>(tileDofs + laneQ, ldq, 16 * w + 4 * g, tot[0], aUnR, one, nullptr);
+  if (valid) updateRows<B, V4>(tileDofs + laneQ, ldq, 16 * w + 4 * g, tot[0]);
 }
 
 // the arrays have the default layout: DOF blocks [9][B] back to back, the
@@ -1048,7 +836,7 @@ void launchVariants(bool v4, bool def, F&& launch) {
 // lts == nullptr: the proxy/GTS local pass (traces written, derivatives never);
 // otherwise the LTS local pass: buffers and derivatives per the cells' setup,
 // traces written only when the layer has them
-template <int O, int V>
+template <int O>
 int localImpl(const EngineState& st, const double* coeffs, const sdg_layer* L, bool writeIntegrated,
               hipStream_t stream, const LtsOut* lts = nullptr) {
   using S = MShape<O>;
@@ -1064,13 +852,13 @@ int localImpl(const EngineState& st, const double* coeffs, const sdg_layer* L, b
   auto launch = [&](auto vec, auto def) {
     constexpr bool kV4 = decltype(vec)::value, kDef = decltype(def)::value;
     if (lts != nullptr)
-      kLocalMfma<O, V, kV4, true, kDef><<<grid, S::THREADS, 0, stream>>>(
-          n, static_cast<const uint16_t*>(st.mfmaFrags), static_cast<const float*>(st.mfmaTables), cf,
+      kLocalMfma<O, kV4, true, kDef><<<grid, S::THREADS, 0, stream>>>(
+          n, static_cast<const uint16_t*>(st.mfmaFrags), cf,
           static_cast<float*>(L->dofs), integ, static_cast<float*>(L->face_traces),
           static_cast<const float*>(L->star), static_cast<const float*>(L->aplus), L->face_types, lay, *lts);
     else
-      kLocalMfma<O, V, kV4, false, kDef><<<grid, S::THREADS, 0, stream>>>(
-          n, static_cast<const uint16_t*>(st.mfmaFrags), static_cast<const float*>(st.mfmaTables), cf,
+      kLocalMfma<O, kV4, false, kDef><<<grid, S::THREADS, 0, stream>>>(
+          n, static_cast<const uint16_t*>(st.mfmaFrags), cf,
           static_cast<float*>(L->dofs), integ, static_cast<float*>(L->face_traces),
           static_cast<const float*>(L->star), static_cast<const float*>(L->aplus), L->face_types, lay, LtsOut{});
   };
@@ -1079,7 +867,7 @@ int localImpl(const EngineState& st, const double* coeffs, const sdg_layer* L, b
   return SDG_OK;
 }
 
-template <int O, int V>
+template <int O>
 int neighborImpl(const EngineState& st, const sdg_layer* L, hipStream_t stream) {
   using S = MShape<O>;
   const int64_t n = L->num_elements;
@@ -1089,7 +877,7 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, hipStream_t stream) 
   if (!vectorAccess(lay, L->dofs, nullptr, "matrix-core neighbour pass", v4)) return SDG_ERR_INVALID;
   const dim3 grid(static_cast<unsigned>((n + kTileElems - 1) / kTileElems));
   auto launch = [&](auto vec, auto def) {
-    kNeighborMfma<O, V, decltype(vec)::value, decltype(def)::value><<<grid, S::THREADS, 0, stream>>>(
+    kNeighborMfma<O, decltype(vec)::value, decltype(def)::value><<<grid, S::THREADS, 0, stream>>>(
         n, static_cast<const uint16_t*>(st.mfmaFrags), static_cast<const float*>(st.mfmaTables),
         static_cast<float*>(L->dofs), static_cast<const float*>(L->face_traces), L->face_neighbors,
         L->face_relations, static_cast<const float*>(L->aminus), L->face_types, lay);
@@ -1099,35 +887,19 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, hipStream_t stream) 
   return SDG_OK;
 }
 
-template <int O>
-int localDispatch(const EngineState& e, const double* coeffs, const sdg_layer* layer, bool writeIntegrated,
-                  hipStream_t stream, const LtsOut* lts) {
-  switch (e.arithmetic) {
-    case SDG_BF16X6: return localImpl<O, 3>(e, coeffs, layer, writeIntegrated, stream, lts);
-    case SDG_F16X3: return localImpl<O, 16>(e, coeffs, layer, writeIntegrated, stream, lts);
-    default: return localImpl<O, 2>(e, coeffs, layer, writeIntegrated, stream, lts);
-  }
-}
-
-template <int O>
-int neighborDispatch(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  if constexpr (O == kSplitNeighborOrder)
-    return e.arithmetic == SDG_F16X3 ? neighborImpl<O, 16>(e, layer, stream) : neighborImpl<O, 2>(e, layer, stream);
-  setError("the split-product neighbour pass is built for one order");
-  return SDG_ERR_UNSUPPORTED;
-}
-
 }  // namespace
 
 // the host entry of one order (explicitly instantiated by its own source)
 template <int O>
 int MfmaOrder<O>::local(const EngineState& e, const double* coeffs, const sdg_layer* layer, bool writeIntegrated,
                         hipStream_t stream, const LtsOut* lts) {
-  return localDispatch<O>(e, coeffs, layer, writeIntegrated, stream, lts);
+  return localImpl<O>(e, coeffs, layer, writeIntegrated, stream, lts);
 }
 template <int O>
 int MfmaOrder<O>::neighbor(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  return neighborDispatch<O>(e, layer, stream);
+  if constexpr (O == kSplitNeighborOrder) return neighborImpl<O>(e, layer, stream);
+  setError("the split-product neighbour pass is built for one order");
+  return SDG_ERR_UNSUPPORTED;
 }
 
 }  // namespace mfma

@@ -85,48 +85,26 @@ float bf16Value(uint16_t h) {
   return f;
 }
 
-uint16_t f16Bits(float f) {
-  const _Float16 h = static_cast<_Float16>(f);  // round to nearest even
-  uint16_t b;
-  std::memcpy(&b, &h, 2);
-  return b;
-}
-float f16Value(uint16_t b) {
-  _Float16 h;
-  std::memcpy(&h, &b, 2);
-  return static_cast<float>(h);
-}
-
-// Split a row-major FP64 matrix (times `scale`) into three planes of bf16 or
-// fp16 (x = hi + mid + lo, each plane the round-to-nearest of the remainder)
-// laid out in the lane order of v_mfma_f32_16x16x32_{bf16,f16}'s A operand:
-// lane l of fragment (mt, ks) holds A[16 mt + l % 16][32 ks + 8 (l / 16) + i], i < 8.
+// Split a row-major FP64 matrix into two planes of bf16 (x = hi + lo, each
+// plane the round-to-nearest of the remainder) laid out in the lane order of
+// v_mfma_f32_16x16x32_bf16's A operand: lane l of fragment (mt, ks) holds
+// A[16 mt + l % 16][32 ks + 8 (l / 16) + i], i < 8.
 void appendFragments(const std::function<double(int, int)>& A, int rows, int cols, int mtiles, int ksteps,
-                     uint16_t* out, bool f16, double scale) {
+                     uint16_t* out) {
   for (int mt = 0; mt < mtiles; ++mt)
     for (int ks = 0; ks < ksteps; ++ks) {
       uint16_t* base = out + (static_cast<int64_t>(mt) * ksteps + ks) * mfma::kFragPair;
       for (int l = 0; l < 64; ++l)
         for (int i = 0; i < 8; ++i) {
           const int r = 16 * mt + l % 16, c = 32 * ks + 8 * (l / 16) + i;
-          double rest = (r < rows && c < cols) ? A(r, c) * scale : 0.0;
-          for (int plane = 0; plane < 3; ++plane) {
-            const uint16_t h = f16 ? f16Bits(static_cast<float>(rest)) : bf16Bits(static_cast<float>(rest));
+          double rest = (r < rows && c < cols) ? A(r, c) : 0.0;
+          for (int plane = 0; plane < 2; ++plane) {
+            const uint16_t h = bf16Bits(static_cast<float>(rest));
             base[plane * mfma::kFragPlane + l * 8 + i] = h;
-            rest -= static_cast<double>(f16 ? f16Value(h) : bf16Value(h));
+            rest -= static_cast<double>(bf16Value(h));
           }
         }
     }
-}
-
-// power of two that brings the largest |entry| into [2^13, 2^14) (fp16 form), else 1
-double fragmentScale(const std::function<double(int, int)>& A, int rows, int cols, bool f16) {
-  if (!f16) return 1.0;
-  double mx = 0.0;
-  for (int r = 0; r < rows; ++r)
-    for (int c = 0; c < cols; ++c) mx = std::max(mx, std::fabs(A(r, c)));
-  if (mx == 0.0) return 1.0;
-  return std::ldexp(1.0, 13 - std::ilogb(mx));
 }
 
 template <int O>
@@ -134,20 +112,15 @@ int uploadMfmaData(EngineState& s, const double* gm) {
   using S = mfma::MShape<O>;
   const auto g = globalMatrixLayout(O);
   const int B = S::B, B2 = S::B2;
-  const bool f16 = s.arithmetic == SDG_F16X3;
   std::vector<uint16_t> frags(S::total, 0);
   std::vector<float> tables(S::tTotal);
   auto add = [&](const std::function<double(int, int)>& A, int rows, int cols, int mtiles, int ksteps,
-                 int64_t offset, int unscaleSlot) {
-    const double sc = fragmentScale(A, rows, cols, f16);
-    appendFragments(A, rows, cols, mtiles, ksteps, frags.data() + offset, f16, sc);
-    tables[S::tAUn + unscaleSlot] = static_cast<float>(1.0 / sc);
-  };
+                 int64_t offset) { appendFragments(A, rows, cols, mtiles, ksteps, frags.data() + offset); };
   for (int j = 0; j < 3; ++j) {
     add([&](int r, int c) { return -gm[g.kDivMT + (j * B + r) * B + c]; }, B, B, S::MT, S::KSB,
-        S::ck + static_cast<int64_t>(j) * S::MT * S::KSB * mfma::kFragPair, j);
+        S::ck + static_cast<int64_t>(j) * S::MT * S::KSB * mfma::kFragPair);
     add([&](int r, int c) { return gm[g.kDivM + (j * B + r) * B + c]; }, B, B, S::MT, S::KSB,
-        S::vol + static_cast<int64_t>(j) * S::MT * S::KSB * mfma::kFragPair, 3 + j);
+        S::vol + static_cast<int64_t>(j) * S::MT * S::KSB * mfma::kFragPair);
   }
   // the four face operands stacked with B2P rows each (rows B2..B2P-1 zero).
   // The local pass forms the traces rT_f I = (fMrT_f / M2) I directly, so its
@@ -158,17 +131,16 @@ int uploadMfmaData(EngineState& s, const double* gm) {
         const int m = r % B2P;
         return m < B2 ? gm[g.fMrT + ((r / B2P) * B2 + m) * B + c] / gm[g.mass2 + m] : 0.0;
       },
-      S::FR, B, S::MTF, S::KSB, S::fmrt, 6);
+      S::FR, B, S::MTF, S::KSB, S::fmrt);
   add([&](int r, int c) {
         const int m = c % B2P;
         return m < B2 ? gm[g.rDivM + ((c / B2P) * B + r) * B2 + m] * gm[g.mass2 + m] : 0.0;
       },
-      B, S::FR, S::MT, S::KSF, S::rdm, 7);
+      B, S::FR, S::MT, S::KSF, S::rdm);
   // rDivM_f per face (k-step f: face f's B2 columns), for the neighbour kernel's face-by-face product
   static_assert(B2P <= 32, "one face's rows fit one k-step");
   add([&](int r, int c) { return c % 32 < B2 ? gm[g.rDivM + ((c / 32) * B + r) * B2 + c % 32] : 0.0; }, B, 128,
-      S::MT, 4, S::rdmF, 8);
-  for (int m = 0; m < B2; ++m) tables[S::tInvM2 + m] = static_cast<float>(1.0 / gm[g.mass2 + m]);
+      S::MT, 4, S::rdmF);
   // fP_h rows as (value, column) lists of O entries, padded with zeros
   for (int h = 0; h < 3; ++h) {
     double mx = 0.0;
@@ -196,16 +168,12 @@ int uploadMfmaData(EngineState& s, const double* gm) {
 }
 
 int uploadMfma(EngineState& s, const double* gm) {
-  switch (s.order) {
-    case 3: return uploadMfmaData<3>(s, gm);
-    case 4: return uploadMfmaData<4>(s, gm);
-    case 5: return uploadMfmaData<5>(s, gm);
-    case 6: return uploadMfmaData<6>(s, gm);
-    case 7: return uploadMfmaData<7>(s, gm);
-    default:
-      setError("matrix-core arithmetic supports orders 3..7");
-      return SDG_ERR_UNSUPPORTED;
+  if (s.order < 3 || s.order > 7) {
+    setError("matrix-core arithmetic supports orders 3..7");
+    return SDG_ERR_UNSUPPORTED;
   }
+  if (!mfma::splitProducts(s)) return SDG_OK;
+  return s.order == 6 ? uploadMfmaData<6>(s, gm) : uploadMfmaData<7>(s, gm);
 }
 
 }  // namespace
