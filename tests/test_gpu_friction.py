@@ -78,6 +78,27 @@ def test_friction_matches_oracle(gpu, order, faces, padded, closed_form):
     np.testing.assert_array_equal(drv.fault.host("slip_rate_updates")[..., :np_], ref["slip_rate_updates"][..., :np_])
 
 
+# one face, a ragged last block, and the two lane groups (up to 32 points, up to 64)
+@pytest.mark.parametrize("order,faces", [(3, 1), (3, 5), (4, 2), (6, 1), (6, 3), (7, 2)])
+@pytest.mark.parametrize("closed_form", [False, True])
+def test_friction_blocks_match_oracle(gpu, order, faces, closed_form):
+    import torch
+    steps, dt = 4, 1e-3
+    setup = make_fault_setup(num_faces=faces, order=order, seed=7, points=None, length=4000.0, nucleation_radius=900.0)
+    print(f"friction order={order} faces={faces} points={setup.points} closed_form_start={closed_form}", flush=True)
+    solver = FrictionSolver(setup.params, order)
+    solver.closed_form_start = closed_form
+    drv = FaultDriver(setup, solver, dt)
+    drv.advance(steps)
+    torch.cuda.synchronize()
+    ref = _run_oracle(setup, steps, dt, closed_form_start=closed_form)
+    np_ = setup.num_points
+    for name in COMPARED:  # the bound of test_friction_matches_oracle
+        assert _rel(drv.fault.host(name)[..., :np_], ref[name][..., :np_]) < 1e-9, name
+    for name in ("convergence_inner", "convergence_outer"):
+        np.testing.assert_array_equal(drv.fault.host(name)[..., :np_], ref[name][..., :np_])
+
+
 def test_mlp_loss_and_gradient_match_oracle(gpu):
     import torch
     rng = np.random.default_rng(1)
