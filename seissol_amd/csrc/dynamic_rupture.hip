@@ -77,8 +77,11 @@ int ensureDrMatrices(EngineState& s) {
 }
 
 constexpr int kDrWaves = 4;   // sides in flight per interpolation workgroup (one per wave)
-constexpr int kDrScan = 1;    // faces of the chunk per thread
-constexpr int kDrChunk = 64 * kDrWaves * kDrScan;  // faces scanned by one interpolation workgroup
+constexpr int kDrChunk = 64 * kDrWaves;  // most faces scanned by one interpolation workgroup
+// Workgroups of a chunk: a plus variant has a quarter of the chunk's plus
+// sides, a minus variant a twelfth of its minus sides, so that three
+// workgroups share a plus variant's.
+constexpr int kDrPlusParts = 3, kDrGroups = 4 * kDrPlusParts + 12;
 
 // position of entry i of the packed derivatives (blocks [9][B(O-d)] one
 // after another) in the layout's derivatives (blocks [9][rows(B(O-d))])
@@ -107,10 +110,15 @@ __host__ __device__ constexpr int columnOffset(int d) {
 
 // Space-time interpolation, batched by the 16 variants of V3mTo2n(i, h)
 // (h = 0: plus side, h = 1..3: minus side with that orientation), as the
-// reference batches per (side, faceRelation): workgroup (chunk, variant)
-// stages its matrix in LDS once and serves every side of its variant among
-// the chunk's kDrChunk faces, listed in face order and dealt round-robin to
-// its waves (one side per wave at a time).  Per side the derivatives are
+// reference batches per (side, faceRelation): workgroup (chunk, group)
+// stages its variant's matrix in LDS once and serves the sides of the variant
+// among the chunk's faces, listed in face order and dealt round-robin to its
+// waves (one side per wave at a time; three workgroups share a plus variant's
+// list, which is three times as long).  Bound by the serial work of a side at
+// one or two waves per SIMD, then by the FP64 output: with one workgroup per
+// variant and 256 faces per chunk the plus lists of 16 sides per wave ran long
+// after the others (10k faces, FP64 ORDER 6: 267 -> 183 us, 3.3 TB/s; 3k faces,
+// FP32 ORDER 5: 105 -> 36).  Per side the derivatives are
 // rotated to the face frame first, dQ'_d[p][l] = sum_q dQ_d[q][l] TinvT(q, p)
 // (the rotation commutes with the interpolation; columns (d, l) spread over
 // the lanes), then interpolated, w_d[k][p] = sum_l V[k][l] dQ'_d[p][l] (lane
@@ -122,7 +130,7 @@ __host__ __device__ constexpr int columnOffset(int d) {
 // gather of a wave's next side is issued before the arithmetic of its
 // current one, so that the loads are in flight while it computes.
 template <typename real, int O>
-__global__ __launch_bounds__(64 * kDrWaves, 2) void kDrInterpolate(int64_t nf, const real* __restrict__ V,
+__global__ __launch_bounds__(64 * kDrWaves, 2) void kDrInterpolate(int64_t nf, int chunk, const real* __restrict__ V,
                                                                 const real* __restrict__ deriv, CellLayout lay,
                                                                 sdg_dr_layer L, StepCoeffs<O> cf,
                                                                 double* __restrict__ outPlus,
@@ -143,65 +151,56 @@ __global__ __launch_bounds__(64 * kDrWaves, 2) void kDrInterpolate(int64_t nf, c
   __shared__ real sT[kDrWaves][96];
   __shared__ int sFace[kDrChunk];  // the chunk's sides of this variant: chunk-local face index
   __shared__ int sElem[kDrChunk];  // and the side's element
-  __shared__ int sCount[kDrScan][kDrWaves];
-  const int variant = blockIdx.y, vi = variant >> 2, vh = variant & 3;
+  __shared__ int sCount[kDrWaves];
+  const int group = blockIdx.y;
+  const bool isPlus = group < 4 * kDrPlusParts;
+  const int vi = (isPlus ? group : group - 4 * kDrPlusParts) / 3, third = group % 3;
+  const int vh = isPlus ? 0 : 1 + third;
+  // this workgroup's sides: first, first + step, ... of the variant's list, per wave
+  const int part = isPlus ? third : 0, step = kDrWaves * (isPlus ? kDrPlusParts : 1);
   const int side = vh == 0 ? 0 : 1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const real* Vv = V + static_cast<int64_t>(vi * 4 + vh) * NP * B;
-  const int64_t f0 = static_cast<int64_t>(blockIdx.x) * kDrChunk;
+  const int64_t f0 = static_cast<int64_t>(blockIdx.x) * chunk;
   // the start-up loads (the variant's matrix, the chunk's face data), all
   // issued before the first is used
   real vv[VI];
 #pragma unroll
   for (int u = 0; u < VI; ++u) vv[u] = Vv[min(static_cast<int>(threadIdx.x) + NT * u, NP * B - 1)];
-  bool match[kDrScan];
-  int elem[kDrScan];
-#pragma unroll
-  for (int s = 0; s < kDrScan; ++s) {
-    const int64_t f = min(f0 + threadIdx.x + NT * s, nf - 1);  // nf >= 1 here
+  bool match;
+  int elem;
+  {
+    const int64_t f = min(f0 + threadIdx.x, nf - 1);  // nf >= 1 here
     const int faceSide = min(static_cast<int>(L.face_info[f * 3 + side]), 3);
     // faceRelation = orientation + 1 lies in [1, 3]; clamped so that a malformed
     // entry still names a minus-side variant (0 would match no workgroup)
     const int h = side == 0 ? 0 : min(max(static_cast<int>(L.face_info[f * 3 + 2]), 1), 3);
-    const int el = side == 0 ? L.plus_element[f] : L.minus_element[f];
-    match[s] = f0 + threadIdx.x + NT * s < nf && faceSide == vi && h == vh;
-    elem[s] = el;
+    elem = side == 0 ? L.plus_element[f] : L.minus_element[f];
+    match = static_cast<int>(threadIdx.x) < chunk && f0 + threadIdx.x < nf && faceSide == vi && h == vh;
   }
-  unsigned long long mask[kDrScan];
-#pragma unroll
-  for (int s = 0; s < kDrScan; ++s) {
-    mask[s] = __ballot(match[s]);
-    if (lane == 0) sCount[s][wave] = __popcll(mask[s]);
-  }
+  const unsigned long long mask = __ballot(match);
+  if (lane == 0) sCount[wave] = __popcll(mask);
 #pragma unroll
   for (int u = 0; u < VI; ++u) {
     const int i = threadIdx.x + NT * u;
     if (u + 1 < VI || i < NP * B) sV[(i / B) * LDV + i % B] = vv[u];
   }
   __syncthreads();
-  // the chunk's sides of this variant in face order: scan s, then wave
-  int total = 0;
+  // the chunk's sides of this variant in face order
+  int total = 0, base = 0;
 #pragma unroll
-  for (int s = 0; s < kDrScan; ++s)
-#pragma unroll
-    for (int w = 0; w < kDrWaves; ++w) total += sCount[s][w];
+  for (int w = 0; w < kDrWaves; ++w) {
+    base += w < wave ? sCount[w] : 0;
+    total += sCount[w];
+  }
   total = __builtin_amdgcn_readfirstlane(total);
-#pragma unroll
-  for (int s = 0; s < kDrScan; ++s) {
-    int base = 0;
-#pragma unroll
-    for (int s1 = 0; s1 < kDrScan; ++s1)
-#pragma unroll
-      for (int w = 0; w < kDrWaves; ++w)
-        base += (s1 < s || (s1 == s && w < wave)) ? sCount[s1][w] : 0;
-    if (match[s]) {
-      const int at = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                                static_cast<unsigned>(mask[s] >> 32),
-                                __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask[s]), 0u)));
-      sFace[at] = threadIdx.x + NT * s;
-      sElem[at] = elem[s];
-    }
+  if (match) {
+    const int at = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                              static_cast<unsigned>(mask >> 32),
+                              __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u)));
+    sFace[at] = threadIdx.x;
+    sElem[at] = elem;
   }
   __syncthreads();
   const int P = L.points;
@@ -227,8 +226,9 @@ __global__ __launch_bounds__(64 * kDrWaves, 2) void kDrInterpolate(int64_t nf, c
 #pragma unroll
     for (int c = 0; c < 2; ++c) preT[c] = L.tinv_t[f * 81 + min(ln + 64 * c, 80)];
   };
-  if (wave < total) fetch(wave);
-  for (int j = wave; j < total; j += kDrWaves) {
+  const int first = wave + kDrWaves * part;
+  if (first < total) fetch(first);
+  for (int j = first; j < total; j += step) {
     const int64_t f = f0 + __builtin_amdgcn_readfirstlane(sFace[j]);
     waveSync();  // the previous side's reads of sD/sT are done
 #pragma unroll
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(64 * kDrWaves, 2) void kDrInterpolate(int64_t nf, c
       if (i < 81) sT[wave][i] = static_cast<real>(preT[c]);
     }
     waveSync();
-    if (j + kDrWaves < total) fetch(j + kDrWaves);
+    if (j + step < total) fetch(j + step);
     const int c16 = lane & 15;
     // rotation to the face frame first (it commutes with the interpolation):
     // dQ_d[p][l] <- sum_q dQ_d[q][l] TinvT(q, p) in place, one column (d, l)
@@ -454,10 +454,17 @@ int interpolateImpl(EngineState& st, const double* coeffs, const void* deriv, co
   StepCoeffs<O> cf{};
   for (int o = 0; o < O; ++o)
     for (int d = 0; d < O; ++d) cf.c[o][d] = coeffs[o * O + d];
-  const dim3 grid(static_cast<unsigned>((L->num_faces + kDrChunk - 1) / kDrChunk), 16);
-  kDrInterpolate<real, O><<<grid, 64 * kDrWaves, 0, stream>>>(L->num_faces, static_cast<const real*>(st.drMatrices),
-                                                              static_cast<const real*>(deriv), engineLayout(st), *L,
-                                                              cf, qp, qm);
+  // Faces per chunk: as many as leave four workgroups per CU (fewer mean longer
+  // lists per wave, more stage the matrix again).  Both passes around the
+  // solve, with chunks of 256 -> 128 -> 64 -> 32 faces: FP64 ORDER 6 10k faces
+  // 322, 320, 328, 340 us; 1k 84, 64, 59, 60; FP32 ORDER 5 3k 81, 71, 58, 58;
+  // 300 faces 50, 36, 27, 22.
+  int chunk = kDrChunk;
+  while (chunk > 32 && (L->num_faces + chunk - 1) / chunk * kDrGroups < 4 * 256) chunk /= 2;
+  const dim3 grid(static_cast<unsigned>((L->num_faces + chunk - 1) / chunk), kDrGroups);
+  kDrInterpolate<real, O><<<grid, 64 * kDrWaves, 0, stream>>>(
+      L->num_faces, chunk, static_cast<const real*>(st.drMatrices), static_cast<const real*>(deriv), engineLayout(st),
+      *L, cf, qp, qm);
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;
 }

@@ -6,7 +6,7 @@ import pytest
 import oracle
 from helpers import PolyField, project, rel_l2
 from seissol_amd import _capi
-from seissol_amd.dr import DeviceDrFaces, collocation_coefficients, face_matrices, plane_faces
+from seissol_amd.dr import DeviceDrFaces, DrFaces, collocation_coefficients, face_matrices, plane_faces
 from seissol_amd.kernels import Engine, Local, Neighbor, Spacetime, global_matrices, monomial_integrate
 from seissol_amd.proxy import DeviceLayer, make_setup
 
@@ -58,6 +58,36 @@ def test_space_time_interpolation_matches_oracle(gpu, order, arith, tol, extra):
     ep, em = rel_l2(gp, rp), rel_l2(gm_, rm)
     print(f"rel L2 vs oracle: plus {ep:.2e} minus {em:.2e}")
     assert ep < tol and em < tol
+
+
+# every chunk length (32 to 256 faces, by the number of faces) against calls of
+# a few faces each: a face's arithmetic does not depend on its chunk
+@pytest.mark.parametrize("order,arith,nf", [(3, "fp64", 33), (3, "fp64", 2750), (4, "fp32", 5500), (3, "fp32", 11001)])
+def test_interpolation_of_many_faces_equals_that_of_few(gpu, order, arith, nf):
+    import torch
+    print(f"dr interpolate order={order} {arith} faces={nf}", flush=True)
+    eng, cells, points = Engine(order, arith), 500, (order + 1) ** 2
+    rng = np.random.default_rng(nf)
+    deriv = torch.from_numpy(rng.uniform(-1, 1, (cells, eng.layout_sizes()[2]))).cuda()
+    deriv = deriv if arith == "fp64" else deriv.float()
+    info = np.stack([rng.integers(0, 4, nf), rng.integers(0, 4, nf), rng.integers(1, 4, nf)], 1).astype(np.uint8)
+    plus, minus = (rng.integers(0, cells, nf).astype(np.int32) for _ in range(2))
+    tinv = rng.uniform(-1, 1, (nf, 81))
+    c = collocation_coefficients(order, 1e-3)
+
+    def run(a, b):
+        flux = np.zeros((b - a, 81))
+        dr = DeviceDrFaces(DrFaces(plus[a:b], minus[a:b], info[a:b], np.full((cells, 4), -1, np.int32), tinv[a:b], flux,
+                                   flux, np.zeros((b - a, 11)), points))
+        q = [torch.full((b - a, order, 9, points), np.nan, dtype=torch.float64, device="cuda") for _ in range(2)]
+        dr.interpolate(eng, c, deriv, *q)
+        torch.cuda.synchronize()
+        return q
+
+    whole = run(0, nf)
+    few = [run(a, min(a + 500, nf)) for a in range(0, nf, 500)]
+    for side in range(2):
+        assert torch.equal(whole[side], torch.cat([f[side] for f in few]))
 
 
 @pytest.mark.parametrize("order,arith,tol", [(2, "fp64", 1e-12), (3, "fp64", 1e-12), (6, "fp64", 1e-12),
