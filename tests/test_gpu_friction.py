@@ -120,6 +120,24 @@ def test_mlp_loss_and_gradient_match_oracle(gpu):
     assert np.all(tr.grads.cpu().numpy()[:14] == 0.0)  # normalisation constants are not trained
 
 
+# one sample, ragged groups of 32, more groups than blocks (256)
+@pytest.mark.parametrize("n", [1, 31, 33, 8193])
+def test_mlp_gradient_of_ragged_batches(gpu, n):
+    import torch
+    samples = np.random.default_rng(n).normal(size=(n, 7)).astype(np.float32)
+    tr = WarmStartTrainer(seed=4)
+    tr.params[0:6], tr.params[6:12], tr.params[12], tr.params[13] = 0.0, 1.0, 0.0, 1.0
+    tr.grads.fill_(np.nan)  # the call clears what it adds to
+    tr.loss.fill_(np.nan)
+    tr.loss_grad(torch.from_numpy(samples).cuda())
+    torch.cuda.synchronize()
+    p = tr.params.cpu().double().numpy()
+    loss, g = oracle.mlp_loss_grad(samples[:, :6].astype(np.float64), samples[:, 6].astype(np.float64), p[14:])
+    assert abs(tr.loss.item() - loss) <= 1e-5 * loss
+    assert _rel(tr.grads.cpu().double().numpy()[14:], g) < 1e-4
+    assert np.all(tr.grads.cpu().numpy()[:14] == 0.0)
+
+
 def test_mlp_training_reduces_loss(gpu):
     import torch
     rng = np.random.default_rng(2)
