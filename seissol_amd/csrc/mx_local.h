@@ -102,12 +102,15 @@ struct Ahead {
   static constexpr int stress = sizeof(real) == 8 ? 4 : 8, velocity = 2, trace = sizeof(real) == 8 ? 2 : 4;
 };
 
-// the star values of one direction that feed the stresses: FP32 has the
-// registers to read them ahead of the direction's products, FP64 reads them
-// two quantities ahead of their use
-template <typename real>
+// registers to spare: FP32, and FP64 at low orders
+template <int O, typename real>
+constexpr bool kRoomy = sizeof(real) == 4 || O <= 4;
+
+// the star values of one direction that feed the stresses, read ahead of the
+// direction's products (ROOMY) or two quantities ahead of their use
+template <typename real, bool ROOMY>
 struct StressStar {
-  static constexpr int AHEAD = sizeof(real) == 8 ? 2 : 6;
+  static constexpr int AHEAD = ROOMY ? 6 : 2;
   real v[6][3];
   const real* at;
   __device__ inline void read(int p) {
@@ -157,14 +160,14 @@ __device__ inline void loadStress(const Run<real>& run, int lane, real (&cur)[Ah
 // one stream over the directions and on into the next run: `cur` holds this
 // run's first k-steps on entry and the next run's on return, so that their
 // latency passes behind the products and the barrier between the runs.
-template <int KS, int LD, typename real>
+template <int KS, int LD, bool ROOMY, typename real>
 __device__ inline void starStress(const Run<real>& run, const Run<real>& next, const real* x, const real* sS, int lane,
                                   typename Vec<real>::V4 (&y)[6], real (&cur)[Ahead<real>::stress]) {
   using V4 = typename Vec<real>::V4;
   constexpr int U = Ahead<real>::stress;
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
-    StressStar<real> star(sS, j);
+    StressStar<real, ROOMY> star(sS, j);
     V4 acc[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) acc[i] = V4{0, 0, 0, 0};
@@ -299,12 +302,12 @@ __device__ inline void starVelocity(const Run<real> (&run)[TW], const Run<real> 
 // products are too short to hide a fragment's way from L2, so the leading
 // 10 x 20 block of the three matrices is kept in LDS, [direction][k-step][g][row].
 // KL: k-steps; a: the lane's entry of the block
-template <int KL, int LD, typename real>
+template <int KL, int LD, bool ROOMY, typename real>
 __device__ inline void lateStress(const real* a, const real* x, const real* sS, typename Vec<real>::V4 (&y)[6]) {
   using V4 = typename Vec<real>::V4;
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
-    StressStar<real> star(sS, j);
+    StressStar<real, ROOMY> star(sS, j);
     V4 acc[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) acc[i] = V4{0, 0, 0, 0};
@@ -370,12 +373,12 @@ __device__ inline void gemm(typename Vec<real>::V4 (&acc)[NQ], const Run<real>& 
 
 // W = T A for the four rows of a lane's quad, two rows at a time (more
 // outgrow the registers); A is read at lds[at + 9 p + q], one column at a
-// time (else all 81 entries are loaded at once), in FP32 ahead of its use
-template <typename real>
+// time (else all 81 entries are loaded at once), ahead of its use (ROOMY)
+template <typename real, bool ROOMY>
 __device__ inline void mixRows(typename Vec<real>::V4 (&t)[9], const real* lds, int at, bool zero) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    constexpr int N = sizeof(real) == 8 ? 1 : 2;  // columns in flight
+    constexpr int N = ROOMY ? 2 : 1;  // columns in flight
     real w0[9], w1[9], a[N][9];
     auto column = [&](int p, real(&c)[9]) {
       int col = at + 9 * p;
@@ -536,9 +539,9 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
       for (int t = 0; t < TW; ++t)
         if (runs[t].lo < runs[t].hi) {
           if (TW == 2 && t == 0)
-            starStress<KS, LD, real>(runs[0], runs[1].lo < runs[1].hi ? runs[1] : next[0], x, sS, lane, y[0], aheadS);
+            starStress<KS, LD, kRoomy<O, real>, real>(runs[0], runs[1].lo < runs[1].hi ? runs[1] : next[0], x, sS, lane, y[0], aheadS);
           else
-            starStress<KS, LD, real>(runs[t], next[0], x, sS, lane, y[t], aheadS);
+            starStress<KS, LD, kRoomy<O, real>, real>(runs[t], next[0], x, sS, lane, y[t], aheadS);
         }
     }
   };
@@ -632,7 +635,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
 #pragma unroll
           for (int p = 0; p < NP; ++p) y[p] = V4{0, 0, 0, 0};
           if constexpr (VEL) lateVelocity<KL, LD, real>(late, xr + source(d), sS, y);
-          else lateStress<KL, LD, real>(late, xr + source(d), sS, y);
+          else lateStress<KL, LD, kRoomy<O, real>, real>(late, xr + source(d), sS, y);
         }
         if constexpr (d == 1) __syncthreads();  // dQ_1 takes the place of Q
         if (w < 2) finish(d, m, 0, y);
@@ -692,6 +695,18 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
     real aheadT[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) aheadT[u] = trace[0].fr[min(trace[0].lo + u, trace[0].hi - 1) * 64 + lane];
+    // one value of each 128-byte line of the tile's AplusT, to have it in L2
+    // when it is staged (1M cells in FP32 at ORDER 6: 5.00 -> 4.93 ms, 400k in
+    // FP64: 4.58 -> 4.46; at the lower FP32 orders, which have more workgroups
+    // in flight, it cost 1 %)
+    constexpr int LINES = RS == 8 || O >= 6 ? cdiv(324 * RS, 128) : 0, NT = cdiv(kElems * LINES, THREADS);
+    const Buffer<real> aplus(A.aplus + E0 * lay.aplusStride, (cells - 1) * lay.aplusStride + 324);
+    real touch[NT > 0 ? NT : 1];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int i = threadIdx.x + u * THREADS, el = i / maxOf(LINES, 1);
+      touch[u] = aplus.load1(el < cells ? el * static_cast<int>(lay.aplusStride) * RS + i % maxOf(LINES, 1) * 128 : kNowhere, 0);
+    }
     product(runs, runs, xr, acc);
     // face traces rT_f I
     V4 tr[TT][9];
@@ -716,7 +731,8 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
     {
       typedef real VP __attribute__((ext_vector_type(16 / RS)));
       constexpr int W = 16 / RS, PIECES = 324 / W, N = cdiv(kElems * PIECES, THREADS), N1 = N / 2;
-      const Buffer<real> aplus(A.aplus + E0 * lay.aplusStride, (cells - 1) * lay.aplusStride + 324);
+#pragma unroll
+      for (int u = 0; u < NT; ++u) asm volatile("" ::"v"(touch[u]));
       const int stride = static_cast<int>(lay.aplusStride);
       auto load = [&](int u) {
         const int i = threadIdx.x + u * THREADS, el = i / PIECES;
@@ -745,7 +761,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
         const int f = G::traceFace(tt[t], g) & 3;
         bool dr = false;
         if (A.faceTypes != nullptr) dr = A.faceTypes[(E0 + min(e, cells - 1)) * 4 + f] == SDG_FACE_DYNAMIC_RUPTURE;
-        mixRows<real>(tr[t], xs, e * kAplusLd<real> + f * 81, dr);
+        mixRows<real, kRoomy<O, real>>(tr[t], xs, e * kAplusLd<real> + f * 81, dr);
       }
     // local flux, two faces at a time: Q += rDivM_f diag(M2) W_f, in units of
     // (row tile, face), each unit's fragments loaded during the ones before
