@@ -21,7 +21,10 @@
 // All four faces' operands stay in LDS (110 KB in FP64 at ORDER 6, one
 // workgroup of eight waves per CU; 56 KB in FP32), which leaves two barriers
 // per tile.  Bound by the matrix instructions (FP64) or, on random links, by
-// the gather of four neighbours' DOFs per element.
+// the gather of four neighbours' DOFs per element; AminusT and the old DOFs are
+// loaded across the barriers (400k cells in FP64 at ORDER 6 from traces 2.04 ->
+// 1.93 ms, 350k in FP32 at ORDER 5 with LTS 1.09 -> 1.05, 100k in FP32 at ORDER
+// 6 from DOFs 537 -> 514 us).
 // From traces this replaced a kernel that went face by face, nine barriers a
 // tile, one wave per row tile: FP64 steps of 60k cells 608 -> 286 us at ORDER
 // 3, 487 -> 428 at 4, 793 -> 721 at 5, 2148 -> 1952 at 7; 400k cells at ORDER
@@ -43,6 +46,10 @@ struct NeighborCoeffs {
   real gts[O], sub[O];  // time-basis coefficients: GTS relation, sub-interval of a larger step
 };
 
+// what the neighbour pass reads: the neighbours' buffers, buffers or
+// derivatives (local time stepping), or the face traces rT_j I of the local pass
+constexpr int kFromDofs = 0, kFromLts = 1, kFromTraces = 2;
+
 // geometry and LDS of the neighbour kernel
 template <int O, typename real>
 struct NeighborGeo {
@@ -52,10 +59,15 @@ struct NeighborGeo {
   // element stride: the 16 elements' operand reads conflict-free, quads aligned
   static constexpr int ES = columnStride<real>(4 * FS);
   static constexpr int bytes = kElems * ES * static_cast<int>(sizeof(real)) +
-                               3 * G::B2 * O * (static_cast<int>(sizeof(real)) + 4) + 2048;
+                               3 * G::B2 * O * (static_cast<int>(sizeof(real)) + 4) + 1024;
   static constexpr int wanted = (163840 / bytes) * WAVES / 4;  // waves per SIMD that the LDS allows
-  static constexpr int cap = sizeof(real) == 8 ? 2 : 4;
-  static constexpr int SIMD_WAVES = maxOf(cdiv(WAVES, 4), wanted < cap ? wanted : cap);
+  // waves per SIMD asked of the register allocator: all that the LDS allows,
+  // but no more than two or four for the sums over derivatives (LTS) and the
+  // DOF operands of the high orders, which would spill
+  static constexpr int simdWaves(bool lean) {
+    const int cap = sizeof(real) == 8 ? (lean ? 3 : 2) : (lean ? 6 : 4);
+    return maxOf(cdiv(WAVES, 4), wanted < cap ? wanted : cap);
+  }
   static constexpr int MAXGROUPS = 7;  // sum over four sides of ceil(tasks / 16), 64 tasks
 };
 
@@ -72,12 +84,9 @@ __device__ inline void loadPair(const real* __restrict__ q, int row, real (&v)[2
   }
 }
 
-// what the neighbour pass reads: the neighbours' buffers, buffers or
-// derivatives (local time stepping), or the face traces rT_j I of the local pass
-constexpr int kFromDofs = 0, kFromLts = 1, kFromTraces = 2;
-
 template <typename real, int O, int SRC>
-__global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, real>::SIMD_WAVES)) void kNeighborMx(
+__global__ __launch_bounds__((NeighborGeo<O, real>::THREADS),
+                             (NeighborGeo<O, real>::simdWaves(SRC == kFromTraces || (SRC == kFromDofs && O <= 5)))) void kNeighborMx(
     int64_t n, const real* __restrict__ frag, const int* __restrict__ ranges, real* __restrict__ dofs,
     const real* __restrict__ integ, const real* __restrict__ deriv, const int32_t* __restrict__ neighbors,
     const uint8_t* __restrict__ faceRel, const real* __restrict__ aminus, const uint8_t* __restrict__ faceTypes,
@@ -87,6 +96,9 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
   using V4 = typename Vec<real>::V4;
   constexpr int B = G::B, B2 = G::B2, B2P = G::B2P, FS = N::FS, ES = N::ES, RS = sizeof(real);
   constexpr bool LTS = SRC == kFromLts;
+  // AminusT and the old DOFs ahead across the barriers, unless the registers for
+  // it cost waves (FP32 at ORDER 5 from traces, 60k cells: 101 us, 109 ahead)
+  constexpr bool AHEAD = LTS || N::wanted < 6;
   __shared__ __attribute__((aligned(16))) real sU[kElems * ES];  // U, then W: [element][face][quantity][B2P]
   __shared__ real sFP[3 * B2 * O];
   __shared__ int sFPCol[3 * B2 * O];
@@ -252,19 +264,24 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
       }
     }
   }
-  __syncthreads();
-
-  // phase 2: a task per 16-lane row, lane c its face rows c (and c + 16)
+  // phase 2: a task per 16-lane row, lane c its face rows c (and c + 16).
   constexpr int RF = cdiv(B2P, 16);
+  real rowA[9];  // lane c: row min(c, 8) of AminusT
+  auto loadA = [&](int t, real(&a)[9]) {
+    const real* const A = aminus + (E0 + min(t >> 2, cells - 1)) * lay.aminusStride + 81 * (t & 3) + min(c, 8);
+#pragma unroll
+    for (int p = 0; p < 9; ++p) a[p] = A[9 * p];
+  };
+  if constexpr (AHEAD) loadA(4 * w + g, rowA);
+  __syncthreads();
 #pragma unroll 1
   for (int t0 = 4 * w; t0 < 64; t0 += 4 * N::WAVES) {
     const int t = t0 + g;
     const int meta = sMeta[t], h = meta >> 1 & 3;
     const bool regular = meta & 1;
-    const real* const A = aminus + (E0 + min(t >> 2, cells - 1)) * lay.aminusStride + 81 * (t & 3) + min(c, 8);
-    real rowA[9];  // lane c: row min(c, 8) of AminusT
-#pragma unroll
-    for (int p = 0; p < 9; ++p) rowA[p] = A[9 * p];
+    real nextA[9];
+    if constexpr (AHEAD) loadA(min(t + 4 * N::WAVES, 63), nextA);
+    else loadA(t, rowA);
     real* const us = sU + (t >> 2) * ES + (t & 3) * FS;
     real u[RF][9];
 #pragma unroll
@@ -296,11 +313,25 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
       if (c + 16 * r < B2P)
 #pragma unroll
         for (int p = 0; p < 9; ++p) us[p * B2P + c + 16 * r] = regular && c + 16 * r < B2 ? wv[r][p] : real(0);
+    if constexpr (AHEAD)
+#pragma unroll
+      for (int p = 0; p < 9; ++p) rowA[p] = nextA[p];
   }
-  __syncthreads();
 
   // phase 3: wave (row tile, quantities 0-4 or 5-8)
   const int tile = w >> 1, p0 = 5 * (w & 1), np = (w & 1) ? 4 : 5;
+  const Buffer<real> q(dofs + E0 * lay.qStride, cells * lay.qStride);
+  const int cell = c < cells ? c * static_cast<int>(lay.qStride) * RS : kNowhere;
+  const int row = 16 * tile + 4 * g;
+  V4 old[5];
+  auto loadOld = [&] {
+#pragma unroll
+    for (int p = 0; p < 5; ++p)
+      old[p] = q.template loadQuad<B>(p < np ? cell : kNowhere, row, (p0 + p) * lay.ldq * RS);
+  };
+  if constexpr (AHEAD) loadOld();
+  __syncthreads();
+
   V4 acc[5];
 #pragma unroll
   for (int p = 0; p < 5; ++p) acc[p] = V4{0, 0, 0, 0};
@@ -320,13 +351,7 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS), (NeighborGeo<O, re
           if (p < np) acc[p] = mma(a[k], xr[f * FS + p * B2P + 4 * k], acc[p]);
       }
   }
-  const Buffer<real> q(dofs + E0 * lay.qStride, cells * lay.qStride);
-  const int cell = c < cells ? c * static_cast<int>(lay.qStride) * RS : kNowhere;
-  const int row = 16 * tile + 4 * g;
-  V4 old[5];
-#pragma unroll
-  for (int p = 0; p < 5; ++p)
-    old[p] = q.template loadQuad<B>(p < np ? cell : kNowhere, row, (p0 + p) * lay.ldq * RS);
+  if constexpr (!AHEAD) loadOld();
 #pragma unroll
   for (int p = 0; p < 5; ++p)
     q.storeQuad(old[p] + acc[p], p < np ? cell : kNowhere, row, B, (p0 + p) * lay.ldq * RS);
