@@ -25,8 +25,8 @@ int localPass(const EngineState& e, const double* coeffs, const sdg_layer* layer
       !mfma::vectorAccess(cellLayout(e, &own), own.dofs, own.time_integrated, "matrix-core local pass", v4))
     return SDG_ERR_INVALID;
   mx::LtsOut out{};
-  if (lts != nullptr) out = {lts->setup, lts->deriv, lts->reset, 0};
-  return launchLocalTracesMx(e, coeffs, &own, lts != nullptr ? &out : nullptr, stream);
+  if (lts != nullptr) out = {lts->setup, lts->deriv};
+  return launchLocalTracesMx(e, coeffs, lts != nullptr ? lts->reset : 1, &own, lts != nullptr ? &out : nullptr, stream);
 }
 }  // namespace
 

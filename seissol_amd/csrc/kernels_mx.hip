@@ -11,6 +11,7 @@
 
 #include "engine.h"
 #include "global_matrices.h"
+#include "mfma_common.h"
 #include "mx_common.h"
 
 namespace sdg {
@@ -178,45 +179,76 @@ bool hasMx(const EngineState& e) { return e.mxFrags != nullptr && e.kernels == S
 
 bool hasNeighborMx(const EngineState& e) { return hasMx(e) && e.mxNeighbor; }
 
+namespace {
+// every cell of the layer in one step
+mx::ClusterStep whole(const sdg_layer* layer, const double* coeffs, const double* sub, int reset) {
+  return {0, layer->num_elements, coeffs, sub, reset};
+}
+}  // namespace
+
 int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
                      const double* subtimeCoeffs, hipStream_t stream) {
-  return orders(e, [&](auto o) { return o.neighbor(e, layer, timeCoeffs, subtimeCoeffs, false, stream); });
+  const mx::ClusterStep step = whole(layer, timeCoeffs, subtimeCoeffs, 1);
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, &step, 1, false, stream); });
+}
+
+int launchNeighborClustersMx(const EngineState& e, const mx::ClusterStep* steps, int clusters, const sdg_layer* layer,
+                             hipStream_t stream) {
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, steps, clusters, false, stream); });
 }
 
 int launchNeighborTracesMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  return orders(e, [&](auto o) { return o.neighbor(e, layer, nullptr, nullptr, true, stream); });
+  const mx::ClusterStep step = whole(layer, nullptr, nullptr, 1);
+  return orders(e, [&](auto o) { return o.neighbor(e, layer, &step, 1, true, stream); });
 }
 
 int launchAderMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
-  const mx::LtsOut lts{layer->lts_setup, layer->derivatives, 1, 0};
-  return orders(e, [&](auto o) { return o.local(e, mx::kPredict, coeffs, layer, false, &lts, stream); });
+  const mx::LtsOut lts{layer->lts_setup, layer->derivatives};
+  const mx::ClusterStep step = whole(layer, coeffs, nullptr, 1);
+  return orders(e, [&](auto o) { return o.local(e, mx::kPredict, &step, 1, layer, false, &lts, stream); });
 }
 
 int launchLocalMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  return orders(e, [&](auto o) { return o.local(e, mx::kFlux, nullptr, layer, false, nullptr, stream); });
+  const mx::ClusterStep step = whole(layer, nullptr, nullptr, 1);
+  return orders(e, [&](auto o) { return o.local(e, mx::kFlux, &step, 1, layer, false, nullptr, stream); });
 }
 
 int launchAderLocalMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream) {
   // only the FP64 neighbour pass reads traces of this kernel
   const bool fp64 = e.arithmetic == SDG_FP64;
   // FP64: the buffer and derivatives of every cell; FP32: per the layer's LTS setup where it has one
-  const mx::LtsOut lts{fp64 ? nullptr : layer->lts_setup, layer->derivatives, 1, 0};
+  const mx::LtsOut lts{fp64 ? nullptr : layer->lts_setup, layer->derivatives};
   const bool some = lts.deriv != nullptr || lts.setup != nullptr;
+  const mx::ClusterStep step = whole(layer, coeffs, nullptr, 1);
   return orders(e, [&](auto o) {
-    return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, fp64, some ? &lts : nullptr, stream);
+    return o.local(e, mx::kPredict | mx::kFlux, &step, 1, layer, fp64, some ? &lts : nullptr, stream);
   });
 }
 
-int launchLocalTracesMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, const mx::LtsOut* lts,
-                        hipStream_t stream) {
-  return orders(e, [&](auto o) { return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, true, lts, stream); });
+int launchLocalTracesMx(const EngineState& e, const double* coeffs, int reset, const sdg_layer* layer,
+                        const mx::LtsOut* lts, hipStream_t stream) {
+  const mx::ClusterStep step = whole(layer, coeffs, nullptr, reset);
+  return orders(e, [&](auto o) { return o.local(e, mx::kPredict | mx::kFlux, &step, 1, layer, true, lts, stream); });
+}
+
+int launchLocalClustersMx(const EngineState& e, const mx::ClusterStep* steps, int clusters, const sdg_layer* layer,
+                          hipStream_t stream) {
+  bool v4 = false;
+  if (matrixCore(e.arithmetic) &&
+      !mfma::vectorAccess(cellLayout(e, layer), layer->dofs, layer->time_integrated, "matrix-core local pass", v4))
+    return SDG_ERR_INVALID;
+  const mx::LtsOut lts{layer->lts_setup, layer->derivatives};
+  return orders(e, [&](auto o) {
+    return o.local(e, mx::kPredict | mx::kFlux, steps, clusters, layer, false, &lts, stream);
+  });
 }
 
 int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
                              hipStream_t stream) {
-  const mx::LtsOut lts{layer->lts_setup, layer->derivatives, resetBuffers, 0};
+  const mx::LtsOut lts{layer->lts_setup, layer->derivatives};
+  const mx::ClusterStep step = whole(layer, coeffs, nullptr, resetBuffers);
   return orders(e, [&](auto o) {
-    return o.local(e, mx::kPredict | mx::kFlux, coeffs, layer, e.arithmetic == SDG_FP64, &lts, stream);
+    return o.local(e, mx::kPredict | mx::kFlux, &step, 1, layer, e.arithmetic == SDG_FP64, &lts, stream);
   });
 }
 

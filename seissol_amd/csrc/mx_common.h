@@ -245,14 +245,59 @@ struct Buffer {
 
 // local-time-stepping outputs of the local pass (TimeCluster.cpp:380-434):
 // per cell its LtsSetup bits say whether it stores its buffer (accumulated
-// over the sub-steps a slower neighbour sees unless `reset`) and its
+// over the sub-steps a slower neighbour sees unless its cluster resets it) and its
 // derivatives; setup == nullptr: the buffer and (if any) the derivatives of
 // every cell
 struct LtsOut {
   const uint16_t* setup = nullptr;
   void* deriv = nullptr;
+};
+
+// One launch over several clusters of a layer (local time stepping: the
+// clusters that step at the same time), each with its own range of cells, time
+// coefficients and reset flag; tiles do not cross the ranges.  Small clusters
+// are bound by the chain of one tile, 20 us whatever their size, so they run
+// beside the others.
+struct ClusterStep {
+  int64_t start = 0, end = 0;  // cells of the layer
+  const double* coeffs = nullptr;  // time integral over the cluster's step
+  const double* sub = nullptr;     // neighbour pass: over the sub-interval of a larger step
   int reset = 1;
-  int pad_ = 0;
+};
+constexpr int kMaxClusters = 16;
+
+template <int O, typename real, int SETS>
+struct Segments {
+  int count = 0;
+  int firstBlock[kMaxClusters] = {};
+  int reset[kMaxClusters] = {};
+  int64_t start[kMaxClusters] = {}, end[kMaxClusters] = {};
+  real c[kMaxClusters][SETS][O] = {};
+
+  // the number of blocks
+  int64_t fill(const ClusterStep* steps, int n) {
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) {
+      if (steps[i].end <= steps[i].start) continue;
+      firstBlock[count] = static_cast<int>(blocks);
+      start[count] = steps[i].start;
+      end[count] = steps[i].end;
+      reset[count] = steps[i].reset;
+      for (int d = 0; d < O; ++d) {
+        c[count][0][d] = steps[i].coeffs != nullptr ? static_cast<real>(steps[i].coeffs[d]) : real(0);
+        if (SETS == 2) c[count][SETS - 1][d] = steps[i].sub != nullptr ? static_cast<real>(steps[i].sub[d]) : real(0);
+      }
+      blocks += (steps[i].end - steps[i].start + kElems - 1) / kElems;
+      ++count;
+    }
+    return blocks;
+  }
+  // the segment of this block (uniform)
+  __device__ inline int find() const {
+    int s = 0;
+    for (int i = 1; i < count; ++i) s = static_cast<int>(blockIdx.x) >= firstBlock[i] ? i : s;
+    return s;
+  }
 };
 
 // parts of the local pass
@@ -261,11 +306,11 @@ constexpr int kPredict = 1, kFlux = 2;
 // host entry points of one order (explicitly instantiated per order)
 template <int O>
 struct Order {
-  static int local(const EngineState& e, int parts, const double* coeffs, const sdg_layer* layer, bool traces,
-                   const LtsOut* lts, hipStream_t stream);
-  // neighbour flux; gts / sub: time coefficients of the LTS pass (nullptr: global time stepping);
-  // traces: from the layer's face traces instead of the neighbours' DOFs
-  static int neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub, bool traces,
+  static int local(const EngineState& e, int parts, const ClusterStep* steps, int clusters, const sdg_layer* layer,
+                   bool traces, const LtsOut* lts, hipStream_t stream);
+  // neighbour flux; steps without coefficients: global time stepping; traces: from the layer's face traces
+  // instead of the neighbours' DOFs
+  static int neighbor(const EngineState& e, const sdg_layer* layer, const ClusterStep* steps, int clusters, bool traces,
                       hipStream_t stream);
 };
 
@@ -274,6 +319,11 @@ struct Order {
 // the fused local pass in FP32 or FP64 writing the layer's face traces, with
 // the outputs of `lts` (nullptr: neither derivatives nor LTS setup; a layer
 // without time_integrated: no buffer)
-int launchLocalTracesMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, const mx::LtsOut* lts,
-                        hipStream_t stream);
+int launchLocalTracesMx(const EngineState& e, const double* coeffs, int reset, const sdg_layer* layer,
+                        const mx::LtsOut* lts, hipStream_t stream);
+// the LTS passes of several clusters of a layer at once (its arrays whole)
+int launchLocalClustersMx(const EngineState& e, const mx::ClusterStep* steps, int clusters, const sdg_layer* layer,
+                          hipStream_t stream);
+int launchNeighborClustersMx(const EngineState& e, const mx::ClusterStep* steps, int clusters, const sdg_layer* layer,
+                             hipStream_t stream);
 }  // namespace sdg

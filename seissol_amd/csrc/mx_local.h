@@ -49,11 +49,6 @@ namespace sdg {
 namespace mx {
 namespace {
 
-template <int O, typename real>
-struct Coeffs {
-  real c[O];
-};
-
 // the block of the predictor matrices kept in LDS (see lateStress)
 constexpr int kLateRows = 10, kLateSteps = 5, kLate = 3 * kLateSteps * 4 * kLateRows;
 
@@ -410,10 +405,12 @@ __device__ inline void mixRows(typename Vec<real>::V4 (&t)[9], const real* lds, 
 
 template <typename real, int O>
 struct LocalArgs {
-  int64_t n;
+  int64_t E0;  // the tile's first cell
+  int cells;   // its cells: columns beyond load zeros and store nothing
+  int reset;
   const real* frag;
   const int* ranges;
-  const Coeffs<O, real>& cf;
+  const real (&c)[O];
   real* dofs;
   real* integ;
   real* traces;
@@ -431,8 +428,8 @@ template <typename real, int O, bool LATE>
 __device__ inline void stage(const LocalArgs<real, O>& A, real* const sStar, real* const sLate) {
   using G = Geo<O>;
   constexpr int THREADS = Waves<O, real>::THREADS, N = cdiv(kElems * 72, THREADS), NL = LATE ? cdiv(kLate, THREADS) : 1;
-  const int64_t E0 = static_cast<int64_t>(blockIdx.x) * kElems;
-  const int cells = static_cast<int>(min(A.n - E0, int64_t(kElems)));
+  const int64_t E0 = A.E0;
+  const int cells = A.cells;
   const CellLayout& lay = A.lay;
   const Buffer<real> star(A.star + E0 * lay.starStride, (cells - 1) * lay.starStride + (lay.starCompact ? 72 : 243));
   const int stride = static_cast<int>(lay.starStride) * static_cast<int>(sizeof(real));
@@ -488,9 +485,8 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
   int tile[TW];
   tile[0] = w >> 1;
   if constexpr (TW == 2) tile[1] = 2 * PAIRS - 1 - (w >> 1);
-  // the tile's cells: columns beyond the last cell load zeros and store nothing
-  const int64_t E0 = static_cast<int64_t>(blockIdx.x) * kElems;
-  const int cells = static_cast<int>(min(A.n - E0, int64_t(kElems)));
+  const int64_t E0 = A.E0;
+  const int cells = A.cells;
   const Buffer<real> dofs(A.dofs + E0 * lay.qStride, cells * lay.qStride);
   const Buffer<real> integ(A.integ + E0 * lay.qStride, A.integ != nullptr ? cells * lay.qStride : 0);
   const int cell = e < cells ? e * static_cast<int>(lay.qStride) * RS : kNowhere;
@@ -578,7 +574,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
-      for (int p = 0; p < NP; ++p) ia[t][p] *= A.cf.c[0];
+      for (int p = 0; p < NP; ++p) ia[t][p] *= A.c[0];
     __syncthreads();
     [[maybe_unused]] int doff = 9 * ldq;
     // dQ_{d-1} is read at row source(d), dQ_d stored at row target(d)
@@ -587,7 +583,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
     // dQ_d of row tile t: into X, the time integral and the derivatives
     auto finish = [&](int d, int m, int t, V4(&y)[NP]) {
       const int row = 16 * tile[t] + 4 * g, ldm = lay.rows(m) * RS;
-      const real cd = A.cf.c[d];
+      const real cd = A.c[d];
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
 #pragma unroll
@@ -649,7 +645,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
       if constexpr (LTS) mine = (setup & SDG_LTS_HAS_BUFFERS) ? cell : kNowhere;
       [[maybe_unused]] int before = kNowhere;  // the old buffer, where it accumulates (else zeros are loaded)
       if constexpr (LTS)
-        before = A.lts.setup != nullptr && !A.lts.reset && (setup & SDG_LTS_ACCUMULATE_BUFFERS) ? mine : kNowhere;
+        before = A.lts.setup != nullptr && !A.reset && (setup & SDG_LTS_ACCUMULATE_BUFFERS) ? mine : kNowhere;
 #pragma unroll
       for (int t = 0; t < TW; ++t) {
         const int row = 16 * tile[t] + 4 * g;
@@ -828,32 +824,31 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
 // flux from the predictor's time integral, or without it from `integ`)
 template <typename real, int O, int PARTS, bool LTS>
 __global__ __launch_bounds__((Waves<O, real>::THREADS), (LocalLds<O, real>::SIMD_WAVES)) void kLocalMx(
-    int64_t n, const real* __restrict__ frag, const int* __restrict__ ranges, Coeffs<O, real> cf,
-    real* __restrict__ dofs, real* __restrict__ integ, real* __restrict__ traces, const real* __restrict__ starAll,
+    Segments<O, real, 1> seg, const real* __restrict__ frag, const int* __restrict__ ranges, real* __restrict__ dofs, real* __restrict__ integ, real* __restrict__ traces, const real* __restrict__ starAll,
     const real* __restrict__ aplus, const uint8_t* __restrict__ faceTypes, CellLayout lay, LtsOut lts) {
   __shared__ __attribute__((aligned(16))) real xs[LocalLds<O, real>::X];
   __shared__ real sStar[kElems * kStarLd];
   __shared__ real sLate[kLate];
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const LocalArgs<real, O> A{n, frag, ranges, cf, dofs, integ, traces, starAll, aplus, faceTypes, lay, lts};
+  const int s = LTS ? seg.find() : 0;
+  const int64_t E0 = seg.start[s] + static_cast<int64_t>(static_cast<int>(blockIdx.x) - (LTS ? seg.firstBlock[s] : 0)) * kElems;
+  const int cells = static_cast<int>(min(seg.end[s] - E0, int64_t(kElems)));
+  const LocalArgs<real, O> A{E0, cells, seg.reset[s], frag, ranges, seg.c[s][0], dofs, integ, traces, starAll, aplus, faceTypes, lay, lts};
   if (w & 1) localWave<real, O, PARTS, LTS, true>(A, xs, sStar, sLate, w);
   else localWave<real, O, PARTS, LTS, false>(A, xs, sStar, sLate, w);
 }
 
 template <typename real, int O>
-int localImpl(const EngineState& st, int parts, const double* coeffs, const sdg_layer* L, bool writeTraces,
-              const LtsOut* lts, hipStream_t stream) {
-  using G = Geo<O>;
-  const int64_t n = L->num_elements;
-  if (n == 0) return SDG_OK;
-  Coeffs<O, real> cf{};
-  if (coeffs != nullptr)
-    for (int i = 0; i < O; ++i) cf.c[i] = static_cast<real>(coeffs[i]);
+int localImpl(const EngineState& st, int parts, const ClusterStep* steps, int clusters, const sdg_layer* L,
+              bool writeTraces, const LtsOut* lts, hipStream_t stream) {
+  Segments<O, real, 1> seg;
+  const int64_t blocks = seg.fill(steps, clusters);
+  if (blocks == 0) return SDG_OK;
   const CellLayout lay = cellLayout(st, L);
-  const dim3 grid(static_cast<unsigned>((n + kElems - 1) / kElems));
+  const dim3 grid(static_cast<unsigned>(blocks));
   auto launch = [&](auto partsI, auto ltsI) {
     kLocalMx<real, O, decltype(partsI)::value, decltype(ltsI)::value><<<grid, Waves<O, real>::THREADS, 0, stream>>>(
-        n, static_cast<const real*>(st.mxFrags), st.mxRanges, cf, static_cast<real*>(L->dofs),
+        seg, static_cast<const real*>(st.mxFrags), st.mxRanges, static_cast<real*>(L->dofs),
         static_cast<real*>(L->time_integrated), writeTraces ? static_cast<real*>(L->face_traces) : nullptr,
         static_cast<const real*>(L->star), static_cast<const real*>(L->aplus), L->face_types, lay,
         lts != nullptr ? *lts : LtsOut{});
@@ -869,10 +864,10 @@ int localImpl(const EngineState& st, int parts, const double* coeffs, const sdg_
 }  // namespace
 
 template <int O>
-int Order<O>::local(const EngineState& e, int parts, const double* coeffs, const sdg_layer* layer, bool traces,
-                    const LtsOut* lts, hipStream_t stream) {
-  return e.arithmetic == SDG_FP64 ? localImpl<double, O>(e, parts, coeffs, layer, traces, lts, stream)
-                                  : localImpl<float, O>(e, parts, coeffs, layer, traces, lts, stream);
+int Order<O>::local(const EngineState& e, int parts, const ClusterStep* steps, int clusters, const sdg_layer* layer,
+                    bool traces, const LtsOut* lts, hipStream_t stream) {
+  return e.arithmetic == SDG_FP64 ? localImpl<double, O>(e, parts, steps, clusters, layer, traces, lts, stream)
+                                  : localImpl<float, O>(e, parts, steps, clusters, layer, traces, lts, stream);
 }
 
 }  // namespace mx

@@ -41,11 +41,6 @@ namespace sdg {
 namespace mx {
 namespace {
 
-template <int O, typename real>
-struct NeighborCoeffs {
-  real gts[O], sub[O];  // time-basis coefficients: GTS relation, sub-interval of a larger step
-};
-
 // what the neighbour pass reads: the neighbours' buffers, buffers or
 // derivatives (local time stepping), or the face traces rT_j I of the local pass
 constexpr int kFromDofs = 0, kFromLts = 1, kFromTraces = 2;
@@ -87,10 +82,10 @@ __device__ inline void loadPair(const real* __restrict__ q, int row, real (&v)[2
 template <typename real, int O, int SRC>
 __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS),
                              (NeighborGeo<O, real>::simdWaves(SRC == kFromTraces || (SRC == kFromDofs && O <= 5)))) void kNeighborMx(
-    int64_t n, const real* __restrict__ frag, const int* __restrict__ ranges, real* __restrict__ dofs,
+    Segments<O, real, 2> seg, const real* __restrict__ frag, const int* __restrict__ ranges, real* __restrict__ dofs,
     const real* __restrict__ integ, const real* __restrict__ deriv, const int32_t* __restrict__ neighbors,
     const uint8_t* __restrict__ faceRel, const real* __restrict__ aminus, const uint8_t* __restrict__ faceTypes,
-    const uint16_t* __restrict__ setups, NeighborCoeffs<O, real> cf, CellLayout lay) {
+    const uint16_t* __restrict__ setups, CellLayout lay) {
   using G = Geo<O>;
   using N = NeighborGeo<O, real>;
   using V4 = typename Vec<real>::V4;
@@ -109,8 +104,9 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS),
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int g = lane >> 4, c = lane & 15;
-  const int64_t E0 = static_cast<int64_t>(blockIdx.x) * kElems;
-  const int cells = static_cast<int>(min(n - E0, int64_t(kElems)));
+  const int s = LTS ? seg.find() : 0;
+  const int64_t E0 = seg.start[s] + static_cast<int64_t>(static_cast<int>(blockIdx.x) - (LTS ? seg.firstBlock[s] : 0)) * kElems;
+  const int cells = static_cast<int>(min(seg.end[s] - E0, int64_t(kElems)));
 
   for (int i = threadIdx.x; i < 3 * B2 * O; i += N::THREADS) {
     sFP[i] = frag[G::fP + i];
@@ -207,7 +203,7 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS),
           staticFor<O>([&](auto dI) {
             constexpr int d = decltype(dI)::value, m = basis3(O - d);
             const int ldm = lay.rows(m);
-            const real cd = gts ? cf.gts[d] : cf.sub[d];
+            const real cd = gts ? seg.c[s][0][d] : seg.c[s][1][d];  // GTS relation, sub-interval of a larger step
 #pragma unroll
             for (int k = 0; k < cdiv(m, 8); ++k)
 #pragma unroll
@@ -358,28 +354,23 @@ __global__ __launch_bounds__((NeighborGeo<O, real>::THREADS),
 }
 
 template <typename real, int O>
-int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, const double* sub, bool traces,
+int neighborImpl(const EngineState& st, const sdg_layer* L, const ClusterStep* steps, int clusters, bool traces,
                  hipStream_t stream) {
   using N = NeighborGeo<O, real>;
-  const int64_t n = L->num_elements;
-  if (n == 0) return SDG_OK;
-  NeighborCoeffs<O, real> cf{};
-  if (gts != nullptr)
-    for (int i = 0; i < O; ++i) {
-      cf.gts[i] = static_cast<real>(gts[i]);
-      cf.sub[i] = static_cast<real>(sub[i]);
-    }
+  Segments<O, real, 2> seg;
+  const int64_t blocks = seg.fill(steps, clusters);
+  if (blocks == 0) return SDG_OK;
   const CellLayout lay = cellLayout(st, L);
-  const dim3 grid(static_cast<unsigned>((n + kElems - 1) / kElems));
+  const dim3 grid(static_cast<unsigned>(blocks));
   auto launch = [&](auto srcI) {
     kNeighborMx<real, O, decltype(srcI)::value><<<grid, N::THREADS, 0, stream>>>(
-        n, static_cast<const real*>(st.mxFrags), st.mxRanges, static_cast<real*>(L->dofs),
+        seg, static_cast<const real*>(st.mxFrags), st.mxRanges, static_cast<real*>(L->dofs),
         static_cast<const real*>(traces ? L->face_traces : L->time_integrated),
         static_cast<const real*>(L->derivatives), L->face_neighbors, L->face_relations,
-        static_cast<const real*>(L->aminus), L->face_types, L->lts_setup, cf, lay);
+        static_cast<const real*>(L->aminus), L->face_types, L->lts_setup, lay);
   };
   if (traces) launch(std::integral_constant<int, kFromTraces>{});
-  else if (gts != nullptr && L->lts_setup != nullptr) launch(std::integral_constant<int, kFromLts>{});
+  else if (steps[0].coeffs != nullptr && L->lts_setup != nullptr) launch(std::integral_constant<int, kFromLts>{});
   else launch(std::integral_constant<int, kFromDofs>{});
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;
@@ -388,10 +379,10 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, const double* gts, c
 }  // namespace
 
 template <int O>
-int Order<O>::neighbor(const EngineState& e, const sdg_layer* layer, const double* gts, const double* sub, bool traces,
+int Order<O>::neighbor(const EngineState& e, const sdg_layer* layer, const ClusterStep* steps, int clusters, bool traces,
                        hipStream_t stream) {
-  return e.arithmetic == SDG_FP64 ? neighborImpl<double, O>(e, layer, gts, sub, traces, stream)
-                                  : neighborImpl<float, O>(e, layer, gts, sub, traces, stream);
+  return e.arithmetic == SDG_FP64 ? neighborImpl<double, O>(e, layer, steps, clusters, traces, stream)
+                                  : neighborImpl<float, O>(e, layer, steps, clusters, traces, stream);
 }
 
 }  // namespace mx

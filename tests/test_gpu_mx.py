@@ -165,3 +165,43 @@ def test_neighbour_pass_from_traces(gpu, arith, order, tol):
         err = float((got - want).abs().max() / want.abs().max())
         print(f"  largest difference / largest value {err:.1e}", flush=True)
         assert err < tol
+
+
+# clusters that step together share a launch: a cluster of one cell, an empty one, ragged ones, and a launch
+# of several with another variant's between them, against the VALU kernels cluster by cluster
+@pytest.mark.parametrize("arith,tol", [("fp64", 1e-12), ("fp32", 5e-5), ("f16x3", 5e-5)])
+@pytest.mark.parametrize("order", [3, 6])
+@pytest.mark.parametrize("graph", [False, True])
+def test_clusters_in_one_launch_equal_the_valu_kernels(gpu, order, arith, tol, graph):
+    import torch
+    starts = [0, 100, 101, 101, 134, 150]
+    n, C_ = starts[-1], len(starts) - 1
+    print(f"clusters {arith} order={order} graph={graph}", flush=True)
+    sides = []
+    for valu in (False, True):
+        eng = Engine(order, arith)
+        eng.set_layout(0, "compact")
+        a = random_layer(eng, order, arith, n, 0, "compact", 11 * order)
+        gen = torch.Generator(device="cuda").manual_seed(order)
+        draw = lambda hi, shape, t: torch.randint(0, hi, shape, generator=gen, device="cuda").to(t)
+        a["neighbors"] = draw(n, (n, 4), torch.int32)
+        a["relations"] = torch.stack([draw(4, (n, 4), torch.uint8), draw(3, (n, 4), torch.uint8)], -1)
+        a["aminus"] = torch.rand((n, 4, 81), generator=gen, device="cuda", dtype=a["dofs"].dtype) * 2 - 1
+        a["setup"] = draw(1 << 11, (n,), torch.int16)
+        for k in ("star", "aplus", "aminus"):
+            a[k] *= 0.02  # 16 steps without growth
+        v = a["view"]
+        v.star, v.aplus, v.aminus = ptr(a["star"]), ptr(a["aplus"]), ptr(a["aminus"])
+        v.face_neighbors, v.face_relations, v.lts_setup = ptr(a["neighbors"]), ptr(a["relations"]), ptr(a["setup"])
+        handle, cuts = C.c_void_p(), (C.c_int64 * (C_ + 1))(*starts)
+        check(lib().sdg_lts_create(C.byref(handle), eng.handle, C.byref(v), C_, cuts, 1e-2), "create")
+        for c in range(C_):
+            if valu or c == 3:
+                check(lib().sdg_lts_set_tile_variant(handle, c, 0, 1), "local variant")
+                check(lib().sdg_lts_set_tile_variant(handle, c, 1, 1), "neighbour variant")
+        s = torch.cuda.current_stream().cuda_stream
+        check((lib().sdg_lts_graph_advance if graph else lib().sdg_lts_advance)(handle, 1, s), "advance")
+        torch.cuda.synchronize()
+        check(lib().sdg_lts_destroy(handle), "destroy")
+        sides.append(a)
+    same(*sides, ("dofs", "integrated", "derivatives"), tol, f"clusters {arith}")
