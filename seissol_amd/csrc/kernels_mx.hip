@@ -91,7 +91,9 @@ int uploadOrder(EngineState& s, const double* gm) {
     }
   }
   for (int t = 0; t < G::MTF; ++t) {
+    // k-steps from the last columns to the first (see gemm, mx_local.h)
     const Matrix F = [=](int r, int c) {
+      c = 4 * (KS - 1 - c / 4) + c % 4;
       const int f = G::traceFace(t, r / 4), m = G::traceRow(t, r / 4) + r % 4;
       return m < B2 && c < B ? gm[g.fMrT + (f * B2 + m) * B + c] : 0.0;
     };
@@ -101,7 +103,7 @@ int uploadOrder(EngineState& s, const double* gm) {
           return m < B2 ? F(r, c) / gm[g.mass2 + m] : 0.0;
         },
         KS, frags.data() + G::trace + static_cast<int64_t>(t) * KS * 64);
-    tileRange({F}, 16, B, tolF, 4, ranges.data() + G::rTrace + 2 * t);
+    tileRange({F}, 16, G::KB, tolF, 4, ranges.data() + G::rTrace + 2 * t);
   }
   // rT_j of the neighbour pass: lane l of block k holds columns 8 k + 2 (l / 16) + {0, 1}
   const double tolU = largest(gm + g.rT, 4LL * B2 * B);

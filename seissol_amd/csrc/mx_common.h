@@ -63,7 +63,7 @@ struct Geo {
   // fragment offsets (reals)
   static constexpr int64_t ck = 0;                               // [MT][3][KS]
   static constexpr int64_t vol = ck + 3LL * MT * KS * 64;        // [MT][3][KS]
-  static constexpr int64_t trace = vol + 3LL * MT * KS * 64;     // [MTF][KS]     rT_f = fMrT_f / M2
+  static constexpr int64_t trace = vol + 3LL * MT * KS * 64;     // [MTF][KS]     rT_f = fMrT_f / M2, last k-step first
   static constexpr int64_t flux = trace + 1LL * MTF * KS * 64;   // [MT][4][KSF]  rDivM_f diag(M2)
   // neighbour pass: rT_j in blocks of 8 columns (a lane's two consecutive
   // ones in one load), rDivM_f, and fP_h as rows of O (value, column) entries

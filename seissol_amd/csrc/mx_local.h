@@ -333,9 +333,13 @@ __device__ inline void lateVelocity(const real* a, const real* x, const real* sS
   }
 }
 
-// acc[q] += A(tile) X_q, q < NQ, over the k-steps of `run` (one direction); x:
+// acc[q] += A(tile) X_q, q < NQ, over the k-steps of `run`, which are stored
+// from the last rows of X to the first: the high degrees, small in a smooth
+// solution and with many columns that feed few rows, are summed first, so that
+// a matrix instruction, which rounds every product it adds, has smaller sums to
+// round (error of the traces' products at ORDER 6 1.9e-7 -> 1.1e-7 in FP32); x:
 // the lane's column of the first quantity at row g; `cur` and `next` as above
-template <int LD, int NQ, int U, typename real>
+template <int KS, int LD, int NQ, int U, typename real>
 __device__ inline void gemm(typename Vec<real>::V4 (&acc)[NQ], const Run<real>& run, const Run<real>& next,
                             const real* x, int lane, real (&cur)[U]) {
 #pragma unroll 1
@@ -353,7 +357,7 @@ __device__ inline void gemm(typename Vec<real>::V4 (&acc)[NQ], const Run<real>& 
 #pragma unroll
       for (int u = 0; u < XU; ++u)
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) v[u][q] = x[q * 16 * LD + 4 * min(k + u0 + u, run.hi - 1)];
+        for (int q = 0; q < NQ; ++q) v[u][q] = x[q * 16 * LD + 4 * (KS - 1 - min(k + u0 + u, run.hi - 1))];
 #pragma unroll
       for (int u = 0; u < XU; ++u)
         if (k + u0 + u < run.hi) {
@@ -712,7 +716,7 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
 #pragma unroll
       for (int q = 0; q < 9; ++q) tr[t][q] = V4{0, 0, 0, 0};
       if (tt[t] < G::MTF) {
-        gemm<LD, 9, U, real>(tr[t], trace[t], trace[t + 1 < TT ? t + 1 : t], xr, lane, aheadT);
+        gemm<KS, LD, 9, U, real>(tr[t], trace[t], trace[t + 1 < TT ? t + 1 : t], xr, lane, aheadT);
         const int f = G::traceFace(tt[t], g), row = G::traceRow(tt[t], g);
         if (A.traces != nullptr) {
           const int at = e < cells && row < B2P ? ((e * 4 + f) * 9 * B2P + row) * RS : kNowhere;
@@ -761,6 +765,13 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
       }
     // local flux, two faces at a time: Q += rDivM_f diag(M2) W_f, in units of
     // (row tile, face), each unit's fragments loaded during the ones before
+    // In FP32 two faces' flux is summed on its own before it joins the rest: a
+    // matrix instruction rounds every product it adds, and on top of the volume's
+    // sum, twice the result, every one of these roundings would be larger (error
+    // of the local pass against 64 bits at ORDER 6 3.9e-7 -> 3.1e-7, with the
+    // traces' order of summation 2.7e-7; 1M cells 7.24 -> 7.26 ms a step, four
+    // LTS clusters of 600k cells at ORDER 5 22.70 -> 22.84)
+    constexpr bool OWN = sizeof(real) == 4;
     constexpr int KSF = G::KSF, UNITS = 2 * TW, FAR = VEL && sizeof(real) == 4 ? 2 : 1;
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
@@ -791,17 +802,26 @@ __device__ inline void localWave(const LocalArgs<real, O>& A, real* const xs, re
               *reinterpret_cast<V4*>(xs + (p * 16 + e) * LD + (f & 1) * B2P + row) = tr[t][p];
         }
       __syncthreads();
+      [[maybe_unused]] V4 pair[NP];
 #pragma unroll
       for (int u = 0; u < UNITS; ++u) {
         if (u + FAR < UNITS) load(u + FAR);
+        if (OWN && u % 2 == 0)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) pair[p] = V4{0, 0, 0, 0};
         const real* const x = xr + P0 * 16 * LD + u % 2 * B2P;
 #pragma unroll
         for (int k = 0; k < KSF; ++k)
           if (k >= lo[u] && k < hi[u]) {  // uniform
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
-              acc[u / 2][p] = mma(a[u % (FAR + 1)][k], x[p * 16 * LD + 4 * k], acc[u / 2][p]);
+            for (int p = 0; p < NP; ++p) {
+              V4& sum = OWN ? pair[p] : acc[u / 2][p];
+              sum = mma(a[u % (FAR + 1)][k], x[p * 16 * LD + 4 * k], sum);
+            }
           }
+        if (OWN && u % 2 == 1)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) acc[u / 2][p] += pair[p];
         __builtin_amdgcn_sched_barrier(0);
       }
     }

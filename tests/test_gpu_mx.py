@@ -9,6 +9,7 @@ import pytest
 from seissol_amd import _capi
 from seissol_amd._capi import check, lib, ptr
 from seissol_amd.kernels import Engine, global_matrices, num_basis, num_face_basis, padded_face_basis
+from seissol_amd.proxy import DeviceLayer, make_setup, run_proxy
 
 pytestmark = pytest.mark.gpu
 
@@ -205,3 +206,25 @@ def test_clusters_in_one_launch_equal_the_valu_kernels(gpu, order, arith, tol, g
         check(lib().sdg_lts_destroy(handle), "destroy")
         sides.append(a)
     same(*sides, ("dofs", "integrated", "derivatives"), tol, f"clusters {arith}")
+
+
+# A step's rounding against 64 bits on the same single-precision inputs.  The bounds are the errors that
+# the split products the two forms are named after (two scaled fp16 planes, three bf16 planes) had in
+# this test: what runs in their place may not be less accurate.
+@pytest.mark.parametrize("arith,order,bound", [
+    ("f16x3", 3, 1.79e-7), ("f16x3", 4, 1.97e-7), ("f16x3", 5, 2.11e-7), ("f16x3", 6, 2.36e-7), ("f16x3", 7, 2.58e-7),
+    ("bf16x6", 4, 1.90e-7), ("bf16x6", 5, 2.12e-7), ("bf16x6", 6, 2.38e-7), ("bf16x6", 7, 2.74e-7)])
+def test_a_step_is_as_accurate_as_the_split_products(gpu, arith, order, bound):
+    import torch
+    print(f"step accuracy {arith} order={order}", flush=True)
+    setup = make_setup(order, n=3000, mesh="proxy", seed=17)
+    layers = [(eng, DeviceLayer(eng, setup)) for eng in (Engine(order, arith), Engine(order, "fp64"))]
+    for k in ("dofs", "star", "aplus", "aminus"):
+        getattr(layers[1][1], k).copy_(getattr(layers[0][1], k))
+    for eng, layer in layers:
+        run_proxy(eng, layer, "all", 1, setup.dt)
+    torch.cuda.synchronize()
+    got, want = (layer.dofs.double() for _, layer in layers)
+    err = float((got - want).norm() / want.norm())
+    print(f"  error {err:.3e}, split products {bound:.2e}", flush=True)
+    assert err <= bound
