@@ -135,11 +135,11 @@ __device__ inline bool faceAll(bool pred, int numPoints) {
   return ((b >> seg) & full) == full;
 }
 
-// element i of an array with a uniform base, i * sizeof(T) below 2^32
-template <typename T>
-__device__ inline T& lane(T* base, unsigned i) {
+// element i of an array with a uniform base; I: unsigned where i * sizeof(T) stays below 2^32
+template <typename T, typename I>
+__device__ inline T& lane(T* base, I i) {
   typedef std::conditional_t<std::is_const_v<T>, const char, char> Byte;
-  return *reinterpret_cast<T*>(reinterpret_cast<Byte*>(base) + i * static_cast<unsigned>(sizeof(T)));
+  return *reinterpret_cast<T*>(reinterpret_cast<Byte*>(base) + i * static_cast<I>(sizeof(T)));
 }
 
 // how the first solve of a time point starts: from the previous slip rate, at
@@ -158,7 +158,7 @@ struct StepArgs {
   double timeWeights[kMaxOrder];
 };
 
-template <int TPF, Start S>
+template <int TPF, Start S, typename I>
 __global__ __launch_bounds__((kBlock<S>), 2) void kFriction(sdg_friction_params prm, sdg_fault_layer L, double fullUpdateTime,
                                                  StepArgs args, const double* __restrict__ resample,
                                                  sdg_friction_options opt) {
@@ -178,9 +178,9 @@ __global__ __launch_bounds__((kBlock<S>), 2) void kFriction(sdg_friction_params 
   // byte offset per lane: 64-bit addresses of the 30 arrays, live from their
   // loads to their stores, would take a register pair each
   const int64_t f0 = static_cast<int64_t>(blockIdx.x) * FPB;
-  const unsigned fl = active ? threadIdx.x / TPF : 0u;
+  const I fl = active ? threadIdx.x / TPF : 0u;
   const int p = active ? pnt : 0;
-  const unsigned k = fl * P + p;
+  const I k = fl * P + p;
   auto at = [&](auto* array) -> decltype(*array)& { return lane(array + f0 * P, k); };
   auto stress = [&](auto* array, int c) -> decltype(*array)& { return lane(array + f0 * 6 * P, (fl * 6 + c) * P + p); };
 
@@ -430,19 +430,33 @@ extern "C" int sdg_friction_evaluate(const sdg_friction_params* params, const sd
   }
   auto st = static_cast<hipStream_t>(stream);
   using friction::Start;
-  auto launch = [&](auto tpf, auto start) {
+  auto launch = [&](auto tpf, auto start, auto index) {
     constexpr int TPF = decltype(tpf)::value, BLOCK = friction::kBlock<decltype(start)::value>, FPB = BLOCK / TPF;
     const unsigned grid = static_cast<unsigned>((L.num_faces + FPB - 1) / FPB);
-    friction::kFriction<TPF, decltype(start)::value>
+    friction::kFriction<TPF, decltype(start)::value, decltype(index)>
         <<<grid, BLOCK, 0, st>>>(*params, L, full_update_time, args, resample, opt);
   };
-  auto points = [&](auto start) {
-    if (L.num_points <= 32) launch(std::integral_constant<int, 32>{}, start);
-    else launch(std::integral_constant<int, 64>{}, start);
+  auto points = [&](auto start, auto index) {
+    if (L.num_points <= 32) launch(std::integral_constant<int, 32>{}, start, index);
+    else launch(std::integral_constant<int, 64>{}, start, index);
   };
-  if (opt.mlp_params != nullptr || opt.samples != nullptr) points(std::integral_constant<Start, friction::kNetwork>{});
-  else if (opt.closed_form_start != 0) points(std::integral_constant<Start, friction::kClosedForm>{});
-  else points(std::integral_constant<Start, friction::kPlain>{});
+  // 32-bit byte offsets reach the interpolated states of a block's faces, the
+  // largest array, up to some 900,000 points (with the network's larger blocks)
+  // or 3.7 million; beyond, 64-bit ones, in the one instantiation that has every start
+  const auto narrow = [&](auto start) {
+    const int fpb = friction::kBlock<decltype(start)::value> / (L.num_points <= 32 ? 32 : 64);
+    return int64_t(fpb) * L.order * 9 * L.points * int64_t(sizeof(double)) <= int64_t(1) << 32;
+  };
+  constexpr std::integral_constant<Start, friction::kPlain> plain;
+  constexpr std::integral_constant<Start, friction::kClosedForm> closedForm;
+  constexpr std::integral_constant<Start, friction::kNetwork> network;
+  auto run = [&](auto start) {
+    if (narrow(start)) points(start, 0u);
+    else points(network, uint64_t(0));
+  };
+  if (opt.mlp_params != nullptr || opt.samples != nullptr) run(network);
+  else if (opt.closed_form_start != 0) run(closedForm);
+  else run(plain);
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;
 }

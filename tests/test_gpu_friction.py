@@ -6,9 +6,9 @@ import numpy as np
 import pytest
 
 import oracle
-from seissol_amd._capi import FrictionOptions, ptr
-from seissol_amd.friction import (FaultDriver, FrictionParameters, FrictionSolver, WarmStartTrainer, dr_quadrature,
-                                  make_fault_setup, mlp_param_count, pulse_loading, step_times)
+from seissol_amd._capi import FAULT_FIELDS, FaultLayer, FrictionOptions, ptr
+from seissol_amd.friction import (DeviceFault, FaultDriver, FrictionParameters, FrictionSolver, WarmStartTrainer,
+                                  dr_quadrature, make_fault_setup, mlp_param_count, pulse_loading, step_times)
 
 pytestmark = pytest.mark.gpu
 
@@ -242,3 +242,42 @@ def test_friction_matches_oracle_at_full_fault_size(gpu):
             faces_off = int((got != want).any(axis=1).sum())
             assert faces_off <= 10, (name, faces_off)
             assert abs(int(got.sum()) - int(want.sum())) <= 1e-5 * int(want.sum()), name
+
+
+# point strides whose offsets within a block of faces pass 2^32 bytes (the padding is never touched)
+@pytest.mark.parametrize("points", [7_400_000, 7_600_000])  # below and above the rule's line for two faces
+@pytest.mark.parametrize("closed_form", [False, True])
+def test_friction_with_a_huge_point_stride(gpu, points, closed_form):
+    import torch
+    order, faces, dt = 4, 2, 1e-3
+    setup = make_fault_setup(num_faces=faces, order=order, seed=5, length=4000.0, nucleation_radius=900.0)
+    print(f"friction points={points} closed_form_start={closed_form}", flush=True)
+    tp, tw, delta = step_times(order, dt)
+    sides = []
+    for wide in (False, True):
+        fault = DeviceFault(setup)
+        load = torch.from_numpy(pulse_loading(setup, 0.2 + tp)).cuda()
+        for side in ("plus", "minus"):
+            fault.t[f"q_interpolated_{side}"][:, :, 3] = load
+        if wide:
+            for k, small in fault.t.items():
+                if k != "imp_and_eta":
+                    fault.t[k] = torch.empty((*small.shape[:-1], points), dtype=small.dtype, device="cuda")
+                    fault.t[k][..., :setup.points] = small
+            fault.view = FaultLayer(faces, points, setup.num_points, order, 0,
+                                    *[ptr(fault.t.get(name)) for name in FAULT_FIELDS])
+        solver = FrictionSolver(setup.params, order)
+        solver.closed_form_start = closed_form
+        solver.setupLayer(fault)
+        for step in range(3):
+            solver.evaluate(step * dt, delta, tw)
+        torch.cuda.synchronize()
+        sides.append({k: v if k == "imp_and_eta" else v[..., :setup.points].clone() for k, v in fault.t.items()})
+        del fault, solver
+    for k, want in sides[0].items():
+        got = sides[1][k]
+        if want.dtype != torch.float64:
+            assert torch.equal(got, want), k
+        else:  # the same operations, compiled once more
+            assert float((got - want).abs().max()) <= 1e-12 * float(want.abs().max()), k
+    torch.cuda.empty_cache()
