@@ -121,7 +121,10 @@ __device__ inline double updateStateVariable(const PointParams& pp, double sr0, 
   const double muSS = pp.muw + (lowV - pp.muw) / sqrt(sqrt(sqrt(1.0 + r8)));
   const double psiSS = pp.a * logsinh(sr0 / V * 2, muSS / pp.a);
   const double pre = -V * (dt / pp.sl0);
-  const double rise = expm1(pre);  // e^pre = 1 + rise to an ulp of 1, which is an ulp of the sum
+  // 1 + rise is e^pre to an ulp of 1, not of itself: the term is off by up to
+  // 1e-16 |svRef|, as the stored state is (it changes by the difference from
+  // svRef) and as the friction sees it (through e^(state / a))
+  const double rise = expm1(pre);
   return psiSS * (-rise) + (1.0 + rise) * svRef;
 }
 
