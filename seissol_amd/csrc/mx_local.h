@@ -39,6 +39,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -859,12 +860,11 @@ __global__ __launch_bounds__((Waves<O, real>::THREADS), (LocalLds<O, real>::SIMD
 }
 
 template <typename real, int O>
-int localImpl(const EngineState& st, int parts, const ClusterStep* steps, int clusters, const sdg_layer* L,
-              bool writeTraces, const LtsOut* lts, hipStream_t stream) {
+int launchTiles(const EngineState& st, int parts, const ClusterStep* steps, int clusters, const sdg_layer* L,
+                const CellLayout& lay, bool writeTraces, const LtsOut* lts, hipStream_t stream) {
   Segments<O, real, 1> seg;
   const int64_t blocks = seg.fill(steps, clusters);
   if (blocks == 0) return SDG_OK;
-  const CellLayout lay = cellLayout(st, L);
   const dim3 grid(static_cast<unsigned>(blocks));
   auto launch = [&](auto partsI, auto ltsI) {
     kLocalMx<real, O, decltype(partsI)::value, decltype(ltsI)::value><<<grid, Waves<O, real>::THREADS, 0, stream>>>(
@@ -878,6 +878,24 @@ int localImpl(const EngineState& st, int parts, const ClusterStep* steps, int cl
   else if (lts != nullptr) launch(std::integral_constant<int, kPredict | kFlux>{}, std::true_type{});
   else launch(std::integral_constant<int, kPredict | kFlux>{}, std::false_type{});
   SDG_HIP_CHECK(hipGetLastError());
+  return SDG_OK;
+}
+
+template <typename real, int O>
+int localImpl(const EngineState& st, int parts, const ClusterStep* steps, int clusters, const sdg_layer* L,
+              bool writeTraces, const LtsOut* lts, hipStream_t stream) {
+  const CellLayout lay = cellLayout(st, L);
+  // a tile reaches its cells' operators by 32-bit offsets: where 16 cells are
+  // further apart than that, launches of as many cells as are not
+  const int64_t apart = std::max(lay.starStride, lay.aplusStride) * static_cast<int64_t>(sizeof(real));
+  const int64_t near = 1 + (0x7ff00000 - 324 * static_cast<int64_t>(sizeof(real))) / apart;
+  if (near >= kElems) return launchTiles<real, O>(st, parts, steps, clusters, L, lay, writeTraces, lts, stream);
+  for (int i = 0; i < clusters; ++i)
+    for (ClusterStep part = steps[i]; part.start < steps[i].end; part.start = part.end) {
+      part.end = std::min(part.start + near, steps[i].end);
+      if (const int rc = launchTiles<real, O>(st, parts, &part, 1, L, lay, writeTraces, lts, stream); rc != SDG_OK)
+        return rc;
+    }
   return SDG_OK;
 }
 

@@ -228,3 +228,40 @@ def test_a_step_is_as_accurate_as_the_split_products(gpu, arith, order, bound):
     err = float((got - want).norm() / want.norm())
     print(f"  error {err:.3e}, split products {bound:.2e}", flush=True)
     assert err <= bound
+
+
+# strides of the per-cell operators at which 16 cells are more than 2^31 bytes apart (the padding
+# between them is never touched): a ragged tile and more than one
+@pytest.mark.parametrize("arith", ["fp64", "fp32", "f16x3"])
+@pytest.mark.parametrize("n,megabytes", [(5, 640), (18, 160)])
+def test_operators_far_apart_equal_dense_ones(gpu, arith, n, megabytes):
+    import torch
+    order = 4
+    stride = megabytes * 2**20 // (8 if arith == "fp64" else 4)
+    print(f"operators {megabytes} MB apart {arith} n={n}", flush=True)
+    for part in ("ader", "local", "lts") if arith != "f16x3" else ("proxy", "lts"):
+        sides = []
+        for far in (False, True):
+            eng = Engine(order, arith)
+            eng.set_layout(0, "compact")
+            a = random_layer(eng, order, arith, n, 0, "compact", n, setup=part == "lts")
+            a["traces"] = torch.zeros((n, 4, 9, padded_face_basis(order)), dtype=a["dofs"].dtype, device="cuda")
+            v = a["view"]
+            if far:
+                for k in ("star", "aplus"):
+                    dense = a[k].reshape(n, -1)
+                    a[k] = torch.empty((n, stride), dtype=dense.dtype, device="cuda")
+                    a[k][:, :dense.shape[1]] = dense
+                v.star, v.aplus, v.star_stride, v.aplus_stride = ptr(a["star"]), ptr(a["aplus"]), stride, stride
+            if part == "proxy":
+                v.face_traces = ptr(a["traces"])
+                s = torch.cuda.current_stream().cuda_stream
+                check(lib().sdg_proxy_run(eng.handle, 1, 1, 1e-3, C.byref(v), s), "local")
+                torch.cuda.synchronize()
+            else:
+                run_local(eng, a, part, 1)
+            sides.append(a)
+        for k in ("dofs", "integrated", "derivatives", "traces"):
+            assert torch.equal(sides[0][k], sides[1][k]), (part, k)
+        del sides, a
+    torch.cuda.empty_cache()
