@@ -123,7 +123,8 @@ int launchNeighborMfma(const EngineState& e, const sdg_layer* layer, hipStream_t
 // flux from a given time integral, both fused (FP64: with face traces when the
 // layer has them), and the LTS local pass
 bool hasMx(const EngineState& e);
-int uploadMx(EngineState& s, const double* globalMatrices);
+// `own`: the generated matrices, which tell a caller's zeros from its small entries
+int uploadMx(EngineState& s, const double* globalMatrices, const double* own);
 int launchAderMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream);
 int launchLocalMx(const EngineState& e, const sdg_layer* layer, hipStream_t stream);
 int launchAderLocalMx(const EngineState& e, const double* coeffs, const sdg_layer* layer, hipStream_t stream);

@@ -21,21 +21,18 @@ using Matrix = std::function<double(int, int)>;
 
 // One row tile (16 rows) of A: fragments over k-steps [0, ksteps) in the lane
 // order of the A operand, and the range of k-steps that holds its non-zeros
-// (entries above 1e-13 of the largest of the whole matrix: the generator's
-// quadrature leaves rounding noise where the exact value is zero)
 template <typename real>
 void tileFragments(const Matrix& A, int ksteps, real* out) {
   for (int ks = 0; ks < ksteps; ++ks)
     for (int l = 0; l < 64; ++l) out[ks * 64 + l] = static_cast<real>(A(mx::fragRow<real>(l % 16), 4 * ks + l / 16));
 }
 // rows < rowEnd, columns < colEnd, in steps of `step` columns; lo < hi always (a zero tile keeps k-step 0)
-void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, double threshold, int step,
-               int* out) {
+void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, int step, int* out) {
   int lo = 1 << 20, hi = 0;
   for (const Matrix& A : As)
     for (int r = 0; r < rowEnd && r < 16; ++r)
       for (int c = 0; c < colEnd; ++c)
-        if (std::fabs(A(r, c)) > threshold) {
+        if (A(r, c) != 0.0) {
           lo = std::min(lo, c / step);
           hi = std::max(hi, c / step + 1);
         }
@@ -45,89 +42,125 @@ void tileRange(const std::vector<Matrix>& As, int rowEnd, int colEnd, double thr
 double largest(const double* p, int64_t n) {
   double m = 0.0;
   for (int64_t i = 0; i < n; ++i) m = std::max(m, std::fabs(p[i]));
-  return 1e-13 * m;
+  return m;
+}
+
+// The matrices `gm` with the rounding noise of their quadrature set to zero:
+// entries at places where the basis makes the exact value zero (there the
+// generated matrices `own` have nothing but noise, up to 3e-15 of their
+// largest entry, and nothing below 2e-6 elsewhere) that are no larger than such
+// noise.  Every other entry of a caller's matrices counts, however small.
+std::vector<double> withoutNoise(int order, const double* gm, const double* own) {
+  const auto g = globalMatrixLayout(order);
+  const int64_t B = numBasis3(order), B2 = numBasis2(order);
+  std::vector<double> out(gm, gm + g.total);
+  auto clean = [&](size_t at, int64_t n) {
+    const double exact = 1e-13 * largest(own + at, n), noise = 1e-14 * largest(gm + at, n);
+    for (size_t i = at; i < at + n; ++i)
+      if (std::fabs(own[i]) <= exact && std::fabs(gm[i]) <= noise) out[i] = 0.0;
+  };
+  clean(g.kDivMT, 3 * B * B);
+  clean(g.kDivM, 3 * B * B);
+  clean(g.fMrT, 4 * B2 * B);
+  clean(g.rDivM, 4 * B * B2);
+  clean(g.rT, 4 * B2 * B);
+  for (int h = 0; h < 3; ++h) clean(g.fP + h * B2 * B2, B2 * B2);
+  return out;
 }
 
 template <typename real, int O>
-int uploadOrder(EngineState& s, const double* gm) {
+int uploadOrder(EngineState& s, const double* gm, const double* own) {
   using G = mx::Geo<O>;
   const auto g = globalMatrixLayout(O);
   constexpr int B = G::B, B2 = G::B2, B2P = G::B2P, KS = G::KS;
   std::vector<real> frags(G::total, real(0));
   std::vector<int> ranges(G::rTotal, 0);
-  const double tolT = largest(gm + g.kDivMT, 3LL * B * B), tolV = largest(gm + g.kDivM, 3LL * B * B);
-  const double tolF = largest(gm + g.fMrT, 4LL * B * B2), tolR = largest(gm + g.rDivM, 4LL * B * B2);
+  const std::vector<double> nz = withoutNoise(O, gm, own);  // for the ranges
   // a caller's own matrices may have fuller rows: an FP32 engine has no
-  // neighbour pass here then, every other one refuses them
+  // neighbour pass here then, every other one refuses them; with entries that the
+  // lists below leave out, no engine has it
   bool sparseFP = true;
   for (int t = 0; t < G::MT; ++t) {
     std::vector<Matrix> ck, vol;
     for (int j = 0; j < 3; ++j) {
-      ck.push_back([=](int r, int c) {
-        r += 16 * t;
-        return r < B && c < B ? -gm[g.kDivMT + (j * B + r) * B + c] : 0.0;
-      });
-      vol.push_back([=](int r, int c) {
-        r += 16 * t;
-        return r < B && c < B ? gm[g.kDivM + (j * B + r) * B + c] : 0.0;
-      });
-      tileFragments<real>(ck[j], KS, frags.data() + G::ck + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
-      tileFragments<real>(vol[j], KS, frags.data() + G::vol + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
+      auto block = [=](const double* m, size_t at) {
+        return Matrix([=](int r, int c) {
+          r += 16 * t;
+          return r < B && c < B ? m[at + (j * B + r) * B + c] : 0.0;
+        });
+      };
+      const Matrix T = block(gm, g.kDivMT);
+      tileFragments<real>([&](int r, int c) { return -T(r, c); }, KS,
+                          frags.data() + G::ck + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
+      tileFragments<real>(block(gm, g.kDivM), KS, frags.data() + G::vol + (static_cast<int64_t>(t) * 3 + j) * KS * 64);
+      ck.push_back(block(nz.data(), g.kDivMT));
+      vol.push_back(block(nz.data(), g.kDivM));
     }
     // derivative d has basis3(O - d) rows of basis3(O - d + 1) columns
     for (int d = 1; d < O; ++d)
-      tileRange(ck, mx::basis3(O - d) - 16 * t, mx::basis3(O - d + 1), tolT, 4,
+      tileRange(ck, mx::basis3(O - d) - 16 * t, mx::basis3(O - d + 1), 4,
                 ranges.data() + G::rCk + 2 * ((d - 1) * G::MT + t));
-    tileRange(vol, 16, B, tolV, 4, ranges.data() + G::rVol + 2 * t);
+    tileRange(vol, 16, B, 4, ranges.data() + G::rVol + 2 * t);
     for (int f = 0; f < 4; ++f) {
-      const Matrix R = [=](int r, int c) {
-        r += 16 * t;
-        return r < B && c < B2 ? gm[g.rDivM + (f * B + r) * B2 + c] : 0.0;
+      auto block = [=](const double* m) {
+        return Matrix([=](int r, int c) {
+          r += 16 * t;
+          return r < B && c < B2 ? m[g.rDivM + (f * B + r) * B2 + c] : 0.0;
+        });
       };
+      const Matrix R = block(gm);
       tileFragments<real>([&](int r, int c) { return c < B2 ? R(r, c) * gm[g.mass2 + c] : 0.0; }, G::KSF,
                           frags.data() + G::flux + (static_cast<int64_t>(t) * 4 + f) * G::KSF * 64);
       tileFragments<real>(R, G::KSF, frags.data() + G::rdm + (static_cast<int64_t>(t) * 4 + f) * G::KSF * 64);
-      tileRange({R}, 16, B2, tolR, 4, ranges.data() + G::rFlux + 2 * (t * 4 + f));
+      tileRange({block(nz.data())}, 16, B2, 4, ranges.data() + G::rFlux + 2 * (t * 4 + f));
     }
   }
   for (int t = 0; t < G::MTF; ++t) {
     // k-steps from the last columns to the first (see gemm, mx_local.h)
-    const Matrix F = [=](int r, int c) {
-      c = 4 * (KS - 1 - c / 4) + c % 4;
-      const int f = G::traceFace(t, r / 4), m = G::traceRow(t, r / 4) + r % 4;
-      return m < B2 && c < B ? gm[g.fMrT + (f * B2 + m) * B + c] : 0.0;
+    auto block = [=](const double* matrices) {
+      return Matrix([=](int r, int c) {
+        c = 4 * (KS - 1 - c / 4) + c % 4;
+        const int f = G::traceFace(t, r / 4), m = G::traceRow(t, r / 4) + r % 4;
+        return m < B2 && c < B ? matrices[g.fMrT + (f * B2 + m) * B + c] : 0.0;
+      });
     };
+    const Matrix F = block(gm);
     tileFragments<real>(
         [&](int r, int c) {
           const int m = G::traceRow(t, r / 4) + r % 4;
           return m < B2 ? F(r, c) / gm[g.mass2 + m] : 0.0;
         },
         KS, frags.data() + G::trace + static_cast<int64_t>(t) * KS * 64);
-    tileRange({F}, 16, G::KB, tolF, 4, ranges.data() + G::rTrace + 2 * t);
+    tileRange({block(nz.data())}, 16, G::KB, 4, ranges.data() + G::rTrace + 2 * t);
   }
   // rT_j of the neighbour pass: lane l of block k holds columns 8 k + 2 (l / 16) + {0, 1}
-  const double tolU = largest(gm + g.rT, 4LL * B2 * B);
   for (int j = 0; j < 4; ++j)
     for (int r = 0; r < G::RT; ++r) {
-      const Matrix U = [=](int i, int c) {
-        i += 16 * r;
-        return i < B2 && c < B ? gm[g.rT + (j * B2 + i) * B + c] : 0.0;
+      auto block = [=](const double* m) {
+        return Matrix([=](int i, int c) {
+          i += 16 * r;
+          return i < B2 && c < B ? m[g.rT + (j * B2 + i) * B + c] : 0.0;
+        });
       };
+      const Matrix U = block(gm);
       real* const out = frags.data() + G::rt + (static_cast<int64_t>(j) * G::RT + r) * G::KB8 * 128;
       for (int k = 0; k < G::KB8; ++k)
         for (int l = 0; l < 64; ++l)
           for (int i = 0; i < 2; ++i)
             out[(k * 64 + l) * 2 + i] = static_cast<real>(U(mx::fragRow<real>(l % 16), 8 * k + 2 * (l / 16) + i));
-      tileRange({U}, 16, B, tolU, 8, ranges.data() + G::rRt + 2 * (j * G::RT + r));
+      tileRange({block(nz.data())}, 16, B, 8, ranges.data() + G::rRt + 2 * (j * G::RT + r));
     }
   // fP_h as rows of at most O non-zeros, padded with zeros
   for (int h = 0; h < 3; ++h) {
-    const double tolP = largest(gm + g.fP + h * B2 * B2, int64_t(B2) * B2);
+    const double tolP = 1e-13 * largest(gm + g.fP + h * B2 * B2, int64_t(B2) * B2);
     for (int r = 0; r < B2; ++r) {
       int cnt = 0;
       for (int c = 0; c < B2; ++c) {
         const double v = gm[g.fP + (h * B2 + r) * B2 + c];
-        if (std::fabs(v) <= tolP) continue;
+        if (std::fabs(v) <= tolP) {
+          if (nz[g.fP + (h * B2 + r) * B2 + c] != 0.0) sparseFP = false;
+          continue;
+        }
         if (cnt == O) {
           if (sizeof(real) == 8 || matrixCore(s.arithmetic)) {
             setError("face permutation matrix with more than `order` non-zeros in a row");
@@ -165,14 +198,14 @@ int orders(const EngineState& e, F&& f) {
 
 }  // namespace
 
-int uploadMx(EngineState& s, const double* gm) {
+int uploadMx(EngineState& s, const double* gm, const double* own) {
   const bool dbl = s.arithmetic == SDG_FP64;
   switch (s.order) {
-    case 3: return dbl ? uploadOrder<double, 3>(s, gm) : uploadOrder<float, 3>(s, gm);
-    case 4: return dbl ? uploadOrder<double, 4>(s, gm) : uploadOrder<float, 4>(s, gm);
-    case 5: return dbl ? uploadOrder<double, 5>(s, gm) : uploadOrder<float, 5>(s, gm);
-    case 6: return dbl ? uploadOrder<double, 6>(s, gm) : uploadOrder<float, 6>(s, gm);
-    case 7: return dbl ? uploadOrder<double, 7>(s, gm) : uploadOrder<float, 7>(s, gm);
+    case 3: return dbl ? uploadOrder<double, 3>(s, gm, own) : uploadOrder<float, 3>(s, gm, own);
+    case 4: return dbl ? uploadOrder<double, 4>(s, gm, own) : uploadOrder<float, 4>(s, gm, own);
+    case 5: return dbl ? uploadOrder<double, 5>(s, gm, own) : uploadOrder<float, 5>(s, gm, own);
+    case 6: return dbl ? uploadOrder<double, 6>(s, gm, own) : uploadOrder<float, 6>(s, gm, own);
+    case 7: return dbl ? uploadOrder<double, 7>(s, gm, own) : uploadOrder<float, 7>(s, gm, own);
     default: return SDG_OK;  // orders 2 and 8: the VALU kernels
   }
 }

@@ -483,7 +483,7 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic) {
   generateGlobalMatrices(order, gm.data());
   int rc = uploadMatrices(e->s, gm.data());
   if (rc == SDG_OK && matrixCore(arithmetic)) rc = uploadMfma(e->s, gm.data());
-  if (rc == SDG_OK) rc = uploadMx(e->s, gm.data());
+  if (rc == SDG_OK) rc = uploadMx(e->s, gm.data(), gm.data());
   if (rc != SDG_OK) {
     if (e->s.matrices) (void)hipFree(e->s.matrices);
     if (e->s.mfmaFrags) (void)hipFree(e->s.mfmaFrags);
@@ -501,7 +501,9 @@ int sdg_engine_set_global_matrices(sdg_engine* engine, const double* host_matric
   if (engine == nullptr || host_matrices == nullptr) { setError("invalid arguments"); return SDG_ERR_INVALID; }
   int rc = uploadMatrices(engine->s, host_matrices);
   if (rc == SDG_OK && matrixCore(engine->s.arithmetic)) rc = uploadMfma(engine->s, host_matrices);
-  if (rc == SDG_OK) rc = uploadMx(engine->s, host_matrices);
+  std::vector<double> own(globalMatrixLayout(engine->s.order).total);
+  generateGlobalMatrices(engine->s.order, own.data());
+  if (rc == SDG_OK) rc = uploadMx(engine->s, host_matrices, own.data());
   return rc;
 }
 
