@@ -270,7 +270,9 @@ int sdg_proxy_run_static(sdg_engine* engine, int kernel_id, int steps, double dt
 
 /* Work of one element-update of a proxy kernel (PerformanceEstimate,
  * src/Monitoring/Metric.h:16-50, summed by src/Proxy/Runner.cpp:120-150),
- * per element: non-zero and hardware FLOP, bytes (DOF blocks and
+ * per element: non-zero and hardware FLOP (dense contractions, times three
+ * where the kernel runs split bf16 products; SDG_BF16X6 counts the six
+ * products it is named after, its kernels run one), bytes (DOF blocks and
  * per-element operators moved once) and kernel bytes (what the kernels of
  * this arithmetic move, face traces included).  The DR kernels 5-7 (every
  * arithmetic; the DR parts in the engine's real type) count the proxy's

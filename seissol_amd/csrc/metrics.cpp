@@ -5,16 +5,20 @@
 // per non-zero of the sparse operand, from the sparsity of this library's
 // generated global matrices (entries below 1e-13 of the matrix maximum count
 // as zero) and the 24 non-zeros of an elastic star matrix.  Hardware FLOP:
-// the same contractions with dense operands, times the number of bf16
-// products of the split forms.  Bytes: DOF blocks and per-element operators
-// each moved once (global matrices excluded); kernel bytes count the face
-// traces that the matrix-core forms exchange instead of I.
+// the same contractions with dense operands, times three where the kernel runs
+// split bf16 products (bf16x3, fused local pass at orders 6 and 7 and neighbour
+// pass at ORDER 6; every other pass runs one product in the real type).
+// bf16x6 keeps the count of the six products it is named after.  Bytes: DOF
+// blocks and per-element operators each moved once (global matrices
+// excluded); kernel bytes count the face traces that the matrix-core forms
+// exchange instead of I.
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
 #include "engine.h"
 #include "global_matrices.h"
+#include "mfma_common.h"
 
 namespace sdg {
 namespace {
@@ -129,15 +133,19 @@ extern "C" int sdg_performance_estimate(int order, int arithmetic, int kernel_id
   const Work w = elementWork(order, gm);
   const int B = numBasis3(order), B2 = numBasis2(order);
   const double s = arithmetic == SDG_FP64 ? 8.0 : 4.0;
-  const double products = arithmetic == SDG_BF16X6 ? 6.0 : (matrixCore(arithmetic) ? 3.0 : 1.0);
+  // products of the fused local pass and of the neighbour pass
+  const bool split = mfma::splitProducts(arithmetic, order);
+  const double nominal = arithmetic == SDG_BF16X6 ? 6.0 : 1.0;
+  const double localProducts = split ? 3.0 : nominal;
+  const double neighborProducts = split && order == mfma::kSplitNeighborOrder ? 3.0 : nominal;
   const bool traces = matrixCore(arithmetic);
   const int B2P = (B2 + 3) / 4 * 4;  // padded face rows of the matrix-core traces
   const double q = 9.0 * B, traceBytes = 4.0 * 9 * B2P * 4;
   Counts c;
   double bytes = 0, kernelBytes = 0;
-  auto add = [&](const Counts& x) {
+  auto add = [&](const Counts& x, double products = 1.0) {
     c.nz += x.nz;
-    c.dense += x.dense;
+    c.dense += x.dense * products;
   };
   if (kernel_id >= 5) {
     // the proxy's DR layer: all four faces of every cell are DR faces and
@@ -180,12 +188,14 @@ extern "C" int sdg_performance_estimate(int order, int arithmetic, int kernel_id
   const bool ader = kernel_id == 0 || kernel_id == 1 || kernel_id == 3;
   const bool local = kernel_id == 0 || kernel_id == 1 || kernel_id == 4;
   const bool neigh = kernel_id == 0 || kernel_id == 2;
-  if (ader) add(w.ader);
+  // the predictor and the local integral alone (3, 4) run one product in every form
+  const double products = kernel_id >= 3 ? 1.0 : localProducts;
+  if (ader) add(w.ader, products);
   if (local) {
-    add(w.volume);
-    add(w.localFlux);
+    add(w.volume, products);
+    add(w.localFlux, products);
   }
-  if (neigh) add(w.neighborFlux);
+  if (neigh) add(w.neighborFlux, neighborProducts);
   // kernel ids: 0 all, 1 local (ader + integral), 2 neigh, 3 ader, 4 localwoader
   if (kernel_id == 3) bytes = (2 * q + 3 * kStarNonZeros) * s;                    // Q in, I out, star
   if (kernel_id == 1 || kernel_id == 0) bytes += (3 * q + 3 * kStarNonZeros + 4 * 81) * s;  // Q in/out, I out
@@ -197,7 +207,7 @@ extern "C" int sdg_performance_estimate(int order, int arithmetic, int kernel_id
   if (traces && (kernel_id == 0 || kernel_id == 1)) kernelBytes += traceBytes - q * s;
   if (traces && neigh) kernelBytes += traceBytes - q * s;
   out->nonzero_flop = c.nz;
-  out->hardware_flop = c.dense * products;
+  out->hardware_flop = c.dense;
   out->bytes = bytes;
   out->kernel_bytes = kernelBytes;
   return SDG_OK;

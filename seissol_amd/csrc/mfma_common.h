@@ -90,7 +90,8 @@ inline bool vectorAccess(const CellLayout& lay, const void* dofs, const void* in
 // 171 -> 121, ORDER 4 280 -> 189, ORDER 5 448 -> 326; bf16x6 ORDER 6 60k 784 ->
 // 529, ORDER 7 120k 2225 -> 1914; bf16x3 60k ORDER 5 403 -> 326, but ORDER 6
 // 200k 1335 -> 1392 and ORDER 7 120k 1677 -> 1914.
-inline bool splitProducts(const EngineState& e) { return e.arithmetic == SDG_BF16X3 && e.order >= 6; }
+constexpr bool splitProducts(int arithmetic, int order) { return arithmetic == SDG_BF16X3 && order >= 6; }
+inline bool splitProducts(const EngineState& e) { return splitProducts(e.arithmetic, e.order); }
 // Their neighbour pass: at ORDER 7 the FP32 pass from the traces is faster (60k
 // cells 921 -> 862 us a step), at ORDER 6 it is not (459 -> 478).
 constexpr int kSplitNeighborOrder = 6;

@@ -77,6 +77,20 @@ def test_work_estimates_match_the_reference_sparsity():
     assert _capi.lib().sdg_performance_estimate(9, 0, 0, ctypes.byref(_capi.WorkEstimate())) != 0
 
 
+def test_hardware_flop_count_the_products_that_run():
+    # one product per contraction everywhere but in the split bf16 products: three in bf16x3's fused
+    # local pass at orders 6 and 7 and in its neighbour pass at ORDER 6
+    for order in range(3, 8):
+        one = {k: _estimate(order, _capi.SDG_FP32, k).hardware_flop for k in range(5)}
+        assert one[0] == one[1] + one[2]
+        for k in range(5):
+            assert _estimate(order, _capi.SDG_FP64, k).hardware_flop == one[k]
+            assert _estimate(order, _capi.SDG_F16X3, k).hardware_flop == one[k]
+        local, neigh = (3 if order >= 6 else 1) * one[1], (3 if order == 6 else 1) * one[2]
+        assert [_estimate(order, _capi.SDG_BF16X3, k).hardware_flop for k in range(5)] == [
+            local + neigh, local, neigh, one[3], one[4]]
+
+
 def test_dr_work_estimates_known_answers():
     # the proxy's DR layer: 4 DR faces per cell, all cell faces DR
     order, B, NP = 6, 56, 49
