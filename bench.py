@@ -215,6 +215,19 @@ def friction_bench(args) -> dict:
     }
 
 
+def lts_launches(run, lts, args) -> int:
+    """Launches of one macro step: the clusters on a matrix-core pass that start (local) or end
+    (neighbour) a step at the same time share one, except those on split products."""
+    mc, sizes, total = run.matrix_core(), np.diff(lts.cluster_start), 0
+    shared = {"local": not (args.lts_form == "bf16x3" and args.lts_order >= 6), "neigh": True}
+    for k in range(1 << (lts.num_clusters - 1)):
+        for kind, t in (("local", k), ("neigh", k + 1)):
+            at = [c for c in range(lts.num_clusters) if t % (1 << c) == 0 and sizes[c] > 0]
+            together = [c for c in at if shared[kind] and mc[c][kind]]
+            total += len(at) - len(together) + bool(together)
+    return total
+
+
 def lts_bench(args) -> dict:
     """Rate-2 local time stepping (clusters 60/25/10/5 %, dt ratios 1:2:4:8),
     macro steps enqueued eagerly and replayed from a captured hipGraph."""
@@ -268,16 +281,17 @@ def lts_bench(args) -> dict:
         "value": out["graph"]["element_updates_per_s"],
         "graph_vs_eager": out["eager_autotuned"]["ms_per_macro_step"] / out["graph"]["ms_per_macro_step"], "unit": "element-updates/s", "higher_is_better": True,
         "modes": out, "tiles": {str(c): t for c, t in run.tiles().items()},
-        "tile_variants": ("VALU 0-3: bit 0 one more basis row per lane, bit 1 two waves per block; neighbour "
-                          "4: one element per 16-lane row; matrix-core engines, local kernel: 0 = matrix-core "
-                          "pass, 1 + v = FP32 VALU variant v"),
-        "dtype": {"fp64": "f64", "fp32": "f32"}.get(args.lts_form,
-                                                   f"f32 ({args.lts_form} matrix-core local pass, FP32 neighbour)"),
+        "matrix_core": {str(c): t for c, t in run.matrix_core().items()},
+        "tile_variants": ("where `matrix_core` is false: VALU 0-3: bit 0 one more basis row per lane, bit 1 two "
+                          "waves per block; neighbour 4: one element per 16-lane row; local kernel of the "
+                          "matrix-core forms and FP64 at orders 3-7: 0 = matrix-core pass, 1 + v = VALU variant v"),
+        "dtype": "f64" if args.lts_form == "fp64" else (
+            "f32 (2-plane split-bf16 local pass)" if args.lts_form == "bf16x3" and args.lts_order >= 6 else "f32"),
         "config": {"workload": f"ORDER {args.lts_order} elastic, {lts.setup.n} tetrahedra (periodic box "
                                f"{lts.setup.dims}), clusters {np.diff(lts.cluster_start).tolist()} with dt0 * 2^c, "
                                f"{args.lts_steps} macro steps",
                    "cluster_sizes": np.diff(lts.cluster_start).tolist(), "dt0": lts.dt0,
-                   "updates_per_macro_step": upd, "launches_per_macro_step": 2 << (C_ - 1),
+                   "updates_per_macro_step": upd, "launches_per_macro_step": lts_launches(run, lts, args),
                    "updates_saved_vs_global_dt0": gts_updates / upd, "finite": finite},
         "data": "synthetic",
     }

@@ -105,8 +105,8 @@ int sdg_engine_create(sdg_engine** engine, int order, int arithmetic);
 int sdg_engine_set_global_matrices(sdg_engine* engine, const double* host_matrices);
 /* Kernel family of an engine (no reference counterpart: the reference picks
  * its generated kernels at build time).  SDG_KERNELS_AUTO (default): the
- * matrix-core passes where the engine has them (the split-16-bit forms; the
- * FP64 engine's fused ader + local pass at orders 3-7 on v_mfma_f64_16x16x4);
+ * matrix-core passes at orders 3-7 (predictor, local and neighbour integral,
+ * fused and LTS passes of every arithmetic, in the real type or on split bf16);
  * SDG_KERNELS_VALU: the FP64/FP32 VALU kernels only (FP64 and FP32 engines). */
 #define SDG_KERNELS_AUTO 0
 #define SDG_KERNELS_VALU 1
@@ -197,10 +197,11 @@ int sdg_compute_batched_ader_local(sdg_engine* engine, const double* coeffs, dou
                                    const sdg_layer* layer, void* stream);
 
 /* ---------------------------------------------------------------------- */
-/* Local time stepping (rate 2).  Every engine: the matrix-core engines    */
-/* (orders 3-7) run the local pass on the matrix cores; the neighbour pass  */
-/* runs on the VALU kernel of the engine's real type (FP32 for the split   */
-/* forms, FP64 for the FP64 engine).                                        */
+/* Local time stepping (rate 2).  Every engine; at orders 3-7 (kernel      */
+/* family AUTO) both passes run on the matrix cores (the neighbour pass in  */
+/* the engine's real type: FP32 for the split forms), elsewhere on the VALU  */
+/* kernels.  Clusters that step at the same time share the matrix-core      */
+/* passes' launches.                                                        */
 /* ---------------------------------------------------------------------- */
 /* deriveLtsSetups (src/Initializer/InitProcedure/Internal/LtsSetup.cpp:97-330,
  * getLtsSetup + normalizeLtsSetup), host: LTS bits of every cell from the
@@ -239,14 +240,22 @@ int sdg_lts_graph_advance(sdg_lts* lts, int macro_steps, void* stream);
  * cluster's data, keeps the fastest and restores the cells' state.
  * Allocates temporaries for the saved state; synchronises `stream`. */
 int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream);
-/* Tile variant in use for `cluster` and kernel 0 (local) / 1 (neighbour).
+/* VALU variant of `cluster` and kernel 0 (local) / 1 (neighbour).
  * VALU variants 0-3: bit 0 = one more basis row per lane, bit 1 = two waves
  * per block; neighbour variant 4 = one element per 16-lane row (the default
  * of the FP32 neighbour pass at orders 3-6 and of the FP64 one at orders
- * 4-5, else 0).  Matrix-core engines,
- * local kernel: 0 = the matrix-core pass, 1 + v = the FP32 VALU variant v. */
+ * 4-5, else 0).  Local kernel of the matrix-core forms and of the FP64 engine
+ * at orders 3-7 (kernel family AUTO): 0 = the matrix-core pass, 1 + v = the VALU
+ * variant v (FP32 for the matrix-core forms).  The FP32 engine's local pass and
+ * every engine's neighbour pass have a matrix-core pass beside the numbers at
+ * orders 3-7 (AUTO), which runs until sdg_lts_set_tile_variant or the
+ * autotuner chooses a VALU variant (the variant reported meanwhile is the
+ * default VALU one).  sdg_lts_matrix_core: 1 where the matrix-core pass runs,
+ * else 0; sdg_lts_use_matrix_core chooses it again. */
 int sdg_lts_tile_variant(const sdg_lts* lts, int cluster, int kernel);
 int sdg_lts_set_tile_variant(sdg_lts* lts, int cluster, int kernel, int variant);
+int sdg_lts_matrix_core(const sdg_lts* lts, int cluster, int kernel);
+int sdg_lts_use_matrix_core(sdg_lts* lts, int cluster, int kernel);
 int sdg_lts_destroy(sdg_lts* lts);
 
 /* Proxy kernel selection (src/Proxy/Common.cpp:22-41, KernelDevice.cpp:144-165):

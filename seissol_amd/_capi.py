@@ -173,6 +173,8 @@ SIGNATURES = {
     "sdg_lts_autotune": (I32, [P, I32, P]),
     "sdg_lts_tile_variant": (I32, [P, I32, I32]),
     "sdg_lts_set_tile_variant": (I32, [P, I32, I32, I32]),
+    "sdg_lts_matrix_core": (I32, [P, I32, I32]),
+    "sdg_lts_use_matrix_core": (I32, [P, I32, I32]),
 }
 
 _LIB = None

@@ -109,9 +109,6 @@ constexpr int kNeighborRowsVariant = kTileVariants;
 constexpr int kNeighborVariants = kTileVariants + 1;
 int launchLocalIntegration(const EngineState& e, const double* coeffs, const sdg_layer* layer, int resetBuffers,
                            hipStream_t stream, int variant = 0);
-// the neighbour pass's variant before any tuning, which is the matrix-core
-// pass where the engine has it
-int defaultNeighborVariant(const EngineState& e);
 int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs, const double* subtimeCoeffs,
                                  const sdg_layer* layer, hipStream_t stream, int variant = 0);
 // kernels_mfma.hip

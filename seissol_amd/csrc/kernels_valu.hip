@@ -1312,8 +1312,6 @@ int launchLocalIntegration(const EngineState& e, const double* coeffs, const sdg
 }
 int launchNeighboringIntegration(const EngineState& e, const double* timeCoeffs, const double* subtimeCoeffs,
                                  const sdg_layer* layer, hipStream_t stream, int variant) {
-  if (variant == defaultNeighborVariant(e) && hasNeighborMx(e))
-    return launchNeighborMx(e, layer, timeCoeffs, subtimeCoeffs, stream);
   return dispatch<LtsNeighborOp>(e, layer, stream, timeCoeffs, subtimeCoeffs, variant);
 }
 int launchLocal(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {

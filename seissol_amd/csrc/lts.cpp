@@ -29,16 +29,6 @@
 
 using namespace sdg;
 
-// Neighbour-pass variant before any tuning: numbered as the VALU kernel that
-// was measured faster on the vector ALUs (one element per 16-lane row for the
-// FP32 kernel at orders 3-6 and the FP64 kernel at orders 4-5, else tile 0);
-// at orders 3-7 that number runs the matrix-core pass, faster than any of them.
-int sdg::defaultNeighborVariant(const EngineState& e) {
-  const bool fp64 = e.arithmetic == SDG_FP64;
-  const bool rows = fp64 ? (e.order >= 4 && e.order <= 5) : (e.order >= 3 && e.order <= 6);
-  return rows ? kNeighborRowsVariant : 0;
-}
-
 namespace {
 
 constexpr uint16_t kNHD0 = 1u << 0;  // neighbour on face 0 provides derivatives
@@ -65,25 +55,51 @@ bool ltsLayerOk(const sdg_layer* L, bool neighbors, const char* who) {
   return true;
 }
 
-// Local-pass variants: the FP64/FP32 engines have the kTileVariants VALU tile
-// shapes; a matrix-core engine has its matrix-core pass (variant 0) and the
-// FP32 VALU shapes after it.  The neighbour pass is the VALU kernel of the
-// engine's real type (FP32 for the matrix-core engines) with kTileVariants
-// shapes, then the one-element-per-row kernel (kNeighborRowsVariant); its default
-// variant is the matrix-core pass where the engine has it.
-// The FP64 engine (orders 3-7, kernel family AUTO) likewise has its FP64
-// matrix-core pass as variant 0.
-bool matrixCoreLocal(const EngineState& e) { return matrixCore(e.arithmetic) || (e.arithmetic == SDG_FP64 && hasMx(e)); }
-int localVariants(const EngineState& e) { return matrixCoreLocal(e) ? 1 + kTileVariants : kTileVariants; }
+// Kernels of the two passes.  A variant is a number of the public interface:
+// the kTileVariants VALU tile shapes (FP32 ones for the matrix-core forms), for
+// the neighbour pass the one-element-per-row kernel after them
+// (kNeighborRowsVariant), and for the local pass of the matrix-core forms and
+// the FP64 engine (orders 3-7, kernel family AUTO) the matrix-core pass before
+// them (variant 0).  The FP32 engine's local pass and every engine's neighbour
+// pass at orders 3-7 have their matrix-core pass beside the numbers
+// (Tile::matrixCore); it is faster than any VALU variant in all but the
+// smallest clusters and is what runs untuned.
+bool numberedLocal(const EngineState& e) { return matrixCore(e.arithmetic) || (e.arithmetic == SDG_FP64 && hasMx(e)); }
+int localVariants(const EngineState& e) { return numberedLocal(e) ? 1 + kTileVariants : kTileVariants; }
 
-int runLocal(const EngineState& e, const double* coeffs, const sdg_layer* own, int reset, hipStream_t s, int v) {
-  if (!matrixCoreLocal(e))
-    return v == 0 && hasMx(e) ? launchLocalIntegrationMx(e, coeffs, own, reset, s)
-                              : launchLocalIntegration(e, coeffs, own, reset, s, v);
-  if (v == 0)
-    return matrixCore(e.arithmetic) ? launchLocalIntegrationMfma(e, coeffs, own, reset, s)
-                                    : launchLocalIntegrationMx(e, coeffs, own, reset, s);
-  return launchLocalIntegration(e, coeffs, own, reset, s, v - 1);
+// Default VALU variant of the neighbour pass: one element per 16-lane row for
+// the FP32 kernel at orders 3-6 and the FP64 kernel at orders 4-5 (where the
+// autotuner picked it on every cluster), else tile 0.
+int defaultNeighborVariant(const EngineState& e) {
+  const bool fp64 = e.arithmetic == SDG_FP64;
+  const bool rows = fp64 ? (e.order >= 4 && e.order <= 5) : (e.order >= 3 && e.order <= 6);
+  return rows ? kNeighborRowsVariant : 0;
+}
+
+struct Tile {
+  int variant = 0;
+  bool matrixCore = false;  // beside the variants: the matrix-core pass, where the engine has it
+};
+Tile defaultTile(const EngineState& e, int kernel) {
+  if (kernel == 0) return {0, !numberedLocal(e)};
+  return {defaultNeighborVariant(e), true};
+}
+bool runsMx(const EngineState& e, int kernel, const Tile& t) {
+  if (kernel == 1) return t.matrixCore && hasNeighborMx(e);
+  return numberedLocal(e) ? t.variant == 0 : t.matrixCore && hasMx(e);
+}
+
+int runLocal(const EngineState& e, const double* coeffs, const sdg_layer* own, int reset, hipStream_t s,
+             const Tile& t) {
+  if (!runsMx(e, 0, t)) return launchLocalIntegration(e, coeffs, own, reset, s, t.variant - (numberedLocal(e) ? 1 : 0));
+  return matrixCore(e.arithmetic) ? launchLocalIntegrationMfma(e, coeffs, own, reset, s)
+                                  : launchLocalIntegrationMx(e, coeffs, own, reset, s);
+}
+
+int runNeighbor(const EngineState& e, const double* coeffs, const double* sub, const sdg_layer* nbv, hipStream_t s,
+                const Tile& t) {
+  return runsMx(e, 1, t) ? launchNeighborMx(e, nbv, coeffs, sub, s)
+                         : launchNeighboringIntegration(e, coeffs, sub, nbv, s, t.variant);
 }
 
 bool ltsArithmetic(const sdg_engine* e, const char* who) {
@@ -149,7 +165,8 @@ extern "C" int sdg_compute_local_integration(sdg_engine* engine, const double* c
       !ltsLayerOk(layer, false, "sdg_compute_local_integration") ||
       !layerStridesOk(engine->s, layer, "sdg_compute_local_integration"))
     return SDG_ERR_INVALID;
-  return runLocal(engine->s, coeffs, layer, reset_buffers != 0, static_cast<hipStream_t>(stream), 0);
+  return runLocal(engine->s, coeffs, layer, reset_buffers != 0, static_cast<hipStream_t>(stream),
+                  defaultTile(engine->s, 0));
 }
 
 extern "C" int sdg_compute_neighboring_integration(sdg_engine* engine, const double* time_coeffs,
@@ -163,8 +180,8 @@ extern "C" int sdg_compute_neighboring_integration(sdg_engine* engine, const dou
       !ltsLayerOk(layer, true, "sdg_compute_neighboring_integration") ||
       !layerStridesOk(engine->s, layer, "sdg_compute_neighboring_integration"))
     return SDG_ERR_INVALID;
-  return launchNeighboringIntegration(engine->s, time_coeffs, subtime_coeffs, layer,
-                                      static_cast<hipStream_t>(stream), defaultNeighborVariant(engine->s));
+  return runNeighbor(engine->s, time_coeffs, subtime_coeffs, layer, static_cast<hipStream_t>(stream),
+                     defaultTile(engine->s, 1));
 }
 
 struct sdg_lts {
@@ -172,7 +189,7 @@ struct sdg_lts {
   sdg_layer layer{};
   std::vector<int64_t> start;
   double dt0 = 0.0;
-  std::vector<int> tileLocal, tileNeighbor;  // tile variant per cluster
+  std::vector<Tile> tile[2];  // per kernel (local, neighbour) and cluster
   hipStream_t captureStream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -208,14 +225,13 @@ sdg_layer clusterView(const sdg_lts& L, int c, bool neighborPass) {
   return v;
 }
 
-// whether the default variant of a pass takes several clusters in one launch
+// whether the matrix-core local pass takes several clusters in one launch (the neighbour pass does)
 bool mergedLocal(const EngineState& e) { return hasMx(e) && !mfma::splitProducts(e); }
-bool mergedNeighbor(const EngineState& e) { return hasNeighborMx(e); }
 
 // The passes of clusters 0 .. top that start (local) or end (neighbour) a step
 // at the same time.  They are independent: a local pass touches its own cells
 // only, a neighbour pass reads buffers and derivatives and writes its own DOFs.
-// So the clusters with the default variant share a launch: a small cluster
+// So the clusters on the matrix-core pass share a launch: a small cluster
 // takes 20 us for one tile's chain whatever its size (four clusters of 9k cells
 // in FP64 at ORDER 4, a macro step of 30 launches -> 16: 801 -> 614 us).
 int localPasses(const sdg_lts& L, int top, int64_t k, hipStream_t s) {
@@ -228,9 +244,9 @@ int localPasses(const sdg_lts& L, int top, int64_t k, hipStream_t s) {
     if (own.num_elements == 0) continue;
     const int reset = ((k >> c) & 1) == 0;
     sdg_monomial_integrate(e.order, 0.0, L.dt0 * static_cast<double>(int64_t(1) << c), coeffs[c]);
-    if (mergedLocal(e) && L.tileLocal[c] == 0) {
+    if (mergedLocal(e) && runsMx(e, 0, L.tile[0][c])) {
       steps[merged++] = {L.start[c], L.start[c + 1], coeffs[c], nullptr, reset};
-    } else if (const int rc = runLocal(e, coeffs[c], &own, reset, s, L.tileLocal[c]); rc != SDG_OK) {
+    } else if (const int rc = runLocal(e, coeffs[c], &own, reset, s, L.tile[0][c]); rc != SDG_OK) {
       return rc;
     }
   }
@@ -252,10 +268,9 @@ int neighborPasses(const sdg_lts& L, int top, int64_t k, hipStream_t s) {
     // sub-interval of the slower cluster's step
     const double t = c + 1 < C ? L.dt0 * static_cast<double>(begin - ((begin >> (c + 1)) << (c + 1))) : 0.0;
     sdg_monomial_integrate(e.order, t, t + dtc, sub[c]);
-    if (mergedNeighbor(e) && L.tileNeighbor[c] == defaultNeighborVariant(e)) {
+    if (runsMx(e, 1, L.tile[1][c])) {
       steps[merged++] = {L.start[c], L.start[c + 1], coeffs[c], sub[c], 1};
-    } else if (const int rc = launchNeighboringIntegration(e, coeffs[c], sub[c], &nbv, s, L.tileNeighbor[c]);
-               rc != SDG_OK) {
+    } else if (const int rc = runNeighbor(e, coeffs[c], sub[c], &nbv, s, L.tile[1][c]); rc != SDG_OK) {
       return rc;
     }
   }
@@ -304,11 +319,26 @@ extern "C" int sdg_lts_create(sdg_lts** out, sdg_engine* engine, const sdg_layer
   L->layer = *layer;
   L->start.assign(cluster_start, cluster_start + num_clusters + 1);
   L->dt0 = dt0;
-  L->tileLocal.assign(num_clusters, 0);
-  L->tileNeighbor.assign(num_clusters, defaultNeighborVariant(engine->s));
+  for (int k = 0; k < 2; ++k) L->tile[k].assign(num_clusters, defaultTile(engine->s, k));
   *out = L;
   return SDG_OK;
 }
+
+namespace {
+bool tileArguments(const sdg_lts* lts, int cluster, int kernel, const char* who) {
+  if (lts != nullptr && cluster >= 0 && cluster < static_cast<int>(lts->tile[0].size()) && (kernel == 0 || kernel == 1))
+    return true;
+  setError(std::string(who) + ": invalid arguments");
+  return false;
+}
+// a captured macro step used the previous tiles
+void dropGraph(sdg_lts* lts) {
+  if (lts->exec != nullptr) (void)hipGraphExecDestroy(lts->exec);
+  if (lts->graph != nullptr) (void)hipGraphDestroy(lts->graph);
+  lts->exec = nullptr;
+  lts->graph = nullptr;
+}
+}  // namespace
 
 // Tile autotuner: times every tile variant of both kernels on every cluster
 // (`repeats` launches each, HIP events on `stream`) and keeps the fastest;
@@ -319,10 +349,11 @@ extern "C" int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream) {
     return SDG_ERR_INVALID;
   }
   const auto st = static_cast<hipStream_t>(stream);
-  const int order = lts->engine->s.order;
+  const EngineState& e = lts->engine->s;
+  const int order = e.order;
   const int64_t n = lts->layer.num_elements;
-  const int64_t rs = lts->engine->s.arithmetic == SDG_FP64 ? 8 : 4;
-  const CellLayout lay = cellLayout(lts->engine->s, &lts->layer);
+  const int64_t rs = e.arithmetic == SDG_FP64 ? 8 : 4;
+  const CellLayout lay = cellLayout(e, &lts->layer);
   const int64_t qBytes = n * lay.qStride * rs;
   const int64_t dBytes = n * lay.dsize * rs;
   void* saved[3] = {nullptr, nullptr, nullptr};
@@ -353,13 +384,16 @@ extern "C" int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream) {
     if (own.num_elements == 0) continue;
     for (int kind = 0; kind < 2 && rc == SDG_OK; ++kind) {
       float best = 0.0f;
-      int bestV = 0;
-      const int variants = kind == 0 ? localVariants(lts->engine->s) : kNeighborVariants;
-      for (int v = 0; v < variants && rc == SDG_OK; ++v) {
+      Tile bestTile;
+      std::vector<Tile> candidates;
+      for (int v = 0; v < (kind == 0 ? localVariants(e) : kNeighborVariants); ++v) candidates.push_back({v, false});
+      if (runsMx(e, kind, defaultTile(e, kind)) && !(kind == 0 && numberedLocal(e)))
+        candidates.push_back(defaultTile(e, kind));
+      for (const Tile& t : candidates) {
         (void)hipEventRecord(e0, st);
         for (int r = 0; r < repeats && rc == SDG_OK; ++r)
-          rc = kind == 0 ? runLocal(lts->engine->s, coeffs.data(), &own, 1, st, v)
-                         : launchNeighboringIntegration(lts->engine->s, coeffs.data(), coeffs.data(), &nbv, st, v);
+          rc = kind == 0 ? runLocal(e, coeffs.data(), &own, 1, st, t)
+                         : runNeighbor(e, coeffs.data(), coeffs.data(), &nbv, st, t);
         (void)hipEventRecord(e1, st);
         if (rc != SDG_OK) break;
         const hipError_t err = hipEventSynchronize(e1);
@@ -368,12 +402,12 @@ extern "C" int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream) {
           rc = hipFail(err != hipSuccess ? err : hipErrorUnknown, "sdg_lts_autotune timing");
           break;
         }
-        if (v == 0 || ms < best) {
+        if (&t == &candidates.front() || ms < best) {
           best = ms;
-          bestV = v;
+          bestTile = t;
         }
       }
-      (kind == 0 ? lts->tileLocal : lts->tileNeighbor)[c] = bestV;
+      lts->tile[kind][c] = bestTile;
     }
   }
   // restore whenever the state was saved, also after a failed tuning launch
@@ -388,43 +422,41 @@ extern "C" int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream) {
     if (saved[i] != nullptr) (void)hipFree(saved[i]);
   if (e0 != nullptr) (void)hipEventDestroy(e0);
   if (e1 != nullptr) (void)hipEventDestroy(e1);
-  // a captured macro step used the previous tiles
-  if (lts->exec != nullptr) {
-    (void)hipGraphExecDestroy(lts->exec);
-    lts->exec = nullptr;
-  }
-  if (lts->graph != nullptr) {
-    (void)hipGraphDestroy(lts->graph);
-    lts->graph = nullptr;
-  }
+  dropGraph(lts);
   return rc;
 }
 
 extern "C" int sdg_lts_set_tile_variant(sdg_lts* lts, int cluster, int kernel, int variant) {
-  if (lts == nullptr || cluster < 0 || cluster >= static_cast<int>(lts->tileLocal.size()) || kernel < 0 ||
-      kernel > 1 || variant < 0 || variant >= (kernel == 0 ? localVariants(lts->engine->s) : kNeighborVariants)) {
+  if (!tileArguments(lts, cluster, kernel, "sdg_lts_set_tile_variant")) return SDG_ERR_INVALID;
+  if (variant < 0 || variant >= (kernel == 0 ? localVariants(lts->engine->s) : kNeighborVariants)) {
     setError("sdg_lts_set_tile_variant: invalid arguments");
     return SDG_ERR_INVALID;
   }
-  (kernel == 0 ? lts->tileLocal : lts->tileNeighbor)[cluster] = variant;
-  if (lts->exec != nullptr) {
-    (void)hipGraphExecDestroy(lts->exec);
-    lts->exec = nullptr;
-  }
-  if (lts->graph != nullptr) {
-    (void)hipGraphDestroy(lts->graph);
-    lts->graph = nullptr;
-  }
+  lts->tile[kernel][cluster] = {variant, false};
+  dropGraph(lts);
   return SDG_OK;
 }
 
 extern "C" int sdg_lts_tile_variant(const sdg_lts* lts, int cluster, int kernel) {
-  if (lts == nullptr || cluster < 0 || cluster >= static_cast<int>(lts->tileLocal.size()) || kernel < 0 ||
-      kernel > 1) {
-    setError("sdg_lts_tile_variant: invalid arguments");
-    return SDG_ERR_INVALID;
+  if (!tileArguments(lts, cluster, kernel, "sdg_lts_tile_variant")) return SDG_ERR_INVALID;
+  return lts->tile[kernel][cluster].variant;
+}
+
+extern "C" int sdg_lts_matrix_core(const sdg_lts* lts, int cluster, int kernel) {
+  if (!tileArguments(lts, cluster, kernel, "sdg_lts_matrix_core")) return SDG_ERR_INVALID;
+  return runsMx(lts->engine->s, kernel, lts->tile[kernel][cluster]) ? 1 : 0;
+}
+
+extern "C" int sdg_lts_use_matrix_core(sdg_lts* lts, int cluster, int kernel) {
+  if (!tileArguments(lts, cluster, kernel, "sdg_lts_use_matrix_core")) return SDG_ERR_INVALID;
+  const Tile tile = defaultTile(lts->engine->s, kernel);
+  if (!runsMx(lts->engine->s, kernel, tile)) {
+    setError("sdg_lts_use_matrix_core: the engine has no matrix-core pass for this kernel");
+    return SDG_ERR_UNSUPPORTED;
   }
-  return kernel == 0 ? lts->tileLocal[cluster] : lts->tileNeighbor[cluster];
+  lts->tile[kernel][cluster] = tile;
+  dropGraph(lts);
+  return SDG_OK;
 }
 
 extern "C" int sdg_lts_advance(sdg_lts* lts, int macro_steps, void* stream) {

@@ -181,6 +181,17 @@ class LocalTimeStepping:
             out[c] = {k: int(lib().sdg_lts_tile_variant(self.handle, c, i)) for i, k in enumerate(("local", "neigh"))}
         return out
 
+    def matrix_core(self) -> dict:
+        """Whether the matrix-core pass runs, per cluster and kernel."""
+        return {c: {k: lib().sdg_lts_matrix_core(self.handle, c, i) == 1 for i, k in enumerate(("local", "neigh"))}
+                for c in range(self.layer.lts.num_clusters)}
+
+    def use_matrix_core(self):
+        """Choose the matrix-core passes again for every cluster."""
+        for c in range(self.layer.lts.num_clusters):
+            for k in (0, 1):
+                check(lib().sdg_lts_use_matrix_core(self.handle, c, k), "sdg_lts_use_matrix_core")
+
     def close(self):
         if self.handle:
             check(lib().sdg_lts_destroy(self.handle), "sdg_lts_destroy")

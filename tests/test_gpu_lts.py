@@ -225,3 +225,35 @@ def test_lts_rejects_missing_setup(gpu):
     layer64.view.lts_setup = None
     with pytest.raises(_capi.SdgError):
         LocalTimeStepping(eng64, layer64)
+
+
+# VALU variant numbers name the VALU kernels under either family (bit for bit); the matrix-core passes,
+# which run untuned, can be chosen again
+@pytest.mark.parametrize("order,arith", [(3, "fp32"), (6, "fp32"), (4, "fp64"), (5, "fp64"), (7, "fp64")])
+def test_variant_numbers_name_the_valu_kernels(gpu, order, arith):
+    import torch
+    lts = make_lts_setup(order, fractions=(0.5, 0.3, 0.2), dims=(8, 6, 6), seed=4)
+
+    def macro_step(family, local, neigh, again=False):
+        eng = Engine(order, arith)
+        eng.set_kernels(family)
+        layer = DeviceLtsLayer(eng, lts)
+        run = LocalTimeStepping(eng, layer)
+        if local is not None:
+            run.set_tile(local, kernel=0)
+            run.set_tile(neigh, kernel=1)
+        if again:
+            run.use_matrix_core()
+        assert run.matrix_core() == ({c: dict(local=local is None or again, neigh=local is None or again)
+                                      for c in range(3)} if family == "auto" else
+                                     {c: dict(local=False, neigh=False) for c in range(3)})
+        run.advance(1)
+        torch.cuda.synchronize()
+        return layer.dofs.clone()
+
+    for variant in range(5):
+        print(f"variant numbers order={order} {arith} variant={variant}", flush=True)
+        tile = min(variant, 3)
+        first = 1 if arith == "fp64" else 0  # FP64's local variant 0 is the matrix-core pass
+        assert torch.equal(macro_step("auto", first + tile, variant), macro_step("valu", tile, variant))
+    assert torch.equal(macro_step("auto", None, None), macro_step("auto", 1, 4, again=True))
