@@ -236,8 +236,10 @@ int sdg_lts_advance(sdg_lts* lts, int macro_steps, void* stream);
  * (StreamRuntime::runGraph, src/Parallel/Runtime/Stream.h:163-190). */
 int sdg_lts_graph_advance(sdg_lts* lts, int macro_steps, void* stream);
 /* Tile autotuner (no reference counterpart: tile shapes are the engine's
- * own): times the tile variants of both kernels of every cluster on the
- * cluster's data, keeps the fastest and restores the cells' state.
+ * own): times the kernels of both passes of every cluster on the cluster's
+ * data, keeps the fastest (a VALU variant in place of a matrix-core pass that
+ * shares its launch: only if the whole macro step gets faster) and restores
+ * the cells' state.
  * Allocates temporaries for the saved state; synchronises `stream`. */
 int sdg_lts_autotune(sdg_lts* lts, int repeats, void* stream);
 /* VALU variant of `cluster` and kernel 0 (local) / 1 (neighbour).

@@ -257,3 +257,28 @@ def test_variant_numbers_name_the_valu_kernels(gpu, order, arith):
         first = 1 if arith == "fp64" else 0  # FP64's local variant 0 is the matrix-core pass
         assert torch.equal(macro_step("auto", first + tile, variant), macro_step("valu", tile, variant))
     assert torch.equal(macro_step("auto", None, None), macro_step("auto", 1, 4, again=True))
+
+
+@pytest.mark.parametrize("order,arith", [(3, "fp64"), (3, "fp32"), (4, "fp64")])
+def test_autotuning_does_not_slow_small_clusters_down(gpu, order, arith):
+    # clusters that share launches: a variant that is faster alone must not take its cluster out of them
+    import torch
+    lts = make_lts_setup(order, fractions=(0.6, 0.25, 0.1, 0.05), dims=(32, 4, 4), seed=2)
+    eng = Engine(order, arith)
+    layer = DeviceLtsLayer(eng, lts)
+    untuned, tuned = LocalTimeStepping(eng, layer), LocalTimeStepping(eng, layer)
+    print(f"autotune order={order} {arith}: {tuned.autotune(repeats=5)} {tuned.matrix_core()}", flush=True)
+
+    def macro_step(run):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        run.advance(10, graph=True)
+        end.record()
+        torch.cuda.synchronize()
+        return start.elapsed_time(end) / 10
+
+    for run in (untuned, tuned):
+        run.advance(1, graph=True)
+    before, after = (min(macro_step(run) for _ in range(7)) for run in (untuned, tuned))
+    print(f"macro step untuned {1e3 * before:.0f} us, tuned {1e3 * after:.0f} us", flush=True)
+    assert after <= 1.1 * before  # repeated timings of one step differ by less than one per cent
