@@ -130,6 +130,16 @@ int launchLocalIntegrationMx(const EngineState& e, const double* coeffs, const s
 // the neighbour pass from the neighbours' buffers (LTS: with the time
 // coefficients, else nullptr: global time stepping)
 bool hasNeighborMx(const EngineState& e);
+// whether one call over `cells` cells, from DOFs or from LTS buffers and
+// derivatives, is faster with it than on the VALU.  Not at ORDER 3 in FP32, nor
+// in FP64 from DOFs up to 24 cells per CU: a tile's two barriers and its groups
+// padded to 16 tasks outweigh 10 x 6 products (periodic and random links, VALU
+// / matrix cores: FP32 300 cells 8.8 / 14.8 and 16.2 us, 5,000 11.2 / 17.6 and
+// 19.3, 50,000 48 / 53 and 57, LTS 2,560 12.6 / 19.0; FP64 5,000 22 / 23 and
+// 26, 6,500 27 / 24 and 27; LTS 2,560 25.9 / 23.0).  The clusters of a layer
+// share its launch, which is faster there as well (a macro step of 51,200 cells
+// in FP32 803 / 779 us).
+bool prefersNeighborMx(const EngineState& e, int64_t cells, bool lts);
 int launchNeighborMx(const EngineState& e, const sdg_layer* layer, const double* timeCoeffs,
                      const double* subtimeCoeffs, hipStream_t stream);
 // the same from the face traces the local pass wrote (layer->face_traces,

@@ -214,6 +214,10 @@ bool hasMx(const EngineState& e) { return e.mxFrags != nullptr && e.kernels == S
 
 bool hasNeighborMx(const EngineState& e) { return hasMx(e) && e.mxNeighbor; }
 
+bool prefersNeighborMx(const EngineState& e, int64_t cells, bool lts) {
+  return hasNeighborMx(e) && (e.order > 3 || (e.arithmetic == SDG_FP64 && (lts || cells > 24 * 256)));
+}
+
 namespace {
 // every cell of the layer in one step
 mx::ClusterStep whole(const sdg_layer* layer, const double* coeffs, const double* sub, int reset) {

@@ -1319,7 +1319,7 @@ int launchLocal(const EngineState& e, const sdg_layer* layer, hipStream_t stream
   return dispatch<LocalOp>(e, layer, stream);
 }
 int launchNeighbor(const EngineState& e, const sdg_layer* layer, hipStream_t stream) {
-  if (hasNeighborMx(e)) return launchNeighborMx(e, layer, nullptr, nullptr, stream);
+  if (prefersNeighborMx(e, layer->num_elements, false)) return launchNeighborMx(e, layer, nullptr, nullptr, stream);
   return dispatch<NeighborOp>(e, layer, stream, static_cast<const double*>(nullptr),
                               static_cast<const double*>(nullptr));
 }

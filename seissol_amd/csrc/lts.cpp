@@ -180,8 +180,9 @@ extern "C" int sdg_compute_neighboring_integration(sdg_engine* engine, const dou
       !ltsLayerOk(layer, true, "sdg_compute_neighboring_integration") ||
       !layerStridesOk(engine->s, layer, "sdg_compute_neighboring_integration"))
     return SDG_ERR_INVALID;
-  return runNeighbor(engine->s, time_coeffs, subtime_coeffs, layer, static_cast<hipStream_t>(stream),
-                     defaultTile(engine->s, 1));
+  Tile tile = defaultTile(engine->s, 1);
+  tile.matrixCore = prefersNeighborMx(engine->s, layer->num_elements, true);
+  return runNeighbor(engine->s, time_coeffs, subtime_coeffs, layer, static_cast<hipStream_t>(stream), tile);
 }
 
 struct sdg_lts {

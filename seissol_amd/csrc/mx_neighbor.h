@@ -371,7 +371,11 @@ int neighborImpl(const EngineState& st, const sdg_layer* L, const ClusterStep* s
   };
   if (traces) launch(std::integral_constant<int, kFromTraces>{});
   else if (steps[0].coeffs != nullptr && L->lts_setup != nullptr) launch(std::integral_constant<int, kFromLts>{});
-  else launch(std::integral_constant<int, kFromDofs>{});
+  else if constexpr (O > 3 || sizeof(real) == 8) launch(std::integral_constant<int, kFromDofs>{});
+  else {  // prefersNeighborMx sends these to the VALU
+    setError("the matrix-core neighbour pass from DOFs starts at ORDER 4 in FP32");
+    return SDG_ERR_UNSUPPORTED;
+  }
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;
 }

@@ -265,3 +265,30 @@ def test_operators_far_apart_equal_dense_ones(gpu, arith, n, megabytes):
             assert torch.equal(sides[0][k], sides[1][k]), (part, k)
         del sides, a
     torch.cuda.empty_cache()
+
+
+# the line between the VALU and the matrix-core neighbour pass at ORDER 3 (24 cells per CU in FP64 from
+# DOFs, the matrix cores in FP64 with LTS, the VALU in FP32): the same kernel below it, the same values above
+@pytest.mark.parametrize("lts", [False, True])
+@pytest.mark.parametrize("arith,n,equal", [("fp64", 6144, True), ("fp64", 6145, False), ("fp32", 6145, True)])
+def test_neighbour_pass_of_order_3(gpu, arith, n, equal, lts):
+    import torch
+    print(f"neighbour order=3 {arith} n={n} lts={lts}", flush=True)
+    results = []
+    for family in ("auto", "valu"):
+        eng = Engine(3, arith)
+        eng.set_kernels(family)
+        a = random_layer(eng, 3, arith, n, 0, "dense", n, setup=True)
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        draw = lambda hi, shape, t: torch.randint(0, hi, shape, generator=gen, device="cuda").to(t)
+        a["neighbors"] = draw(n, (n, 4), torch.int32)
+        a["relations"] = torch.stack([draw(4, (n, 4), torch.uint8), draw(3, (n, 4), torch.uint8)], -1)
+        a["aminus"] = torch.rand((n, 4, 81), generator=gen, device="cuda", dtype=a["dofs"].dtype) * 2 - 1
+        a["setup"] = draw(1 << 11, (n,), torch.int16)
+        v = a["view"]
+        v.aminus, v.face_neighbors, v.face_relations = ptr(a["aminus"]), ptr(a["neighbors"]), ptr(a["relations"])
+        v.lts_setup = ptr(a["setup"])
+        run_neighbor(eng, a, lts)
+        results.append(a)
+    assert torch.equal(results[0]["dofs"], results[1]["dofs"]) == (equal and not (lts and arith == "fp64"))
+    same(*results, ("dofs",), 1e-12 if arith == "fp64" else 5e-5, f"neighbour order 3 n={n}")
