@@ -11,6 +11,8 @@
 // 50 -> 11 us; a whole training step 57 -> 14.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "engine.h"
 #include "friction_common.h"
 
@@ -22,7 +24,11 @@ constexpr int kStride = kMlpInputs + 1;  // samples: features then target
 constexpr int kGroup = 32, kPerSample = 8, kThreads = kGroup * kPerSample;
 constexpr int kUnits = kMlpHidden / kPerSample;  // units of a layer per thread
 constexpr int kLd = kMlpHidden + 1;              // padded row of 32 units
-constexpr int kMaxBlocks = 256;
+// Blocks: one per group up to one per CU, then as many as have eight groups
+// each, up to four per CU: a block ends with 1,300 atomics, the same addresses
+// for all (a step of 16,384 samples: 128 blocks 36 us, 256 38, 512 52; 131,072:
+// 256 101, 512 86, 1024 107; 2 million: 256 1217, 512 773, 1024 631).
+constexpr int64_t kMinFull = 256, kMaxBlocks = 1024, kGroupsPerBlock = 8;
 
 __global__ void kZero(float* __restrict__ p, int n, float* __restrict__ loss) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -47,9 +53,10 @@ __global__ __launch_bounds__(kThreads) void kLossGrad(const float* __restrict__ 
   }
   const float inv = 1.0f / static_cast<float>(n);
   float lossSum = 0.0f;
-  // this thread's gradients: W2[gk][gj .. gj + 3]; W1[t / 6][t % 6] or, for the
+  // this thread's gradients: W2[gk][gj + 8 i], i < 4 (neighbouring threads add to
+  // neighbouring entries: 16,384 samples 45 -> 38 us); W1[t / 6][t % 6] or, for the
   // last 64 threads, one of b1 and W3 (bk) or b2, and b3
-  const int gk = t / kPerSample, gj = kUnits * (t % kPerSample);
+  const int gk = t / kPerSample, gj = t % kPerSample;
   constexpr int kW1 = kMlpHidden * kMlpInputs;
   static_assert(kThreads == kW1 + 2 * kMlpHidden, "W1's entries, then two threads per unit");
   const int wk = t / kMlpInputs, wj = t % kMlpInputs, bk = (t - kW1) & (kMlpHidden - 1);
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(kThreads) void kLossGrad(const float* __restrict__ 
     for (int q = 0; q < kGroup; ++q) {
       const float x = sD2[q][gk];
 #pragma unroll
-      for (int i = 0; i < kUnits; ++i) gW2[i] += x * sH1[q][gj + i];
+      for (int i = 0; i < kUnits; ++i) gW2[i] += x * sH1[q][gj + kPerSample * i];
     }
     if (t < kW1) {
 #pragma unroll 8
@@ -135,7 +142,7 @@ __global__ __launch_bounds__(kThreads) void kLossGrad(const float* __restrict__ 
     }
   }
 #pragma unroll
-  for (int i = 0; i < kUnits; ++i) atomicAdd(&grads[kOffW2 + gk * kMlpHidden + gj + i], gW2[i]);
+  for (int i = 0; i < kUnits; ++i) atomicAdd(&grads[kOffW2 + gk * kMlpHidden + gj + kPerSample * i], gW2[i]);
   if (t < kW1) {
     atomicAdd(&grads[kOffW1 + t], g0);
   } else if (t < kW1 + kMlpHidden) {
@@ -192,7 +199,8 @@ int sdg_mlp_loss_grad(const float* params, const float* samples, int64_t n, floa
   auto st = static_cast<hipStream_t>(stream);
   friction::kZero<<<(friction::kMlpParams + 255) / 256, 256, 0, st>>>(grads, friction::kMlpParams, loss);
   const int64_t groups = (n + friction::kGroup - 1) / friction::kGroup;
-  const unsigned grid = static_cast<unsigned>(groups < friction::kMaxBlocks ? groups : friction::kMaxBlocks);
+  const int64_t full = std::clamp(groups / friction::kGroupsPerBlock, friction::kMinFull, friction::kMaxBlocks);
+  const unsigned grid = static_cast<unsigned>(std::min(groups, full));
   friction::kLossGrad<<<grid, friction::kThreads, 0, st>>>(params, samples, n, grads, loss);
   SDG_HIP_CHECK(hipGetLastError());
   return SDG_OK;

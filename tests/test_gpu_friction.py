@@ -138,6 +138,12 @@ def test_mlp_gradient_of_ragged_batches(gpu, n):
     assert np.all(tr.grads.cpu().numpy()[:14] == 0.0)
 
 
+# more than eight groups of 32 for each of 256 blocks, and for each of 1,024
+@pytest.mark.parametrize("n", [65_536 + 257, 262_144 + 33])
+def test_mlp_gradient_of_large_batches(gpu, n):
+    test_mlp_gradient_of_ragged_batches(gpu, n)
+
+
 def test_mlp_training_reduces_loss(gpu):
     import torch
     rng = np.random.default_rng(2)
