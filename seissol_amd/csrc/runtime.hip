@@ -604,9 +604,9 @@ int sdg_compute_batched_neighbors_integral(sdg_engine* engine, const sdg_layer* 
   if (engine == nullptr || !validLayer(engine->s, layer, true)) return SDG_ERR_INVALID;
   if (matrixCore(engine->s.arithmetic) && layer->face_traces != nullptr)
     return launchNeighborMfma(engine->s, layer, static_cast<hipStream_t>(stream));
-  // the FP64 engine reads the time-integrated DOFs here, as the reference's
-  // neighbour integral does; its matrix-core neighbour pass runs only inside
-  // the fused proxy step, whose local pass writes the traces it reads
+  // the FP64 and FP32 engines read the time-integrated DOFs here, as the
+  // reference's neighbour integral does; the FP64 engine's pass from face traces
+  // runs only inside the fused proxy step, whose local pass writes them
   return launchNeighbor(engine->s, layer, static_cast<hipStream_t>(stream));
 }
 
